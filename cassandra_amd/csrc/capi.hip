@@ -170,7 +170,18 @@ void upload_programs(cad_patterns* p)
         tslots.push_back(t);
     }
     tern.insert(tern.end(), kTernPadding, 0u);
+    // the index tiles, pattern after pattern
+    IndexTiles it;
+    int slot = 0;
+    for (const PatternInfo& pi : g.patterns) {
+        const int n = int(pi.variations.size());
+        it.add(g.slots.data() + slot, n, slot);
+        slot += n;
+    }
     hipStream_t st = p->ctx->stream;
+    p->ntiles = int(it.tiles.size());
+    p->d_tiles = to_device(it.tiles, st);
+    p->d_weights = to_device(it.weights, st);
     p->d_tslots = to_device(tslots, st);
     p->d_tern = to_device(tern, st);
     p->d_slots = to_device(slots, st);
@@ -188,21 +199,32 @@ void upload_programs(cad_patterns* p)
     p->d_syscol0 = to_device(std::vector<uint32_t>{0u}, st);
 }
 
-void extract(cad_patterns* p, const uint64_t* pos, int64_t n, void* out, int bytes, int64_t slot_stride,
-             int64_t row_stride, int local)
+// Rows a wave of the slot-major extraction takes at a time, per lane: four
+// (8-byte stores of u16 entries) where that still gives every SIMD two waves.
+template <class OutT>
+void extract_slots(hipStream_t s, const TileView& v, const uint64_t* pos, int64_t n, OutT* out, int64_t ld,
+                   int64_t nstore, int local, int cus)
 {
-    if (n <= 0) return;
+    auto launch = [&](auto cc) {
+        constexpr int C = decltype(cc)::value;
+        const bool vec = reinterpret_cast<uintptr_t>(out) % (C * sizeof(OutT)) == 0 && ld % C == 0;
+        hipLaunchKernelGGL((k_index_extract<OutT, C>), dim3(unsigned(grid1(nstore, kRowBlock * C))), dim3(kRowBlock),
+                           0, s, pos, n, nstore, v, out, ld, local, int(vec));
+    };
+    if (nstore >= int64_t(64) * 4 * 8 * cus) launch(std::integral_constant<int, 4>{});
+    else launch(std::integral_constant<int, 1>{});
+    CAD_HIP(hipGetLastError());
+}
+
+void extract_rows(cad_patterns* p, const uint64_t* pos, int64_t n, uint32_t* out)
+{
     const int k = p->group->k();
-    hipStream_t s = p->ctx->stream;
-    const dim3 grid(grid1(n, kRowBlock * kExtractRows));
-    if (bytes == 2)
-        hipLaunchKernelGGL((k_index_extract<uint16_t, kExtractRows>), grid, dim3(kRowBlock), 0, s, pos, n,
-                           p->d_slots.as<DevSlot>(), k, p->d_tslots.as<DevTern>(), p->d_tern.as<uint32_t>(),
-                           p->d_dense.as<uint32_t>(), static_cast<uint16_t*>(out), slot_stride, row_stride, local);
-    else
-        hipLaunchKernelGGL((k_index_extract<uint32_t, kExtractRows>), grid, dim3(kRowBlock), 0, s, pos, n,
-                           p->d_slots.as<DevSlot>(), k, p->d_tslots.as<DevTern>(), p->d_tern.as<uint32_t>(),
-                           p->d_dense.as<uint32_t>(), static_cast<uint32_t*>(out), slot_stride, row_stride, local);
+    const int chunk = std::min(k, kExtractChunk);
+    const int pitch = chunk == k ? k : chunk | 1;
+    const size_t lds = size_t(kRowBlock) * size_t(pitch) * sizeof(uint32_t);
+    hipLaunchKernelGGL(k_index_extract_rows, dim3(unsigned(grid1(n, kRowBlock))), dim3(kRowBlock), lds,
+                       p->ctx->stream, pos, n, p->tiles(), k, chunk, pitch, out,
+                       int(reinterpret_cast<uintptr_t>(out) % 16 == 0));
     CAD_HIP(hipGetLastError());
 }
 
@@ -540,9 +562,9 @@ int cad_index_extract(cad_patterns* p, const uint64_t* d_pos, int64_t n, uint32_
         need(p && n >= 0 && (n == 0 || (d_pos && d_out)), "invalid argument");
         need(p->ctx != nullptr, "host-only pattern group (created without a context)");
         need(layout == CAD_LAYOUT_ROW_MAJOR || layout == CAD_LAYOUT_SLOT_MAJOR, "unknown layout");
-        const int k = p->group->k();
-        if (layout == CAD_LAYOUT_ROW_MAJOR) extract(p, d_pos, n, d_out, 4, 1, k, 0);
-        else extract(p, d_pos, n, d_out, 4, n, 1, 0);
+        if (n == 0) return;
+        if (layout == CAD_LAYOUT_ROW_MAJOR) extract_rows(p, d_pos, n, d_out);
+        else extract_slots<uint32_t>(p->ctx->stream, p->tiles(), d_pos, n, d_out, n, n, 0, p->ctx->cus);
     });
 }
 
@@ -570,11 +592,16 @@ cad_matrix* matrix_from_positions(cad_patterns* p, const uint64_t* d_pos, const 
     if (nsys == 1) default_schedule(m->tune, m->ibytes, n);
     m->ld = padded_rows(n);
     m->d_idx = DBuf(size_t(m->ibytes) * size_t(m->ld) * size_t(g.k()));
-    CAD_HIP(hipMemsetAsync(m->d_idx.p, 0, m->d_idx.bytes, p->ctx->stream));
     std::vector<uint32_t> base(g.k());
     for (int s = 0; s < g.k(); s++) base[s] = m->ibytes == 2 ? m->slot_lo[s] : 0u;
     m->d_base = to_device(base, p->ctx->stream);
-    extract(p, d_pos, n, m->d_idx.p, m->ibytes, m->ld, 1, m->ibytes == 2 ? 1 : 0);
+    // (the padding rows are written as zeros)
+    if (m->ibytes == 2)
+        extract_slots<uint16_t>(p->ctx->stream, p->tiles(), d_pos, n, m->d_idx.as<uint16_t>(), m->ld, m->ld, 1,
+                                p->ctx->cus);
+    else
+        extract_slots<uint32_t>(p->ctx->stream, p->tiles(), d_pos, n, m->d_idx.as<uint32_t>(), m->ld, m->ld, 0,
+                                p->ctx->cus);
     m->nsys = nsys;
     m->sys_row_begin = row_begin;
     m->cols_per_sys = cols_per;
@@ -628,6 +655,9 @@ int cad_matrix_from_positions_mf(cad_patterns* p, const uint64_t* d_pos, int64_t
         copy(m->d_slots, p->d_slots);
         copy(m->d_sq, p->d_sq);
         copy(m->d_dense, p->d_dense);
+        copy(m->d_tiles, p->d_tiles);
+        copy(m->d_weights, p->d_weights);
+        m->ntiles = p->ntiles;
         copy(m->d_tslots, p->d_tslots);
         copy(m->d_tern, p->d_tern);
         m->d_pos = DBuf(sizeof(uint64_t) * 2 * size_t(n));
@@ -787,12 +817,8 @@ int cad_matrix_download(const cad_matrix* m, uint32_t* out)
             std::vector<uint32_t> t(size_t(R) * k);
             if (R > 0) {
                 DBuf tmp(t.size() * 4);
-                hipLaunchKernelGGL((k_index_extract<uint32_t, kExtractRows>), dim3(grid1(R, kRowBlock * kExtractRows)),
-                                   dim3(kRowBlock), 0, s,
-                                   m->d_pos.as<uint64_t>(), R, m->d_slots.as<DevSlot>(), k,
-                                   m->d_tslots.as<DevTern>(), m->d_tern.as<uint32_t>(), m->d_dense.as<uint32_t>(),
-                                   tmp.as<uint32_t>(), R, int64_t(1), 0);
-                CAD_HIP(hipGetLastError());
+                extract_slots<uint32_t>(s, m->tiles(), m->d_pos.as<uint64_t>(), R, tmp.as<uint32_t>(), R, R, 0,
+                                        m->ctx->cus);
                 CAD_HIP(hipMemcpyAsync(t.data(), tmp.p, t.size() * 4, hipMemcpyDeviceToHost, s));
                 CAD_HIP(hipStreamSynchronize(s));
             }

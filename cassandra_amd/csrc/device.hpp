@@ -33,6 +33,38 @@ struct DevTern {
 };
 static_assert(sizeof(DevTern) == 32, "DevTern layout");
 
+// An index tile: up to four consecutive slots of one pattern, whose columns a
+// wave computes for 16 positions with one matrix instruction.  A square list's
+// number sum_j 3^j digit_j is a dot product of the position's 64 digits with
+// the list's weights; a tile's 16 rows of weights (four per slot: roles u, v,
+// w, z) times the digits of 16 positions is one 16x16x64 product of 8-bit
+// integers.  A weight beyond 8 bits is split over two rows, 243 apart (rows
+// of five digits: 3^0 .. 3^4, sums up to 242).  What the roles hold:
+//   kind 0 / 3  a = u + 243 v + 3^10 w + 3^15 z (u, v alone unless wide)
+//   kind 1      a = u, b = v; wide: a = u + 243 w, b = v + 243 z
+//   kind 2      a = u, b = v, d = w + 243 z; wide: the next tile's weights
+//               give the upper halves, a = u + 243 u', b = v + 243 v'
+// and the column is col_offset + a, dense[a], pair(a, b), pair(a, b) ds + d.
+// Every slot of a tile has the same kind, sizes and offset.
+struct IndexTile {
+    uint16_t kind, wide;
+    uint16_t slot_first, nslots;
+    uint32_t hs, ds;
+    uint32_t col_offset;
+    uint32_t dense_offset;
+    uint32_t weights;  // the tile's weights: 64 lanes x 16 bytes at this tile number
+    uint32_t pad;
+};
+static_assert(sizeof(IndexTile) == 32, "IndexTile layout");
+
+// The index tiles of a pattern group on the device.
+struct TileView {
+    const IndexTile* __restrict__ tiles;
+    const uint32_t* __restrict__ weights;  // 256 words a tile
+    const uint32_t* __restrict__ dense;
+    int n;
+};
+
 // A block of rows of one system, for the row-parallel kernels (SpMV and the
 // rows-length vector kernels).  Blocks of one system are contiguous in the
 // work list.

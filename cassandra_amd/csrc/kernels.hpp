@@ -350,40 +350,247 @@ __global__ void k_ternary_rows(const uint64_t* __restrict__ pos, int64_t n, uint
     }
 }
 
-// Pattern/Indexer.cpp InsertIndices for every row, RPT positions a thread
-// (rows r0 + i kRowBlock, so that each slot's stores of a wave stay
-// contiguous): out[s * slot_stride + r * row_stride] = (local ? 0 :
-// col_offset) + index, each slot's index from the position's ternary words.
-template <class OutT, int RPT>
-__global__ __launch_bounds__(kRowBlock) void k_index_extract(
-    const uint64_t* __restrict__ pos, int64_t n, const DevSlot* __restrict__ slots, int k,
-    const DevTern* __restrict__ tslots, const uint32_t* __restrict__ tern, const uint32_t* __restrict__ dense,
-    OutT* __restrict__ out, int64_t slot_stride, int64_t row_stride, int local)
+// ------------------------------------------------------ index tiles --------
+// A wave computes a tile's columns (IndexTile) for 64 rows with four matrix
+// products of 16 positions each: lane (n, g) = (lane % 16, lane / 16) feeds
+// the 16 digits of word g of position n (four registers, byte m of register v
+// the digit of square 16 g + v + 4 m) and receives the four roles of slot g
+// for position n.  Evaluating the square lists digit by digit took two vector
+// instructions per square and about as many scalar ones (FIT12: 444 squares a
+// row, 36 vector instructions per column); the products leave about 10.
+typedef int Int4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ Int4 expand_digits(uint32_t t)
 {
-    const int64_t r0 = blockIdx.x * int64_t(kRowBlock * RPT) + threadIdx.x;
-    if (r0 >= n) return;
-    uint32_t T[RPT][4];
-    bool ok[RPT];
+    return Int4{int(t & 0x03030303u), int((t >> 2) & 0x03030303u), int((t >> 4) & 0x03030303u),
+                int((t >> 6) & 0x03030303u)};
+}
+
+// Lane (n, g)'s digits of row r, read from the positions (word g: 16-bit
+// group g of P and of O).
+__device__ __forceinline__ Int4 digits_of_position(const uint64_t* __restrict__ pos, int64_t r)
+{
+    const int g = (threadIdx.x >> 4) & 3;
+    const uint16_t* __restrict__ h = reinterpret_cast<const uint16_t*>(pos + 2 * r);
+    return expand_digits(spread16(h[g]) | (spread16(h[4 + g]) << 1));
+}
+
+// Rows [4j, 4j+4) of four registers of 16-lane groups, transposed: register p
+// holding slot g of position set p in lane group g becomes register j holding
+// slot j of position set p in lane group p (lane = position).
+__device__ __forceinline__ void transpose_groups(uint32_t (&r)[4])
+{
+    auto s01 = __builtin_amdgcn_permlane16_swap(r[0], r[1], false, false);
+    auto s23 = __builtin_amdgcn_permlane16_swap(r[2], r[3], false, false);
+    auto a = __builtin_amdgcn_permlane32_swap(s01[0], s23[0], false, false);
+    auto b = __builtin_amdgcn_permlane32_swap(s01[1], s23[1], false, false);
+    r[0] = a[0];
+    r[1] = b[0];
+    r[2] = a[1];
+    r[3] = b[1];
+}
+
+// The pattern-local column of slot g of the tile for the four position sets
+// b[0..4) (idx[p]: lane (n, g) holds slot g of position n of set p; lanes of
+// slots past the tile's hold column 0 of some configuration).
+__device__ __forceinline__ void tile_columns(const IndexTile& t, const TileView& tv, const Int4 (&b)[4],
+                                             uint32_t (&idx)[4])
+{
+    const Int4* __restrict__ wt =
+        reinterpret_cast<const Int4*>(tv.weights) + int64_t(t.weights) * 64 + (threadIdx.x & 63);
+    const Int4 w = wt[0], zero = {0, 0, 0, 0};
+    Int4 d[4];
 #pragma unroll
-    for (int i = 0; i < RPT; i++) {
-        const int64_t r = r0 + int64_t(i) * kRowBlock;
-        ok[i] = r < n;
-        const int64_t rr = ok[i] ? r : r0;  // a valid row's words for the lanes past the end
-        ternary_words(pos[2 * rr], pos[2 * rr + 1], T[i]);
+    for (int p = 0; p < 4; p++) d[p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w, b[p], zero, 0, 0, 0);
+    if (t.kind == 0 || t.kind == 3) {
+#pragma unroll
+        for (int p = 0; p < 4; p++) idx[p] = uint32_t(d[p][0]) + __umul24(uint32_t(d[p][1]), 243u);
+        if (t.wide) {
+#pragma unroll
+            for (int p = 0; p < 4; p++)
+                idx[p] += __umul24(uint32_t(d[p][2]), 59049u) + __umul24(uint32_t(d[p][3]), 14348907u);
+        }
+        if (t.kind == 3) {
+#pragma unroll
+            for (int p = 0; p < 4; p++) idx[p] = tv.dense[t.dense_offset + idx[p]];
+        }
+        return;
     }
-    for (int s = 0; s < k; s++) {
-        const DevSlot sl = uniform_load(slots + s);
-        uint32_t v[RPT];
-        slot_index_rows<RPT>(sl, uniform_load(tslots + s), tern, dense, T, v);
-        const uint32_t base = local ? 0u : sl.col_offset;
+    uint32_t a[4], c[4];
 #pragma unroll
-        for (int i = 0; i < RPT; i++)
-            if (ok[i]) out[int64_t(s) * slot_stride + (r0 + int64_t(i) * kRowBlock) * row_stride] = OutT(base + v[i]);
+    for (int p = 0; p < 4; p++) {
+        a[p] = uint32_t(d[p][0]);
+        c[p] = uint32_t(d[p][1]);
+    }
+    if (t.wide) {
+        if (t.kind == 1) {
+#pragma unroll
+            for (int p = 0; p < 4; p++) {
+                a[p] += __umul24(uint32_t(d[p][2]), 243u);
+                c[p] += __umul24(uint32_t(d[p][3]), 243u);
+            }
+        } else {
+            const Int4 w2 = wt[64];
+#pragma unroll
+            for (int p = 0; p < 4; p++) {
+                const Int4 e = __builtin_amdgcn_mfma_i32_16x16x64_i8(w2, b[p], zero, 0, 0, 0);
+                a[p] += __umul24(uint32_t(e[0]), 243u);
+                c[p] += __umul24(uint32_t(e[1]), 243u);
+            }
+        }
+    }
+    // the pair's number, from the smaller and the larger half (below 3^8)
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+        const uint32_t lo = min(a[p], c[p]), hi = max(a[p], c[p]);
+        idx[p] = __umul24(lo, t.hs) + hi - (__umul24(lo, lo + 1u) >> 1);
+    }
+    if (t.kind == 2) {
+#pragma unroll
+        for (int p = 0; p < 4; p++)
+            idx[p] = __umul24(idx[p], t.ds) + uint32_t(d[p][2]) + __umul24(uint32_t(d[p][3]), 243u);
     }
 }
 
-// Positions a thread of k_index_extract.
-constexpr int kExtractRows = 8;
+// A descriptor through the constant address space (scalar loads): for arrays
+// no kernel writes, in kernels without LDS traffic to wait for.
+template <class T>
+__device__ __forceinline__ T constant_load(const T* p)
+{
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    const ConstWords c = (ConstWords)(reinterpret_cast<const uint32_t*>(p));
+    uint32_t r[sizeof(T) / 4];
+#pragma unroll
+    for (int i = 0; i < int(sizeof(T) / 4); i++) r[i] = c[i];
+    T t;
+    __builtin_memcpy(&t, r, sizeof(T));
+    return t;
+}
+
+// Pattern/Indexer.cpp InsertIndices for every row, slot-major: out[s * ld + r]
+// = (local ? 0 : col_offset) + column, rows [n, nstore) as zeros.  A wave takes
+// 64 C rows, lane l the C consecutive rows from its first + l C on, so that
+// a slot's stores are C entries wide (vec: every such run is aligned to its
+// size).  Bound by the stores: 5M rows of FIT8 as u16 take 159 µs for 420 MB,
+// 240 µs (with the clear of the whole matrix that the padding rows cost)
+// digit by digit; 100,000 rows of FIT4 8 µs against 36.
+template <class OutT, int C>
+__global__ __launch_bounds__(kRowBlock) void k_index_extract(const uint64_t* __restrict__ pos, int64_t n,
+                                                             int64_t nstore, TileView tv, OutT* __restrict__ out,
+                                                             int64_t ld, int local, int vec)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t base = (blockIdx.x * int64_t(kRowBlock / 64) + (threadIdx.x >> 6)) * (64 * C);
+    if (base >= nstore) return;
+    Int4 b[C][4];
+#pragma unroll
+    for (int c = 0; c < C; c++)
+#pragma unroll
+        for (int p = 0; p < 4; p++)
+            b[c][p] = digits_of_position(pos, min(base + (16 * p + (lane & 15)) * C + c, n - 1));
+    const int64_t r0 = base + int64_t(lane) * C;
+    for (int t = 0; t < tv.n; t++) {
+        const IndexTile tl = constant_load(tv.tiles + t);
+        const uint32_t off = local ? 0u : tl.col_offset;
+        uint32_t v[C][4];
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            tile_columns(tl, tv, b[c], v[c]);
+            transpose_groups(v[c]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (j >= tl.nslots) break;
+            OutT o[C];
+#pragma unroll
+            for (int c = 0; c < C; c++) o[c] = r0 + c < n ? OutT(off + v[c][j]) : OutT(0);
+            OutT* __restrict__ dst = out + int64_t(tl.slot_first + j) * ld + r0;
+            if (vec && r0 + C <= nstore) {
+                struct alignas(sizeof(OutT) * C) Run {
+                    OutT e[C];
+                };
+                Run run;
+                __builtin_memcpy(&run, o, sizeof(run));
+                *reinterpret_cast<Run*>(dst) = run;
+            } else {
+#pragma unroll
+                for (int c = 0; c < C; c++)
+                    if (r0 + c < nstore) dst[c] = o[c];
+            }
+        }
+    }
+}
+
+// The same row-major (out[r * k + s], the global column).  A wave takes 64
+// rows: the columns of a run of tiles (at most `chunk` slots) go into the
+// wave's part of the LDS and from there to memory in row order, so that a
+// store instruction writes consecutive words; one 4-byte store per column,
+// rows apart, wrote partial lines.  With all slots in one chunk the 64 rows
+// are one run of memory and leave in 16-byte stores (vec: out is aligned).
+// 5M rows of FIT4: 131 µs for 440 MB (3.4 TB/s); 1,051 µs with the scattered
+// stores.
+__global__ __launch_bounds__(kRowBlock) void k_index_extract_rows(const uint64_t* __restrict__ pos, int64_t n,
+                                                                  TileView tv, int k, int chunk, int pitch,
+                                                                  uint32_t* __restrict__ out, int vec)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t* __restrict__ st = reinterpret_cast<uint32_t*>(smem_raw) + wave * 64 * pitch;
+    const int64_t base = (blockIdx.x * int64_t(kRowBlock / 64) + wave) * 64;
+    if (base >= n) return;
+    const int rows = int(min<int64_t>(64, n - base));
+    Int4 b[4];
+#pragma unroll
+    for (int p = 0; p < 4; p++) b[p] = digits_of_position(pos, min<int64_t>(base + 16 * p + (lane & 15), n - 1));
+    uint32_t* __restrict__ dst = out + base * k;
+    int first = 0;  // first slot of the chunk
+    for (int t = 0; t < tv.n; t++) {
+        const IndexTile tl = constant_load(tv.tiles + t);
+        uint32_t v[4];
+        tile_columns(tl, tv, b, v);
+        const int g = lane >> 4;
+        if (g < tl.nslots) {
+#pragma unroll
+            for (int p = 0; p < 4; p++)
+                st[(16 * p + (lane & 15)) * pitch + (tl.slot_first - first) + g] = tl.col_offset + v[p];
+        }
+        const int end = tl.slot_first + tl.nslots;
+        const int next = t + 1 < tv.n ? end + int(constant_load(tv.tiles + t + 1).nslots) : 0;
+        if (t + 1 < tv.n && next - first <= chunk) continue;
+        // the wave's LDS writes land before its reads (in order; the fence
+        // keeps the compiler from moving them)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int nc = end - first;
+        if (nc == k && pitch == k && vec) {
+            const int total = rows * k, whole = total & ~3;
+            for (int e = 4 * lane; e < whole; e += 256)
+                *reinterpret_cast<uint4*>(dst + e) = *reinterpret_cast<const uint4*>(st + e);
+            if (whole + lane < total) dst[whole + lane] = st[whole + lane];
+        } else {
+            // word e of the chunk is slot e % nc of row e / nc
+            const int dr = 64 / nc, ds = 64 % nc;
+            int r = lane / nc, s = lane % nc;
+            while (r < rows) {
+                dst[int64_t(r) * k + first + s] = st[r * pitch + s];
+                r += dr;
+                s += ds;
+                if (s >= nc) {
+                    s -= nc;
+                    r++;
+                }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        first = end;
+    }
+}
+
+// Most slots a chunk of k_index_extract_rows holds in LDS (14 KB a wave), and
+// the row pitch: the chunk itself where it holds all k slots (the LDS then has
+// the layout of the memory), else odd.
+constexpr int kExtractChunk = 56;
 
 // Matrix-free view of a pattern matrix: the column of slot s in row r is
 // recomputed from the row's position (16 bytes) with the slot's program

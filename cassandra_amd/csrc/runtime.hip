@@ -462,6 +462,61 @@ void append_ternary_list(const uint8_t* src, int n, std::vector<uint32_t>& tern,
     }
 }
 
+void IndexTiles::add(const SlotProgram* slots, int n, int first)
+{
+    // row 4 j + role of the tile whose weights start at `at` gains 3^(e mod 5)
+    // for digit e of the list, one role per five digits
+    auto put = [&](size_t at, int j, const SquareList& l, int e0, int role, int limbs, int step) {
+        for (int e = e0; e < int(l.src.size()) && e < e0 + 5 * limbs; e++) {
+            const int row = 4 * j + role + step * ((e - e0) / 5);
+            const int q = l.src[size_t(e)], d = q % 16, lane = 16 * (q / 16) + row;
+            weights[at + size_t(lane) * 16 + size_t(4 * (d % 4) + d / 4)] = int8_t(pow3((e - e0) % 5));
+        }
+    };
+    for (int j0 = 0; j0 < n; j0 += 4) {
+        const SlotProgram& s0 = slots[j0];
+        IndexTile t{};
+        t.slot_first = uint16_t(first + j0);
+        t.nslots = uint16_t(std::min(4, n - j0));
+        t.hs = s0.hs;
+        t.ds = s0.ds;
+        t.col_offset = s0.col_offset;
+        t.dense_offset = s0.dense_offset;
+        size_t longest[3] = {0, 0, 0};
+        for (int j = 0; j < t.nslots; j++)
+            for (int l = 0; l < 3; l++) longest[l] = std::max(longest[l], slots[j0 + j].list[l].src.size());
+        // a pair without a diagonal list is a plain pair (idx * 1 + 0): the
+        // kernels' 24-bit multiply by ds then only meets pairs of at most
+        // seven squares a half (an index below 2^24)
+        t.kind = uint16_t(s0.kind == 2 && longest[2] == 0 ? 1 : s0.kind);
+        const bool pair = t.kind == 1 || t.kind == 2;
+        if (longest[0] > (pair ? 10u : 20u) || longest[1] > 10 || longest[2] > 10)
+            throw Error(CAD_ERR_PATTERN, "a pattern list too long for an index tile");
+        t.wide = (pair ? longest[0] > 5 || longest[1] > 5 : longest[0] > 10) ? 1 : 0;
+        t.weights = uint32_t(weights.size() / 1024);
+        const size_t at = weights.size();
+        weights.resize(at + 1024 * (t.kind == 2 && t.wide ? 2 : 1), 0);
+        for (int j = 0; j < t.nslots; j++) {
+            const SlotProgram& s = slots[j0 + j];
+            if (!pair) {
+                put(at, j, s.list[0], 0, 0, 4, 1);
+            } else if (t.kind == 1) {
+                put(at, j, s.list[0], 0, 0, 2, 2);
+                put(at, j, s.list[1], 0, 1, 2, 2);
+            } else {
+                put(at, j, s.list[0], 0, 0, 1, 1);
+                put(at, j, s.list[1], 0, 1, 1, 1);
+                put(at, j, s.list[2], 0, 2, 2, 1);
+                if (t.wide) {
+                    put(at + 1024, j, s.list[0], 5, 0, 1, 1);
+                    put(at + 1024, j, s.list[1], 5, 1, 1, 1);
+                }
+            }
+        }
+        tiles.push_back(t);
+    }
+}
+
 // Dynamic LDS a window may use: the device limit minus 1 KB kept for the
 // kernels' static LDS (block-reduction scratch).
 size_t lds_budget(const Context& ctx)

@@ -55,6 +55,23 @@ DBuf to_device(const std::vector<T>& v, hipStream_t s)
 void append_ternary_list(const uint8_t* src, int n, std::vector<uint32_t>& tern, DevTern& t, int l);
 constexpr int kTernPadding = 6;
 
+// The index tiles (IndexTile) of a sequence of slot programs, and their
+// weights (1 KB a tile: lane l's 16 bytes are row l % 16 of the tile, squares
+// 16 (l / 16) .. + 15, byte 4 v + m the square v + 4 m of those, the order the
+// kernels expand a ternary word in).  Slots of one pattern (the same kind,
+// sizes and offset) are taken four at a time.
+struct IndexTiles {
+    std::vector<IndexTile> tiles;
+    std::vector<int8_t> weights;
+    // appends the slots [0, n) of one pattern, slot numbers from `first` on
+    void add(const SlotProgram* slots, int n, int first);
+};
+
+inline TileView tile_view(const DBuf& tiles, const DBuf& weights, const DBuf& dense, int n)
+{
+    return TileView{tiles.as<IndexTile>(), weights.as<uint32_t>(), dense.as<uint32_t>(), n};
+}
+
 // The two-stage scatter of one value size: tiles (window x row chunk) that
 // write partial slices, and the column reduction over the slices.
 struct ScatterLists {
@@ -182,6 +199,9 @@ struct cad_patterns {
     std::unique_ptr<cad::PatternGroup> group;
     cad::DBuf d_slots, d_sq, d_dense;
     cad::DBuf d_tslots, d_tern;             // the ternary-word form of the slot programs
+    cad::DBuf d_tiles, d_weights;           // the slots as index tiles
+    int ntiles = 0;
+    cad::TileView tiles() const { return cad::tile_view(d_tiles, d_weights, d_dense, ntiles); }
     std::vector<uint32_t> slot_lo, slot_hi;  // global column range of every slot
     // scatter plans of the evaluator backward, one per minibatch size
     std::map<int64_t, std::unique_ptr<cad::ScatterPlan>> eval_plans;
@@ -212,7 +232,9 @@ struct cad_matrix {
     int64_t ld = 0;                 // rows rounded up to kIndexAlign (rows r >= rows are zero)
     // matrix-free: the positions and a copy of the pattern group's slot programs
     bool mf = false;
-    cad::DBuf d_pos, d_slots, d_sq, d_dense, d_tslots, d_tern, d_tw;
+    cad::DBuf d_pos, d_slots, d_sq, d_dense, d_tslots, d_tern, d_tw, d_tiles, d_weights;
+    int ntiles = 0;
+    cad::TileView tiles() const { return cad::tile_view(d_tiles, d_weights, d_dense, ntiles); }
     std::vector<uint32_t> slot_lo, slot_hi;
     int nsys = 1;
     std::vector<int64_t> sys_row_begin;  // nsys + 1
