@@ -180,6 +180,8 @@ void upload_programs(cad_patterns* p)
     }
     hipStream_t st = p->ctx->stream;
     p->ntiles = int(it.tiles.size());
+    p->slot_tile.clear();
+    for (size_t t = 0; t < it.tiles.size(); t++) p->slot_tile.insert(p->slot_tile.end(), it.tiles[t].nslots, uint32_t(t));
     p->d_tiles = to_device(it.tiles, st);
     p->d_weights = to_device(it.weights, st);
     p->d_tslots = to_device(tslots, st);
@@ -658,6 +660,7 @@ int cad_matrix_from_positions_mf(cad_patterns* p, const uint64_t* d_pos, int64_t
         copy(m->d_tiles, p->d_tiles);
         copy(m->d_weights, p->d_weights);
         m->ntiles = p->ntiles;
+        m->slot_tile = p->slot_tile;
         copy(m->d_tslots, p->d_tslots);
         copy(m->d_tern, p->d_tern);
         m->d_pos = DBuf(sizeof(uint64_t) * 2 * size_t(n));

@@ -145,7 +145,8 @@ struct GatherStep {
     uint32_t lds_off;  // the segment's offset in the staged phase
     uint32_t width;    // the segment's width (windows of a wide segment)
     uint16_t nwin, wflags;
-    uint32_t pad2[2];
+    uint32_t tile_first;  // matrix-free: the first of the step's index tiles
+    uint32_t pad2;
 };
 static_assert(sizeof(GatherStep) == 64, "GatherStep is one 64-byte scalar load");
 

@@ -241,6 +241,21 @@ __device__ __forceinline__ T uniform_load(const T* p)
     return t;
 }
 
+// A descriptor through the constant address space (scalar loads): for arrays
+// no kernel writes, in kernels without LDS traffic to wait for.
+template <class T>
+__device__ __forceinline__ T constant_load(const T* p)
+{
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    const ConstWords c = (ConstWords)(reinterpret_cast<const uint32_t*>(p));
+    uint32_t r[sizeof(T) / 4];
+#pragma unroll
+    for (int i = 0; i < int(sizeof(T) / 4); i++) r[i] = c[i];
+    T t;
+    __builtin_memcpy(&t, r, sizeof(T));
+    return t;
+}
+
 // Element i of a uint16 array the whole wave reads (the array is padded to
 // whole 32-bit words).
 __device__ __forceinline__ int uniform_u16(const uint16_t* p, int i)
@@ -375,7 +390,13 @@ __device__ __forceinline__ Int4 digits_of_position(const uint64_t* __restrict__ 
     return expand_digits(spread16(h[g]) | (spread16(h[4 + g]) << 1));
 }
 
-// Rows [4j, 4j+4) of four registers of 16-lane groups, transposed: register p
+// The same from the rows' ternary words, tw[r].
+__device__ __forceinline__ Int4 digits_of_words(const uint4* __restrict__ tw, int64_t r)
+{
+    return expand_digits(reinterpret_cast<const uint32_t*>(tw + r)[(threadIdx.x >> 4) & 3]);
+}
+
+// Four registers of 16-lane groups, transposed: register p
 // holding slot g of position set p in lane group g becomes register j holding
 // slot j of position set p in lane group p (lane = position).
 __device__ __forceinline__ void transpose_groups(uint32_t (&r)[4])
@@ -393,12 +414,15 @@ __device__ __forceinline__ void transpose_groups(uint32_t (&r)[4])
 // The pattern-local column of slot g of the tile for the four position sets
 // b[0..4) (idx[p]: lane (n, g) holds slot g of position n of set p; lanes of
 // slots past the tile's hold column 0 of some configuration).
-__device__ __forceinline__ void tile_columns(const IndexTile& t, const TileView& tv, const Int4 (&b)[4],
-                                             uint32_t (&idx)[4])
+__device__ __forceinline__ const Int4* tile_weights(const IndexTile& t, const TileView& tv)
 {
-    const Int4* __restrict__ wt =
-        reinterpret_cast<const Int4*>(tv.weights) + int64_t(t.weights) * 64 + (threadIdx.x & 63);
-    const Int4 w = wt[0], zero = {0, 0, 0, 0};
+    return reinterpret_cast<const Int4*>(tv.weights) + int64_t(t.weights) * 64 + (threadIdx.x & 63);
+}
+
+__device__ __forceinline__ void tile_columns(const IndexTile& t, const TileView& tv, const Int4& w,
+                                             const Int4 (&b)[4], uint32_t (&idx)[4])
+{
+    const Int4 zero = {0, 0, 0, 0};
     Int4 d[4];
 #pragma unroll
     for (int p = 0; p < 4; p++) d[p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w, b[p], zero, 0, 0, 0);
@@ -430,7 +454,7 @@ __device__ __forceinline__ void tile_columns(const IndexTile& t, const TileView&
                 c[p] += __umul24(uint32_t(d[p][3]), 243u);
             }
         } else {
-            const Int4 w2 = wt[64];
+            const Int4 w2 = tile_weights(t, tv)[64];
 #pragma unroll
             for (int p = 0; p < 4; p++) {
                 const Int4 e = __builtin_amdgcn_mfma_i32_16x16x64_i8(w2, b[p], zero, 0, 0, 0);
@@ -450,21 +474,6 @@ __device__ __forceinline__ void tile_columns(const IndexTile& t, const TileView&
         for (int p = 0; p < 4; p++)
             idx[p] = __umul24(idx[p], t.ds) + uint32_t(d[p][2]) + __umul24(uint32_t(d[p][3]), 243u);
     }
-}
-
-// A descriptor through the constant address space (scalar loads): for arrays
-// no kernel writes, in kernels without LDS traffic to wait for.
-template <class T>
-__device__ __forceinline__ T constant_load(const T* p)
-{
-    static_assert(sizeof(T) % 4 == 0, "whole words");
-    const ConstWords c = (ConstWords)(reinterpret_cast<const uint32_t*>(p));
-    uint32_t r[sizeof(T) / 4];
-#pragma unroll
-    for (int i = 0; i < int(sizeof(T) / 4); i++) r[i] = c[i];
-    T t;
-    __builtin_memcpy(&t, r, sizeof(T));
-    return t;
 }
 
 // Pattern/Indexer.cpp InsertIndices for every row, slot-major: out[s * ld + r]
@@ -491,11 +500,12 @@ __global__ __launch_bounds__(kRowBlock) void k_index_extract(const uint64_t* __r
     const int64_t r0 = base + int64_t(lane) * C;
     for (int t = 0; t < tv.n; t++) {
         const IndexTile tl = constant_load(tv.tiles + t);
+        const Int4 wt = *tile_weights(tl, tv);
         const uint32_t off = local ? 0u : tl.col_offset;
         uint32_t v[C][4];
 #pragma unroll
         for (int c = 0; c < C; c++) {
-            tile_columns(tl, tv, b[c], v[c]);
+            tile_columns(tl, tv, wt, b[c], v[c]);
             transpose_groups(v[c]);
         }
 #pragma unroll
@@ -547,7 +557,7 @@ __global__ __launch_bounds__(kRowBlock) void k_index_extract_rows(const uint64_t
     for (int t = 0; t < tv.n; t++) {
         const IndexTile tl = constant_load(tv.tiles + t);
         uint32_t v[4];
-        tile_columns(tl, tv, b, v);
+        tile_columns(tl, tv, *tile_weights(tl, tv), b, v);
         const int g = lane >> 4;
         if (g < tl.nslots) {
 #pragma unroll
@@ -604,6 +614,7 @@ struct PositionsView {
     const DevTern* __restrict__ tslots;  // the ternary-word programs of the same slots
     const uint32_t* __restrict__ tern;
     const uint4* __restrict__ tw;        // every row's ternary words (computed once, at creation)
+    TileView tiles;
     __device__ __forceinline__ uint32_t col(int s, int64_t r) const
     {
         const DevSlot sl = slots[s];
@@ -1349,10 +1360,19 @@ __global__ __launch_bounds__(BS) void k_gather_tile(SlotMajor<IdxT> m, const Row
 
 // The LDS-staged gather of a matrix-free pattern matrix: the stored tile
 // kernel's plan (steps over the slots, narrow segments staged side by side in
-// one phase, wide segments window by window), with each thread's RPT rows'
-// ternary words in registers and every slot's column computed by its program
-// where the stored kernel loads it.  A wide step computes its slots' columns
-// once, before the window loop.
+// one phase, wide segments window by window), with every slot's column
+// computed by its index tile where the stored kernel loads it.  A wave owns
+// 64 rows of each of the block's RPT runs of kTileBlock rows and keeps their
+// digits in registers (16 a run); each tile's columns turn from one slot per
+// 16-lane group to one row per lane, and the row sums run in slot order.  A
+// wide step holds one tile (four slots), its columns computed once, before
+// the window loop.
+// 20M rows of FIT12: 1,021 µs (digit by digit 1,764): 54 % of the cycles issue
+// vector instructions, and staging with its barriers takes about a third (26
+// µs a tile of 2,048 rows when nothing else is done).  Four runs are what the
+// registers hold: with two it takes 1,336 µs; a loop over more rows a block,
+// computing during the staging, and taking the digits anew in every phase so
+// that eight runs fit all spilled or took longer (1,180 to 1,450 µs).
 template <class VT, int RPT, class Epi>
 __global__ __launch_bounds__(kTileBlock) void k_gather_tile_mf(PositionsView m, const RowWork* __restrict__ work,
                                                                const uint32_t* __restrict__ sys_col,
@@ -1367,68 +1387,67 @@ __global__ __launch_bounds__(kTileBlock) void k_gather_tile_mf(PositionsView m, 
     const VT* __restrict__ xb = x + sys_col[w.sys];
     const int64_t r0 = w.row_begin + threadIdx.x;
     const int nval = int(max<int64_t>(0, min<int64_t>(w.row_end - r0, int64_t(RPT) * kTileBlock)));
-    uint32_t T[RPT][4];
+    // the wave's first row of run c: wave0 + c kTileBlock (rows past the tile's
+    // end repeat its last)
+    const int64_t wave0 = w.row_begin + (threadIdx.x & ~63u);
+    Int4 b[RPT][4];
     VT acc[RPT];
 #pragma unroll
-    for (int i = 0; i < RPT; i++) {
-        acc[i] = VT(0);
-        uint4 t = make_uint4(0u, 0u, 0u, 0u);
-        if (i * kTileBlock < nval) t = m.tw[r0 + int64_t(i) * kTileBlock];
-        T[i][0] = t.x;
-        T[i][1] = t.y;
-        T[i][2] = t.z;
-        T[i][3] = t.w;
+    for (int c = 0; c < RPT; c++) {
+        acc[c] = VT(0);
+#pragma unroll
+        for (int p = 0; p < 4; p++)
+            b[c][p] = digits_of_words(m.tw, min(wave0 + int64_t(c) * kTileBlock + 16 * p + int(threadIdx.x & 15),
+                                                w.row_end - 1));
     }
     for (int k = 0; k < nsteps; k++) {
         const GatherStep st = step_at(steps, k);
         if (st.nwin > 1) {
-            // a segment wider than the LDS: the step's columns (segment-local),
-            // then its windows, each slot's value kept until the last window
-            uint32_t c[RPT][kMaxSegSlots];
-            VT v[RPT][kMaxSegSlots];
+            // a segment wider than the LDS: the tile's columns
+            // (segment-local), then the windows, each slot's value kept until
+            // the last window
+            const IndexTile tl = uniform_load(m.tiles.tiles + st.tile_first);
+            const Int4 wt = *tile_weights(tl, m.tiles);
+            const uint32_t off = st.off[0] + tl.col_offset;
+            uint32_t ci[RPT][4];
+            VT v[RPT][4];
 #pragma unroll
-            for (int j = 0; j < kMaxSegSlots; j++) {
+            for (int c = 0; c < RPT; c++) {
+                tile_columns(tl, m.tiles, wt, b[c], ci[c]);
+                transpose_groups(ci[c]);
 #pragma unroll
-                for (int i = 0; i < RPT; i++) {
-                    v[i][j] = VT(0);
-                    c[i][j] = 0xFFFFFFFFu;
-                }
-                if (j < st.nslots) {
-                    const DevSlot sl = uniform_load(m.slots + st.slot_first + j);
-                    uint32_t ci[RPT];
-                    slot_index_rows<RPT>(sl, uniform_load(m.tslots + st.slot_first + j), m.tern, m.dense, T, ci);
-#pragma unroll
-                    for (int i = 0; i < RPT; i++)
-                        if (i * kTileBlock < nval) c[i][j] = st.off[j] + sl.col_offset + ci[i];
+                for (int j = 0; j < 4; j++) {
+                    ci[c][j] += off;
+                    v[c][j] = VT(0);
                 }
             }
             const bool rev = st.wflags & kWideReverse;
             for (uint32_t n = 0; n < st.nwin; n++) {
                 const uint32_t wl = (rev ? st.nwin - 1 - n : n) * wmax;
                 const uint32_t W = min(wmax, st.width - wl);
-                uint32_t h;
-                if (n == 0 && (st.wflags & kWideStaged)) {
-                    h = line_head(xb + st.col_lo + wl);  // staged by the step before
-                } else {
+                const uint32_t h = line_head(xb + st.col_lo + wl);
+                if (n > 0 || !(st.wflags & kWideStaged)) {  // (else staged by the step before)
                     __syncthreads();
-                    h = stage_direct<VT, kTileBlock>(xs, xb + st.col_lo + wl, W);
+                    stage_direct<VT, kTileBlock>(xs, xb + st.col_lo + wl, W);
                     __builtin_amdgcn_s_waitcnt(0);
                     __syncthreads();
                 }
 #pragma unroll
-                for (int j = 0; j < kMaxSegSlots; j++) {
+                for (int j = 0; j < 4; j++) {
+                    if (j < st.nslots) {
 #pragma unroll
-                    for (int i = 0; i < RPT; i++) {
-                        const uint32_t cl = c[i][j] - wl;
-                        if (cl < W) v[i][j] = xs[h + cl];
+                        for (int c = 0; c < RPT; c++) {
+                            const uint32_t cl = ci[c][j] - wl;
+                            if (cl < W) v[c][j] = xs[h + cl];
+                        }
                     }
                 }
             }
 #pragma unroll
-            for (int j = 0; j < kMaxSegSlots; j++)
+            for (int j = 0; j < 4; j++)
                 if (j < st.nslots) {
 #pragma unroll
-                    for (int i = 0; i < RPT; i++) acc[i] += v[i][j];
+                    for (int c = 0; c < RPT; c++) acc[c] += v[c][j];
                 }
         } else {
             if (st.phase_count > 0) {
@@ -1441,23 +1460,26 @@ __global__ __launch_bounds__(kTileBlock) void k_gather_tile_mf(PositionsView m, 
                 __syncthreads();
             }
             const uint32_t h = line_head(xb + st.col_lo);
-            for (int j = 0; j < st.nslots; j++) {
-                const DevSlot sl = uniform_load(m.slots + st.slot_first + j);
-                // (read from the descriptor in memory: a run-time index into
-                // the copy in registers would put the step in scratch)
-                const uint32_t off = __builtin_amdgcn_readfirstlane(steps[k].off[j]) + h + sl.col_offset;
-                uint32_t ci[RPT];
-                slot_index_rows<RPT>(sl, uniform_load(m.tslots + st.slot_first + j), m.tern, m.dense, T, ci);
+            for (int t = 0; 4 * t < st.nslots; t++) {
+                const IndexTile tl = uniform_load(m.tiles.tiles + st.tile_first + t);
+                const Int4 wt = *tile_weights(tl, m.tiles);
+                const uint32_t off = st.off[0] + h + tl.col_offset;
 #pragma unroll
-                for (int i = 0; i < RPT; i++)
-                    if (i * kTileBlock < nval) acc[i] += xs[off + ci[i]];
+                for (int c = 0; c < RPT; c++) {
+                    uint32_t ci[4];
+                    tile_columns(tl, m.tiles, wt, b[c], ci);
+                    transpose_groups(ci);
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        if (j < tl.nslots) acc[c] += xs[off + ci[j]];
+                }
             }
         }
     }
     double red = 0.0;
 #pragma unroll
-    for (int i = 0; i < RPT; i++)
-        if (i * kTileBlock < nval) red += epi.row(r0 + int64_t(i) * kTileBlock, acc[i]);
+    for (int c = 0; c < RPT; c++)
+        if (c * kTileBlock < nval) red += epi.row(r0 + int64_t(c) * kTileBlock, acc[c]);
     reduce_tail<kTileBlock>(epi, red, w.sys, g);
 }
 

@@ -642,7 +642,8 @@ void build_gather_plan(cad_matrix* m, GatherPlan& gp, int vbytes, int rpt, int b
             open_step = -1;
             phase_w = 0;
         }
-        const int per_step = wide ? wide_step_slots(rpt * m->ibytes) : kMaxSegSlots;
+        // (a wide step of a matrix-free matrix is one index tile)
+        const int per_step = !wide ? kMaxSegSlots : m->mf ? 4 : wide_step_slots(rpt * m->ibytes);
         for (int j0 = 0; j0 < sg.nslots; j0 += per_step) {
             GatherStep st{};
             st.slot_first = uint16_t(sg.slot_first + j0);
@@ -652,6 +653,7 @@ void build_gather_plan(cad_matrix* m, GatherPlan& gp, int vbytes, int rpt, int b
             st.nwin = sg.nwin;
             st.phase_first = -1;
             st.phase_count = 0;
+            if (m->mf) st.tile_first = m->slot_tile[size_t(st.slot_first)];
             for (int j = 0; j < st.nslots; j++) {
                 const int slot = st.slot_first + j;
                 st.off[j] = (m->ibytes == 2 ? m->slot_lo[size_t(slot)] : 0u) - sg.col_lo;

@@ -201,6 +201,7 @@ struct cad_patterns {
     cad::DBuf d_tslots, d_tern;             // the ternary-word form of the slot programs
     cad::DBuf d_tiles, d_weights;           // the slots as index tiles
     int ntiles = 0;
+    std::vector<uint32_t> slot_tile;        // the index tile of every slot
     cad::TileView tiles() const { return cad::tile_view(d_tiles, d_weights, d_dense, ntiles); }
     std::vector<uint32_t> slot_lo, slot_hi;  // global column range of every slot
     // scatter plans of the evaluator backward, one per minibatch size
@@ -234,6 +235,7 @@ struct cad_matrix {
     bool mf = false;
     cad::DBuf d_pos, d_slots, d_sq, d_dense, d_tslots, d_tern, d_tw, d_tiles, d_weights;
     int ntiles = 0;
+    std::vector<uint32_t> slot_tile;        // the index tile of every slot
     cad::TileView tiles() const { return cad::tile_view(d_tiles, d_weights, d_dense, ntiles); }
     std::vector<uint32_t> slot_lo, slot_hi;
     int nsys = 1;
