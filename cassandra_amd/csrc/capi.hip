@@ -646,6 +646,9 @@ int cad_matrix_from_positions_mf(cad_patterns* p, const uint64_t* d_pos, int64_t
         std::unique_ptr<cad_matrix> m(new_matrix(p->ctx, n, g.k(), int64_t(g.cols())));
         hipStream_t s = p->ctx->stream;
         m->mf = true;
+        m->tune.pack_slots = kPackSlotsMf;
+        m->splan.row_cost = kMfRowCost;
+        for (const SlotProgram& sl : g.slots) m->splan.slot_cost.push_back(sl.kind == 3 ? kMfDenseCost : 1.0);
         m->ibytes = 0;
         m->slot_lo = p->slot_lo;
         m->slot_hi = p->slot_hi;
@@ -661,6 +664,7 @@ int cad_matrix_from_positions_mf(cad_patterns* p, const uint64_t* d_pos, int64_t
         copy(m->d_weights, p->d_weights);
         m->ntiles = p->ntiles;
         m->slot_tile = p->slot_tile;
+        m->d_slot_tile = to_device(m->slot_tile, s);
         copy(m->d_tslots, p->d_tslots);
         copy(m->d_tern, p->d_tern);
         m->d_pos = DBuf(sizeof(uint64_t) * 2 * size_t(n));
@@ -712,6 +716,7 @@ int cad_matrix_set_schedule(cad_matrix* m, const cad_schedule* sc)
     return guarded([&] {
         need(m != nullptr && sc != nullptr, "null argument");
         TuneParams t;
+        t.pack_slots = m->tune.pack_slots;
         t.rpt4 = sc->gather_f32_rpt;
         t.bs4 = sc->gather_f32_block;
         t.sub4 = sc->gather_f32_sub;

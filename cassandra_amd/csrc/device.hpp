@@ -42,8 +42,8 @@ static_assert(sizeof(DevTern) == 32, "DevTern layout");
 // of five digits: 3^0 .. 3^4, sums up to 242).  What the roles hold:
 //   kind 0 / 3  a = u + 243 v + 3^10 w + 3^15 z (u, v alone unless wide)
 //   kind 1      a = u, b = v; wide: a = u + 243 w, b = v + 243 z
-//   kind 2      a = u, b = v, d = w + 243 z; wide: the next tile's weights
-//               give the upper halves, a = u + 243 u', b = v + 243 v'
+//   kind 2      a = u, b = v, d = w + 243 z; wide: the tile's second block of
+//               weights gives the upper halves, a = u + 243 u', b = v + 243 v'
 // and the column is col_offset + a, dense[a], pair(a, b), pair(a, b) ds + d.
 // Every slot of a tile has the same kind, sizes and offset.
 struct IndexTile {
@@ -52,15 +52,14 @@ struct IndexTile {
     uint32_t hs, ds;
     uint32_t col_offset;
     uint32_t dense_offset;
-    uint32_t weights;  // the tile's weights: 64 lanes x 16 bytes at this tile number
-    uint32_t pad;
+    uint32_t pad[2];
 };
 static_assert(sizeof(IndexTile) == 32, "IndexTile layout");
 
 // The index tiles of a pattern group on the device.
 struct TileView {
     const IndexTile* __restrict__ tiles;
-    const uint32_t* __restrict__ weights;  // 256 words a tile
+    const uint32_t* __restrict__ weights;  // two blocks of 256 words a tile
     const uint32_t* __restrict__ dense;
     int n;
 };

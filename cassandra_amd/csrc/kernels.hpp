@@ -414,12 +414,14 @@ __device__ __forceinline__ void transpose_groups(uint32_t (&r)[4])
 // The pattern-local column of slot g of the tile for the four position sets
 // b[0..4) (idx[p]: lane (n, g) holds slot g of position n of set p; lanes of
 // slots past the tile's hold column 0 of some configuration).
-__device__ __forceinline__ const Int4* tile_weights(const IndexTile& t, const TileView& tv)
+// Tile t's weights (two blocks of 64 a tile, the second for wide pairs with a
+// diagonal).
+__device__ __forceinline__ const Int4* tile_weights(int t, const TileView& tv)
 {
-    return reinterpret_cast<const Int4*>(tv.weights) + int64_t(t.weights) * 64 + (threadIdx.x & 63);
+    return reinterpret_cast<const Int4*>(tv.weights) + (128 * t + int(threadIdx.x & 63));
 }
 
-__device__ __forceinline__ void tile_columns(const IndexTile& t, const TileView& tv, const Int4& w,
+__device__ __forceinline__ void tile_columns(const IndexTile& t, int number, const TileView& tv, const Int4& w,
                                              const Int4 (&b)[4], uint32_t (&idx)[4])
 {
     const Int4 zero = {0, 0, 0, 0};
@@ -454,7 +456,7 @@ __device__ __forceinline__ void tile_columns(const IndexTile& t, const TileView&
                 c[p] += __umul24(uint32_t(d[p][3]), 243u);
             }
         } else {
-            const Int4 w2 = tile_weights(t, tv)[64];
+            const Int4 w2 = tile_weights(number, tv)[64];
 #pragma unroll
             for (int p = 0; p < 4; p++) {
                 const Int4 e = __builtin_amdgcn_mfma_i32_16x16x64_i8(w2, b[p], zero, 0, 0, 0);
@@ -474,6 +476,35 @@ __device__ __forceinline__ void tile_columns(const IndexTile& t, const TileView&
         for (int p = 0; p < 4; p++)
             idx[p] = __umul24(idx[p], t.ds) + uint32_t(d[p][2]) + __umul24(uint32_t(d[p][3]), 243u);
     }
+}
+
+// A tile's descriptor and weights on their way from memory, in vector registers
+// (the descriptor the same in every lane): loaded a tile ahead, they are in
+// flight while the tile before is used, and their wait is not one for the LDS.
+struct TileRegs {
+    Int4 desc[2];
+    Int4 weights;
+    __device__ __forceinline__ IndexTile tile() const
+    {
+        uint32_t r[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) r[i] = __builtin_amdgcn_readfirstlane(uint32_t(desc[i >> 2][i & 3]));
+        IndexTile t;
+        __builtin_memcpy(&t, r, sizeof(t));
+        return t;
+    }
+};
+
+__device__ __forceinline__ TileRegs load_tile(const TileView& tv, int t)
+{
+    TileRegs r;
+    int v = 0;
+    asm volatile("" : "+v"(v));  // a vector load
+    const Int4* __restrict__ d = reinterpret_cast<const Int4*>(tv.tiles + t) + v;
+    r.desc[0] = d[0];
+    r.desc[1] = d[1];
+    r.weights = *tile_weights(t, tv);
+    return r;
 }
 
 // Pattern/Indexer.cpp InsertIndices for every row, slot-major: out[s * ld + r]
@@ -500,12 +531,12 @@ __global__ __launch_bounds__(kRowBlock) void k_index_extract(const uint64_t* __r
     const int64_t r0 = base + int64_t(lane) * C;
     for (int t = 0; t < tv.n; t++) {
         const IndexTile tl = constant_load(tv.tiles + t);
-        const Int4 wt = *tile_weights(tl, tv);
+        const Int4 wt = *tile_weights(t, tv);
         const uint32_t off = local ? 0u : tl.col_offset;
         uint32_t v[C][4];
 #pragma unroll
         for (int c = 0; c < C; c++) {
-            tile_columns(tl, tv, wt, b[c], v[c]);
+            tile_columns(tl, t, tv, wt, b[c], v[c]);
             transpose_groups(v[c]);
         }
 #pragma unroll
@@ -557,7 +588,7 @@ __global__ __launch_bounds__(kRowBlock) void k_index_extract_rows(const uint64_t
     for (int t = 0; t < tv.n; t++) {
         const IndexTile tl = constant_load(tv.tiles + t);
         uint32_t v[4];
-        tile_columns(tl, tv, *tile_weights(tl, tv), b, v);
+        tile_columns(tl, t, tv, *tile_weights(t, tv), b, v);
         const int g = lane >> 4;
         if (g < tl.nslots) {
 #pragma unroll
@@ -615,6 +646,11 @@ struct PositionsView {
     const uint32_t* __restrict__ tern;
     const uint4* __restrict__ tw;        // every row's ternary words (computed once, at creation)
     TileView tiles;
+    const uint32_t* __restrict__ slot_tiles;  // the index tile of every slot
+    __device__ __forceinline__ int slot_tile(int s) const
+    {
+        return __builtin_amdgcn_readfirstlane(int(slot_tiles[s]));
+    }
     __device__ __forceinline__ uint32_t col(int s, int64_t r) const
     {
         const DevSlot sl = slots[s];
@@ -1407,13 +1443,13 @@ __global__ __launch_bounds__(kTileBlock) void k_gather_tile_mf(PositionsView m, 
             // (segment-local), then the windows, each slot's value kept until
             // the last window
             const IndexTile tl = uniform_load(m.tiles.tiles + st.tile_first);
-            const Int4 wt = *tile_weights(tl, m.tiles);
+            const Int4 wt = *tile_weights(int(st.tile_first), m.tiles);
             const uint32_t off = st.off[0] + tl.col_offset;
             uint32_t ci[RPT][4];
             VT v[RPT][4];
 #pragma unroll
             for (int c = 0; c < RPT; c++) {
-                tile_columns(tl, m.tiles, wt, b[c], ci[c]);
+                tile_columns(tl, int(st.tile_first), m.tiles, wt, b[c], ci[c]);
                 transpose_groups(ci[c]);
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
@@ -1461,13 +1497,14 @@ __global__ __launch_bounds__(kTileBlock) void k_gather_tile_mf(PositionsView m, 
             }
             const uint32_t h = line_head(xb + st.col_lo);
             for (int t = 0; 4 * t < st.nslots; t++) {
-                const IndexTile tl = uniform_load(m.tiles.tiles + st.tile_first + t);
-                const Int4 wt = *tile_weights(tl, m.tiles);
+                const int number = int(st.tile_first) + t;
+                const IndexTile tl = uniform_load(m.tiles.tiles + number);
+                const Int4 wt = *tile_weights(number, m.tiles);
                 const uint32_t off = st.off[0] + h + tl.col_offset;
 #pragma unroll
                 for (int c = 0; c < RPT; c++) {
                     uint32_t ci[4];
-                    tile_columns(tl, m.tiles, wt, b[c], ci);
+                    tile_columns(tl, number, m.tiles, wt, b[c], ci);
                     transpose_groups(ci);
 #pragma unroll
                     for (int j = 0; j < 4; j++)
@@ -1627,6 +1664,37 @@ __device__ __forceinline__ WT window_term(double v, double fscale)
         return v;
     else
         return WT(__double2ll_rn(v * fscale));
+}
+
+// The fixed-point scale of a block's window (0: the FP64 window): of FP32
+// windows, from the system's max |y| -- formed here from the row blocks' maxima
+// where the instantiation says so -- or LSQR's bound.
+template <class VT, int BS, bool kYmax>
+__device__ __forceinline__ double window_scale(const FixedScale& fx, int sys, VT sc, bool allowed = true)
+{
+    if constexpr (!std::is_same_v<VT, float>) {
+        return 0.0;
+    } else if constexpr (kYmax) {
+        __shared__ unsigned shm[BS / 64];
+        const unsigned b = system_max<BS>(fx, sys, shm);
+        return allowed ? fixed_scale_bits(fx.cbits, true, b, double(sc)) : 0.0;
+    } else {
+        return allowed ? fixed_scale(fx, sys, double(sc)) : 0.0;
+    }
+}
+
+// A finished window as a partial slice.
+template <class VT>
+__device__ __forceinline__ void store_window(const double* __restrict__ win, uint32_t W, double fscale,
+                                             VT* __restrict__ out)
+{
+    if (fscale > 0.0) {
+        const unsigned long long* wu = reinterpret_cast<const unsigned long long*>(win);
+        const double inv = 1.0 / fscale;  // a power of two: exact
+        for (uint32_t i = threadIdx.x; i < W; i += kScatterBlock) out[i] = VT(double((long long)wu[i]) * inv);
+    } else {
+        for (uint32_t i = threadIdx.x; i < W; i += kScatterBlock) out[i] = VT(win[i]);
+    }
 }
 
 // max |VT(y)| as float bits (non-negative floats order as unsigned integers;
@@ -1820,14 +1888,7 @@ __global__ __launch_bounds__(kScatterBlock) void k_scatter_tile(SlotMajor<IdxT> 
     const VT sc = scatter_scale<VT, kScatterBlock, kBeta>(div, mode, w.sys, bsum);
     const int64_t vld = m.ld / RPT;
     // FP32 windows accumulate in fixed point where the scale allows it
-    double fscale = 0.0;
-    if constexpr (kYmax) {
-        __shared__ unsigned shm[kScatterBlock / 64];
-        const unsigned b = system_max<kScatterBlock>(fx, w.sys, shm);
-        if (std::is_same_v<VT, float> && ns <= kMaxSegSlots) fscale = fixed_scale_bits(fx.cbits, true, b, double(sc));
-    } else {
-        fscale = std::is_same_v<VT, float> && ns <= kMaxSegSlots ? fixed_scale(fx, w.sys, double(sc)) : 0.0;
-    }
+    const double fscale = window_scale<VT, kScatterBlock, kYmax>(fx, w.sys, sc, ns <= kMaxSegSlots);
     if (ns <= kMaxSegSlots) {
         int64_t slot[kMaxSegSlots];
         uint32_t off[kMaxSegSlots];
@@ -1898,20 +1959,18 @@ __global__ __launch_bounds__(kScatterBlock) void k_scatter_tile(SlotMajor<IdxT> 
         }
     }
     __syncthreads();
-    VT* __restrict__ out = part + w.part_off;
-    if (fscale > 0.0) {
-        const unsigned long long* wu = reinterpret_cast<const unsigned long long*>(win);
-        const double inv = 1.0 / fscale;  // a power of two: exact
-        for (uint32_t i = threadIdx.x; i < W; i += kScatterBlock) out[i] = VT(double((long long)wu[i]) * inv);
-    } else {
-        for (uint32_t i = threadIdx.x; i < W; i += kScatterBlock) out[i] = VT(win[i]);
-    }
+    store_window<VT>(win, W, fscale, part + w.part_off);
 }
 
-// Stage 1 for a matrix-free matrix: as k_scatter_tile, with each thread's RPT
-// positions loaded once per step and every slot's column computed by its
-// program (the DevSlot is the same for the whole block).
-template <class VT, class YT, int RPT, bool kBeta = false>
+// Stage 1 for a matrix-free matrix: as k_scatter_tile, with every slot's column
+// computed by its index tile.  A wave takes RPT runs of 64 rows a step; the
+// columns turn from one slot per 16-lane group to one row per lane.  A group's
+// slots are runs of whole patterns, so its tiles follow each other.  FP32
+// windows accumulate in fixed point as k_scatter_tile's do.  20M rows of
+// FIT12: 1,430 µs (2,537 with the lists evaluated digit by digit into FP64
+// windows), bound by vector issue: a tile of a 32-slot group takes 395 cycles
+// of a SIMD per 64 rows, about 75 instructions.
+template <class VT, class YT, int RPT, bool kBeta = false, bool kYmax = false>
 __global__ __launch_bounds__(kScatterBlock) void k_scatter_tile_mf(PositionsView m,
                                                                    const ScatterWork* __restrict__ work,
                                                                    const SlotGroup* __restrict__ groups,
@@ -1922,7 +1981,7 @@ __global__ __launch_bounds__(kScatterBlock) void k_scatter_tile_mf(PositionsView
                                                                    VT* __restrict__ part, GridSys bsum)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    double* win = reinterpret_cast<double*>(smem_raw);
+    double* win = reinterpret_cast<double*>(smem_raw);  // 8-byte window words (FP64 or fixed point)
     const ScatterWork w = uniform_load(work + blockIdx.x);
     if (!scatter_selected(div, mode, w.sys)) return;
     const uint32_t W = w.win_hi - w.win_lo;
@@ -1931,40 +1990,89 @@ __global__ __launch_bounds__(kScatterBlock) void k_scatter_tile_mf(PositionsView
     const SlotGroup gr = uniform_load(groups + w.group);
     const uint32_t cb = sys_col[w.sys];
     const VT sc = scatter_scale<VT, kScatterBlock, kBeta>(div, mode, w.sys, bsum);
-    const int64_t last = w.row_end - 1;
-    for (int64_t a = (w.row_begin & ~int64_t(RPT - 1)) + int64_t(RPT) * threadIdx.x; a < w.row_end;
-         a += int64_t(RPT) * kScatterBlock) {
-        bool ok[RPT];
-        double yv[RPT];
-        uint32_t T[RPT][4];
+    const double fscale = window_scale<VT, kScatterBlock, kYmax>(fx, w.sys, sc);
+    // the group's tiles: ntile of them, gr.nslots slots in all
+    const int first = uniform_u16(slot_list, gr.first);
+    const int tile0 = m.slot_tile(first), ntile = m.slot_tile(first + gr.nslots - 1) - tile0 + 1;
+    const int lane = threadIdx.x & 63;
+    auto rows = [&](auto* wn) {
+        using WT = std::remove_pointer_t<decltype(wn)>;
+        // Run c of a step: the wave's rows a + c kScatterBlock + [0, 64).  The
+        // next step's words and y load while this one is added.
+        uint32_t tn[RPT][4];
+        YT yn[RPT];
+        auto load = [&](int64_t a) {
+            const uint32_t* __restrict__ tw = reinterpret_cast<const uint32_t*>(m.tw + a);
+            const YT* __restrict__ ya = y + a;
+            const int last = int(min<int64_t>(w.row_end - a, int64_t(RPT) * kScatterBlock)) - 1;
+            if (last >= (RPT - 1) * kScatterBlock + 63) {
 #pragma unroll
-        for (int i = 0; i < RPT; i++) {
-            ok[i] = a + i >= w.row_begin && a + i < w.row_end;
-            const int64_t r = min(a + i, last);  // clamped: no branch around the loads
-            const double t = double(VT(y[r]) * sc);
-            yv[i] = ok[i] ? t : 0.0;
-            const uint4 tw = m.tw[r];
-            T[i][0] = tw.x;
-            T[i][1] = tw.y;
-            T[i][2] = tw.z;
-            T[i][3] = tw.w;
-        }
-        for (int j = 0; j < gr.nslots; j++) {
-            const int sj = uniform_u16(slot_list, gr.first + j);
-            const DevSlot sl = uniform_load(m.slots + sj);
-            const uint32_t o = cb + sl.col_offset - w.win_lo;
-            uint32_t ci[RPT];
-            slot_index_rows<RPT>(sl, uniform_load(m.tslots + sj), m.tern, m.dense, T, ci);
+                for (int c = 0; c < RPT; c++) {
 #pragma unroll
-            for (int i = 0; i < RPT; i++) {
-                const uint32_t uc = o + ci[i];
-                if (ok[i] && uc < W) atomicAdd(&win[uc], yv[i]);
+                    for (int p = 0; p < 4; p++)
+                        tn[c][p] = tw[uint32_t(4 * (lane & 15) + (lane >> 4)) + uint32_t(4 * (c * kScatterBlock + 16 * p))];
+                    yn[c] = ya[uint32_t(lane) + uint32_t(c * kScatterBlock)];
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < RPT; c++) {
+#pragma unroll
+                    for (int p = 0; p < 4; p++)
+                        tn[c][p] = tw[4 * min(c * kScatterBlock + 16 * p + (lane & 15), last) + (lane >> 4)];
+                    yn[c] = ya[min(c * kScatterBlock + lane, last)];
+                }
+            }
+        };
+        // (the wave's rows through scalar registers: its addresses are a
+        // scalar base and one offset)
+        int64_t a = w.row_begin + __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u);
+        if (a >= w.row_end) return;
+        load(a);
+        TileRegs tr = load_tile(m.tiles, tile0);
+        int at = 0;
+        for (; a < w.row_end; a += RPT * kScatterBlock) {
+            Int4 b[RPT][4];
+            WT yv[RPT];
+            bool ok[RPT];
+#pragma unroll
+            for (int c = 0; c < RPT; c++) {
+#pragma unroll
+                for (int p = 0; p < 4; p++) b[c][p] = expand_digits(tn[c][p]);
+                ok[c] = a + c * kScatterBlock + lane < w.row_end;
+                yv[c] = window_term<WT>(double(VT(yn[c]) * sc), fscale);
+            }
+            if (a + RPT * kScatterBlock < w.row_end) load(a + RPT * kScatterBlock);
+            for (int t = 0; t < ntile; t++) {
+                const IndexTile tl = tr.tile();
+                const Int4 wt = tr.weights;
+                const int number = tile0 + at;
+                at = at + 1 < ntile ? at + 1 : 0;
+                tr = load_tile(m.tiles, tile0 + at);
+                const uint32_t off = cb + tl.col_offset - w.win_lo;
+#pragma unroll
+                for (int c = 0; c < RPT; c++) {
+                    uint32_t ci[4];
+                    tile_columns(tl, number, m.tiles, wt, b[c], ci);
+                    transpose_groups(ci);
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const uint32_t uc = off + ci[j];
+                        if (j < tl.nslots && ok[c] && uc < W) atomicAdd(&wn[uc], yv[c]);
+                    }
+                }
             }
         }
+    };
+    if constexpr (std::is_same_v<VT, float>) {
+        if (fscale > 0.0)
+            rows(reinterpret_cast<unsigned long long*>(win));
+        else
+            rows(win);
+    } else {
+        rows(win);
     }
     __syncthreads();
-    VT* __restrict__ out = part + w.part_off;
-    for (uint32_t i = threadIdx.x; i < W; i += kScatterBlock) out[i] = VT(win[i]);
+    store_window<VT>(win, W, fscale, part + w.part_off);
 }
 
 // Stage 2: z[c] = sum of the window's chunk slices, in chunk order

@@ -134,7 +134,7 @@ void make_groups(const std::vector<uint32_t>& lo, const std::vector<uint32_t>& h
 
 // The scatter groups of a window size (ScatterLists::groups).  Pattern
 // groups come in column order and never overlap.
-void pack_groups(const ScatterPlan& sp, uint32_t wmax, ScatterLists& L)
+void pack_groups(const ScatterPlan& sp, uint32_t wmax, int max_slots, ScatterLists& L)
 {
     L.groups.clear();
     L.slot_list.clear();
@@ -146,7 +146,7 @@ void pack_groups(const ScatterPlan& sp, uint32_t wmax, ScatterLists& L)
         if (g.col_hi - g.col_lo <= wmax)
             for (; j < sp.groups.size(); j++) {
                 const SlotGroup& h = sp.groups[j];
-                if (h.col_lo < g.col_hi || h.col_hi - g.col_lo > wmax || g.nslots + h.nslots > kMaxSegSlots) break;
+                if (h.col_lo < g.col_hi || h.col_hi - g.col_lo > wmax || g.nslots + h.nslots > max_slots) break;
                 slots.insert(slots.end(), sp.slot_list.begin() + h.first, sp.slot_list.begin() + h.first + h.nslots);
                 g.col_hi = h.col_hi;
                 g.nslots = uint16_t(g.nslots + h.nslots);
@@ -311,14 +311,21 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
     L.work.clear();
     L.reduce.clear();
     L.widest = 0;
-    pack_groups(sp, wmax, L);
+    pack_groups(sp, wmax, tune.pack_slots, L);
     const int nsys = int(sys_col.size());
     auto in = [&](int s) { return !on || (*on)[size_t(s)] != 0; };
     // Work of a window per row: its slot loads, and its atomics -- the share
     // of the group's entries that fall into the window, taken as its share of
     // the group's columns.  scatter_balance weighs the two (1: loads only).
     const double lam = std::min(1.0, std::max(0.0, tune.scatter_balance));
+    // (Matrix-free: a slot's columns are computed whether or not they fall into
+    // the window, ScatterPlan::slot_cost, after the row's digits, row_cost.)
     auto win_cost = [&](const SlotGroup& g, uint32_t W) {
+        if (!sp.slot_cost.empty() && vbytes == 8) {
+            double c = sp.row_cost;
+            for (int j = 0; j < g.nslots; j++) c += sp.slot_cost[L.slot_list[size_t(g.first + j)]];
+            return c;
+        }
         const double frac = double(W) / double(std::max<uint32_t>(1, g.col_hi - g.col_lo));
         return g.nslots * (lam + (1.0 - lam) * frac);
     };
@@ -493,9 +500,8 @@ void IndexTiles::add(const SlotProgram* slots, int n, int first)
         if (longest[0] > (pair ? 10u : 20u) || longest[1] > 10 || longest[2] > 10)
             throw Error(CAD_ERR_PATTERN, "a pattern list too long for an index tile");
         t.wide = (pair ? longest[0] > 5 || longest[1] > 5 : longest[0] > 10) ? 1 : 0;
-        t.weights = uint32_t(weights.size() / 1024);
         const size_t at = weights.size();
-        weights.resize(at + 1024 * (t.kind == 2 && t.wide ? 2 : 1), 0);
+        weights.resize(at + 2048, 0);
         for (int j = 0; j < t.nslots; j++) {
             const SlotProgram& s = slots[j0 + j];
             if (!pair) {
@@ -542,6 +548,7 @@ void build_scatter_plan(ScatterPlan& sp, const std::vector<uint32_t>& lo, const 
     t4.blocks_per_cu = std::max(4.0, tune.blocks_per_cu);
     t4.partial_cap = 1.0;
     t4.scatter_balance = 1.0;
+    t4.pack_slots = kMaxSegSlots;  // (the count kernel holds a group's slots in registers)
     make_scatter_lists(sp, sys_rows, sys_col, cols_per_sys, uint32_t(lds / 4), 4, ibytes, ctx.cus, t4, sp.f4);
     make_scatter_lists(sp, sys_rows, sys_col, cols_per_sys, uint32_t(lds / 8), 8, ibytes, ctx.cus, tune, sp.f8);
     const int nsys = int(sys_rows.size()) - 1;

@@ -56,7 +56,7 @@ void append_ternary_list(const uint8_t* src, int n, std::vector<uint32_t>& tern,
 constexpr int kTernPadding = 6;
 
 // The index tiles (IndexTile) of a sequence of slot programs, and their
-// weights (1 KB a tile: lane l's 16 bytes are row l % 16 of the tile, squares
+// weights (two blocks of 1 KB a tile: lane l's 16 bytes are row l % 16 of the tile, squares
 // 16 (l / 16) .. + 15, byte 4 v + m the square v + 4 m of those, the order the
 // kernels expand a ternary word in).  Slots of one pattern (the same kind,
 // sizes and offset) are taken four at a time.
@@ -101,6 +101,10 @@ struct ScatterPlan {
     std::vector<uint16_t> slot_list;
     DBuf d_groups, d_slot_list;
     ScatterLists f4, f8;  // float and double (and uint32 counts) windows
+    // a window's time per row, where it is not the number of its slots
+    // (matrix-free): of each slot, and of the row itself
+    std::vector<double> slot_cost;
+    double row_cost = 0.0;
     DBuf d_ymax;          // per system: bits of max |y| of the last FP32 scatter (fixed-point scale)
     DBuf d_ymax_part;     // the same per row block of the grid plan
 };
@@ -146,8 +150,20 @@ struct TuneParams {
     double partial_cap = 1.0;   // partial-slice traffic cap as a fraction of index traffic
     int scatter_order = 0;      // 0: chunks per window by work share; 1: shared chunks, XCD-major
     double scatter_balance = 1.0; // order 0: weight of slot loads against atomics in a window's work (1: loads)
+    int pack_slots = kMaxSegSlots; // most slots of narrow groups that share a window
     double small_floor_bytes = 8.0 * 1024 * 1024;  // partial slices a window may take to spread a small system
 };
+
+// Most slots sharing a window of a matrix-free scatter: its rows' digits are
+// expanded once for all of them.
+constexpr int kPackSlotsMf = 32;
+
+// Time of a matrix-free scatter window per row, in units of one slot: a group
+// of 32 slots took 24.7 cycles per 64 rows and slot, one of 8 slots 29, of 4
+// slots 44, and one with two slots of dense tables (a lookup each) 48 for 6.
+// With windows weighed by their slots alone the longest tile took 4.68 million
+// cycles and the mean 3.05 (20M rows of FIT12).
+constexpr double kMfRowCost = 3.5, kMfDenseCost = 2.5;
 
 // A matrix (or, in a batch, the systems still iterating) of at most this many
 // rows gathers with the row kernel: a staged tile costs about the same (≈22
@@ -233,7 +249,7 @@ struct cad_matrix {
     int64_t ld = 0;                 // rows rounded up to kIndexAlign (rows r >= rows are zero)
     // matrix-free: the positions and a copy of the pattern group's slot programs
     bool mf = false;
-    cad::DBuf d_pos, d_slots, d_sq, d_dense, d_tslots, d_tern, d_tw, d_tiles, d_weights;
+    cad::DBuf d_pos, d_slots, d_sq, d_dense, d_tslots, d_tern, d_tw, d_tiles, d_weights, d_slot_tile;
     int ntiles = 0;
     std::vector<uint32_t> slot_tile;        // the index tile of every slot
     cad::TileView tiles() const { return cad::tile_view(d_tiles, d_weights, d_dense, ntiles); }

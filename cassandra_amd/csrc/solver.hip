@@ -21,7 +21,7 @@ void with_view(cad_matrix* m, F&& f)
     if (m->mf)
         f(PositionsView{m->d_pos.as<uint64_t>(), m->d_slots.as<DevSlot>(), m->d_sq.as<uint8_t>(),
                         m->d_dense.as<uint32_t>(), m->d_tslots.as<DevTern>(), m->d_tern.as<uint32_t>(),
-                        m->d_tw.as<uint4>(), m->tiles()});
+                        m->d_tw.as<uint4>(), m->tiles(), m->d_slot_tile.as<uint32_t>()});
     else if (m->ibytes == 2)
         f(SlotMajor<uint16_t>{m->d_idx.as<uint16_t>(), m->ld, m->d_base.as<uint32_t>()});
     else
@@ -84,11 +84,11 @@ PT* partials(ScatterLists& L)
 // A^T y in two launches: LDS window tiles into partial slices, then the
 // column reduction in chunk order (which writes every column of z).
 // The first-stage scatter kernel of a view: vector loads of rpt (4, or 8 for
-// u16 indices) consecutive rows for stored indices, 4 positions per step for
-// a matrix-free matrix, one row per step otherwise; f receives the kernel.
-// beta: the instantiation that forms an LSQR iteration's beta itself; ymax:
-// the stored-index instantiation that forms each system's max |y| from the
-// row-block maxima (FixedScale::ypart), used by FP32 PCG.
+// u16 indices) consecutive rows for stored indices, two runs of 64 rows a wave
+// and step for a matrix-free matrix, one row per step otherwise; f receives the
+// kernel.  beta: the instantiation that forms an LSQR iteration's beta itself;
+// ymax: the instantiation that forms each system's max |y| from the row-block
+// maxima (FixedScale::ypart), used by FP32 PCG.
 template <class VT, class YT, class View, class F>
 void with_scatter_kernel(int rpt, bool beta, bool ymax, F&& f)
 {
@@ -100,7 +100,7 @@ void with_scatter_kernel(int rpt, bool beta, bool ymax, F&& f)
         } else if constexpr (std::is_same_v<View, SlotMajor<uint32_t>>) {
             return f(k_scatter_tile<VT, YT, uint32_t, 4, B, Y>);
         } else if constexpr (std::is_same_v<View, PositionsView>) {
-            return f(k_scatter_tile_mf<VT, YT, 4, B>);
+            return f(k_scatter_tile_mf<VT, YT, 2, B, Y>);
         } else {
             return f(k_scatter_part<VT, YT, View, B>);
         }
@@ -117,7 +117,8 @@ template <class VT, class View>
 constexpr bool fixed_point_scatter()
 {
     return std::is_same_v<VT, float> &&
-           (std::is_same_v<View, SlotMajor<uint16_t>> || std::is_same_v<View, SlotMajor<uint32_t>>);
+           (std::is_same_v<View, SlotMajor<uint16_t>> || std::is_same_v<View, SlotMajor<uint32_t>> ||
+            std::is_same_v<View, PositionsView>);
 }
 
 template <class YT>
