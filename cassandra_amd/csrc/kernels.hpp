@@ -1381,6 +1381,179 @@ __device__ __forceinline__ void gather_tile_sub(const SlotMajor<IdxT>& m, const 
     reduce_tail<BS>(epi, red, w.sys, g);
 }
 
+// The stored gather over long tiles: as gather_tile_single, with R runs of
+// kTileBlock * RPT rows a tile that share every staging, wide segments too
+// (their windows are walked once for all runs, in steps of kWide slots whose
+// values stay in registers).  A staging costs a CU about 2 µs (160 KB through
+// the L2, two barriers, the latency) whatever the rows it serves, and a block
+// its start and end; so a CU's rows are one tile where the registers allow
+// it.  (5M rows of FIT8: FP64 165 µs against 334 with 2,048 rows a tile, FP32
+// 99 against 121 with three tiles a CU; 1.2M rows of edax in FP64 46 against
+// 102.)  Steps hold at most kLongStep slots; the entries of the next (step, run)
+// load while this one sums.  Entries of rows outside the tile are read like
+// the others (they are valid columns) and their sums dropped.
+template <class VT, int RPT, class IdxT, class Epi, int R, int kWide>
+__device__ __forceinline__ double gather_long(const SlotMajor<IdxT>& m, const RowWork& w,
+                                              const GatherStep* __restrict__ steps, int nsteps,
+                                              const PhaseSeg* __restrict__ phases, uint32_t wmax,
+                                              const VT* __restrict__ xb, VT* __restrict__ xs, Epi& epi)
+{
+    using V = IdxVec<IdxT, RPT>;
+    using VecT = typename V::T;
+    constexpr int kSub = RPT * kTileBlock;
+    const int64_t a0 = (w.row_begin & ~int64_t(RPT - 1)) + int64_t(RPT) * threadIdx.x;
+    const int64_t vld = m.ld / RPT;
+    VT acc[R][RPT];
+#pragma unroll
+    for (int u = 0; u < R; u++)
+#pragma unroll
+        for (int i = 0; i < RPT; i++) acc[u][i] = VT(0);
+    // up to N slots of step st of run u (threads past the tile read its first
+    // rows; slots past the step's last repeat it)
+    auto load = [&](auto& q, const GatherStep& st, int u) {
+        const int64_t a = a0 + u * kSub;
+        const VecT* __restrict__ v = reinterpret_cast<const VecT*>(m.idx + (a < w.row_end ? a : (w.row_begin & ~int64_t(RPT - 1))));
+        constexpr int N = sizeof(q) / sizeof(q[0]);
+#pragma unroll
+        for (int j = 0; j < N; j++) q[j] = v[int64_t(st.slot_first + min(j, st.nslots - 1)) * vld];
+    };
+    VecT q[kLongStep];
+    GatherStep st = step_at(steps, 0);
+    bool have = false;  // q holds run 0's entries of this step
+    for (int k = 0; k < nsteps; k++) {
+        const bool more = k + 1 < nsteps;
+        const GatherStep nx = step_at(steps, more ? k + 1 : k);
+        if (st.nwin > 1) {
+            VecT qw[R][kWide];
+            VT v[R][RPT][kWide];
+#pragma unroll
+            for (int u = 0; u < R; u++) {
+                load(qw[u], st, u);
+#pragma unroll
+                for (int i = 0; i < RPT; i++)
+#pragma unroll
+                    for (int j = 0; j < kWide; j++) v[u][i][j] = VT(0);
+            }
+            const bool rev = st.wflags & kWideReverse;
+            for (uint32_t n = 0; n < st.nwin; n++) {
+                const uint32_t wl = (rev ? st.nwin - 1 - n : n) * wmax;
+                const uint32_t W = min(wmax, st.width - wl);
+                const uint32_t h = line_head(xb + st.col_lo + wl);
+                if (n > 0 || !(st.wflags & kWideStaged)) {  // (else staged by the step before)
+                    __syncthreads();
+                    stage_direct<VT, kTileBlock>(xs, xb + st.col_lo + wl, W);
+                    __builtin_amdgcn_s_waitcnt(0);
+                    __syncthreads();
+                }
+#pragma unroll
+                for (int u = 0; u < R; u++) {
+#pragma unroll
+                    for (int j = 0; j < kWide; j++) {
+                        if (j < st.nslots) {
+                            // 32-bit offset: base - col_lo wraps for u32
+                            // storage (base 0) and the sum with the entry
+                            // unwraps it
+                            const uint32_t off = st.off[j] - wl;
+#pragma unroll
+                            for (int i = 0; i < RPT; i++) {
+                                const uint32_t c = off + V::get(qw[u][j], i);
+                                const VT t = xs[h + (c < W ? c : 0u)];
+                                v[u][i][j] = c < W ? t : v[u][i][j];
+                            }
+                        }
+                    }
+                }
+            }
+            // the next step's entries, unless it is a step of this kind
+            have = more && nx.nwin <= 1;
+            if (have) load(q, nx, 0);
+#pragma unroll
+            for (int j = 0; j < kWide; j++)
+                if (j < st.nslots) {
+#pragma unroll
+                    for (int u = 0; u < R; u++)
+#pragma unroll
+                        for (int i = 0; i < RPT; i++) acc[u][i] += v[u][i][j];
+                }
+        } else {
+            if (!have) load(q, st, 0);
+            if (st.phase_count > 0) {
+                __syncthreads();
+                for (int p = st.phase_first; p < st.phase_first + st.phase_count; p++) {
+                    const PhaseSeg ps = phases[p];
+                    stage_direct<VT, kTileBlock>(xs + ps.lds_off, xb + ps.col_lo, ps.width);
+                }
+                __builtin_amdgcn_s_waitcnt(0);
+                __syncthreads();
+            }
+            const uint32_t h = line_head(xb + st.col_lo);
+            have = more && nx.nwin <= 1;
+#pragma unroll
+            for (int u = 0; u < R; u++) {
+                // this run's entries must be in before the next loads go out:
+                // the compiler's own wait for them would be one for all
+                __builtin_amdgcn_s_waitcnt(0);
+                VecT qn[kLongStep];
+                if (u + 1 < R) load(qn, st, u + 1);
+                else if (have) load(qn, nx, 0);
+#pragma unroll
+                for (int j = 0; j < kLongStep; j++) {
+                    if (j < st.nslots) {
+                        const uint32_t off = st.off[j] + h;
+#pragma unroll
+                        for (int i = 0; i < RPT; i++) acc[u][i] += xs[off + V::get(q[j], i)];
+                    }
+                }
+                if (u + 1 < R || have) {
+#pragma unroll
+                    for (int j = 0; j < kLongStep; j++) q[j] = qn[j];
+                }
+            }
+        }
+        st = nx;
+    }
+    // a run's RPT rows all in the tile (every thread but the tile's first and
+    // last): the epilogue's vector form; else row by row
+    double red = 0.0;
+#pragma unroll
+    for (int u = 0; u < R; u++) {
+        const int64_t a = a0 + u * kSub;
+        if (a >= w.row_begin && a + RPT <= w.row_end) {
+            red += epi.template rows<RPT>(a, acc[u]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < RPT; i++)
+                if (a + i >= w.row_begin && a + i < w.row_end) red += epi.row(a + i, acc[u][i]);
+        }
+    }
+    return red;
+}
+
+// (a tile with fewer runs of rows than R -- a batch's small systems, the last
+// tile of a system -- runs the body for those)
+template <class VT, int RPT, class IdxT, class Epi, int R, int kWide>
+__global__ __launch_bounds__(kTileBlock) void k_gather_long(SlotMajor<IdxT> m, const RowWork* __restrict__ work,
+                                                            const uint32_t* __restrict__ sys_col,
+                                                            const GatherStep* __restrict__ steps, int nsteps,
+                                                            const PhaseSeg* __restrict__ phases, uint32_t wmax,
+                                                            const VT* __restrict__ x, Epi epi, GridSys g)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    VT* xs = reinterpret_cast<VT*>(smem_raw);
+    const RowWork w = work[blockIdx.x];
+    if (!epi.begin(w.sys)) return;
+    const VT* __restrict__ xb = x + sys_col[w.sys];
+    const int64_t rows = w.row_end - (w.row_begin & ~int64_t(RPT - 1));
+    double red;
+    if (R > 1 && rows <= RPT * kTileBlock)
+        red = gather_long<VT, RPT, IdxT, Epi, 1, kWide>(m, w, steps, nsteps, phases, wmax, xb, xs, epi);
+    else if (R > 2 && rows <= 2 * RPT * kTileBlock)
+        red = gather_long<VT, RPT, IdxT, Epi, R < 2 ? R : 2, kWide>(m, w, steps, nsteps, phases, wmax, xb, xs, epi);
+    else
+        red = gather_long<VT, RPT, IdxT, Epi, R, kWide>(m, w, steps, nsteps, phases, wmax, xb, xs, epi);
+    reduce_tail<kTileBlock>(epi, red, w.sys, g);
+}
+
 template <class VT, int RPT, class IdxT, class Epi, int BS, int S>
 __global__ __launch_bounds__(BS) void k_gather_tile(SlotMajor<IdxT> m, const RowWork* __restrict__ work,
                                                     const uint32_t* __restrict__ sys_col,

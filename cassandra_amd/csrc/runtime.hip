@@ -589,6 +589,56 @@ GridSys ScatterLists::reduce_sys() const
                    d_red_partials.as<double>()};
 }
 
+// Row tiles: a thread owns trpt consecutive rows counted from the tile's first
+// row rounded down to trpt, so a tile spans at most its runs (or sub-tiles) of
+// bs * trpt rows from there; tiles of a system are a multiple of trpt rows long
+// (their misalignment is the system's).  A single system is cut into a
+// multiple of the CU count so that every CU gets the same number of tiles; the
+// systems of a batch into tiles of one length for all, the shortest (of at
+// least kSmallTileRows rows: a tile costs its staging whatever its rows) that
+// makes no more tiles than a multiple of the CU count.
+void cut_tiles(const cad_matrix* m, const GatherPlan& gp, const std::vector<int>* on, std::vector<RowWork>& tiles,
+               std::vector<int32_t>& first, std::vector<int32_t>& count)
+{
+    constexpr int64_t kSmallTileRows = 2048;
+    const int64_t slots = int64_t(std::max(1, m->ctx->cus)) * (kTileBlock / gp.bs);  // blocks resident at once
+    const int64_t t = gp.trpt;
+    const int64_t cap = (int64_t(gp.runs > 0 ? gp.runs : gp.sub) * gp.bs * t - (t - 1)) / t * t;
+    auto rows_of = [&](int s) {
+        return on && !(*on)[size_t(s)] ? int64_t(0) : m->sys_row_begin[s + 1] - m->sys_row_begin[s];
+    };
+    auto tiles_of = [&](int64_t per) {
+        int64_t n = 0;
+        for (int s = 0; s < m->nsys; s++) n += (rows_of(s) + per - 1) / per;
+        return n;
+    };
+    int64_t total = 0;
+    for (int s = 0; s < m->nsys; s++) total += rows_of(s);
+    // rows a tile: the shortest whose tiles fit `waves` per resident block
+    int64_t per = cap;
+    const int64_t least = std::min(cap, m->nsys > 1 ? (kSmallTileRows + t - 1) / t * t : t);
+    for (int64_t waves = std::max<int64_t>(1, (total + slots * cap - 1) / (slots * cap));; waves++) {
+        if (tiles_of(cap) > slots * waves) continue;
+        int64_t lo = least / t, hi = cap / t;  // in units of t rows
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) / 2;
+            if (tiles_of(mid * t) <= slots * waves) hi = mid;
+            else lo = mid + 1;
+        }
+        per = hi * t;
+        break;
+    }
+    tiles.clear();
+    first.assign(size_t(m->nsys), 0);
+    count.assign(size_t(m->nsys), 0);
+    for (int s = 0; s < m->nsys; s++) {
+        const int64_t r0 = m->sys_row_begin[s], R = rows_of(s);
+        first[size_t(s)] = int32_t(tiles.size());
+        for (int64_t a = 0; a < R; a += per) tiles.push_back(RowWork{r0 + a, r0 + std::min(R, a + per), s, 0});
+        count[size_t(s)] = int32_t(tiles.size()) - first[size_t(s)];
+    }
+}
+
 // Segments of the tiled gather: the slot groups must be runs of consecutive
 // slots that follow each other in slot order (true for pattern matrices, whose
 // groups are the patterns); groups wider than the LDS may hold at most
@@ -605,6 +655,22 @@ void build_gather_plan(cad_matrix* m, GatherPlan& gp, int vbytes, int rpt, int b
     if (bs != kTileBlock && (bs != kTileBlock / 2 || m->mf)) return;
     if (sub < 1 || sub > 3 || (sub > 1 && (bs != kTileBlock || m->mf))) return;
     const int per_cu = kTileBlock / bs;  // blocks resident per CU
+    // Long tiles for the full-block kernels over u16 entries with the most rows
+    // a thread that they have, where a CU has more rows than one of their
+    // tiles: as many runs as its rows need, in as few tiles as the registers
+    // allow.
+    gp.runs = 0;
+    gp.trpt = rpt;
+    if (!m->mf && m->ibytes == 2 && bs == kTileBlock && sub == 1 && rpt == (vbytes == 8 ? 2 : 8)) {
+        const int64_t per = (m->rows + ctx.cus - 1) / std::max(1, ctx.cus);
+        if (per > int64_t(rpt) * kTileBlock) {
+            const int64_t run = int64_t(long_rpt(vbytes)) * kTileBlock, most = long_max_runs(vbytes) * run;
+            const int64_t n = (per + most - 1) / most;
+            gp.trpt = long_rpt(vbytes);
+            gp.runs = int(((per + n - 1) / n + gp.trpt + run - 1) / run);
+            gp.runs = std::min(gp.runs, long_max_runs(vbytes));
+        }
+    }
     // A staged run of columns starts at its element offset inside a 16-byte
     // line (up to Q - 1 elements) so that whole lines map to whole LDS lines:
     // windows leave that room, and phase segments start on line boundaries.
@@ -650,7 +716,10 @@ void build_gather_plan(cad_matrix* m, GatherPlan& gp, int vbytes, int rpt, int b
             phase_w = 0;
         }
         // (a wide step of a matrix-free matrix is one index tile)
-        const int per_step = !wide ? kMaxSegSlots : m->mf ? 4 : wide_step_slots(rpt * m->ibytes);
+        const int per_step = gp.runs > 0 ? (wide ? long_wide_slots(vbytes, gp.runs) : kLongStep)
+                             : !wide     ? kMaxSegSlots
+                             : m->mf     ? 4
+                                         : wide_step_slots(rpt * m->ibytes);
         for (int j0 = 0; j0 < sg.nslots; j0 += per_step) {
             GatherStep st{};
             st.slot_first = uint16_t(sg.slot_first + j0);
@@ -690,31 +759,7 @@ void build_gather_plan(cad_matrix* m, GatherPlan& gp, int vbytes, int rpt, int b
             phase_w = (phase_w + sg.width + Q - 1 + Q - 1) / Q * Q;
         }
     }
-    // Row tiles: a thread owns rpt consecutive rows counted from the tile's
-    // first row rounded down to rpt, so a tile spans at most sub * bs * rpt
-    // rows from there; tiles of a system are a multiple of rpt rows long (their
-    // misalignment is the system's).  A single system is cut into a multiple of
-    // the CU count so that every CU gets the same number of tiles.  In a batch,
-    // a small system is cut into tiles of about kSmallTileRows rows (up to
-    // kSmallTiles of them): once the large systems have converged, its
-    // iterations run alone, and full tiles would leave all but a few CUs idle.
-    constexpr int64_t kSmallTileRows = 2048, kSmallTiles = 32;
-    const int64_t cap = int64_t(sub) * bs * rpt - (rpt - 1);
-    gp.tiles.clear();
-    gp.first.assign(m->nsys, 0);
-    gp.count.assign(m->nsys, 0);
-    for (int s = 0; s < m->nsys; s++) {
-        const int64_t r0 = m->sys_row_begin[s], R = m->sys_row_begin[s + 1] - r0;
-        gp.first[s] = int32_t(gp.tiles.size());
-        int64_t n = (R + cap - 1) / cap;
-        if (m->nsys == 1 && n > 0) n = (n + ctx.cus * per_cu - 1) / (ctx.cus * per_cu) * (ctx.cus * per_cu);
-        if (m->nsys > 1) n = std::max(n, std::min((R + kSmallTileRows - 1) / kSmallTileRows, kSmallTiles));
-        int64_t per = n > 0 ? (R + n - 1) / n : 0;
-        per = std::min(cap / rpt * rpt, (per + rpt - 1) / rpt * rpt);
-        for (int64_t t = 0; per > 0 && t * per < R; t++)
-            gp.tiles.push_back(RowWork{r0 + t * per, r0 + std::min(R, (t + 1) * per), s, 0});
-        gp.count[s] = int32_t(gp.tiles.size()) - gp.first[s];
-    }
+    cut_tiles(m, gp, nullptr, gp.tiles, gp.first, gp.count);
     gp.d_segs = to_device(gp.segs, ctx.stream);
     gp.d_steps = to_device(gp.steps, ctx.stream);
     gp.d_phases = to_device(gp.phases, ctx.stream);

@@ -115,6 +115,8 @@ struct GatherPlan {
     int rpt = 0;      // rows per thread
     int bs = 1024;    // threads per block (1024, or 512: two blocks and half the LDS each per CU)
     int sub = 1;      // sub-tiles of bs * rpt rows that share each staging
+    int runs = 0;     // > 0: long tiles of this many runs of kTileBlock * trpt rows (k_gather_long)
+    int trpt = 0;     // consecutive rows a thread takes together
     uint32_t wmax = 0;
     uint32_t lds_elems = 0;
     std::vector<GatherSeg> segs;     // matrix-free kernel: one staging per segment
@@ -273,6 +275,10 @@ struct cad_matrix {
 namespace cad {
 void build_plans(cad_matrix* m);
 void build_gather_plan(cad_matrix* m, GatherPlan& gp, int vbytes, int rpt, int bs, int sub);
+// The row tiles of a gather plan for the systems in `on` (null: all): each
+// system's range of them in first / count.
+void cut_tiles(const cad_matrix* m, const GatherPlan& gp, const std::vector<int>* on, std::vector<RowWork>& tiles,
+               std::vector<int32_t>& first, std::vector<int32_t>& count);
 void build_scatter_plan(ScatterPlan& sp, const std::vector<uint32_t>& lo, const std::vector<uint32_t>& hi,
                         const std::vector<int64_t>& sys_rows, const std::vector<uint32_t>& sys_col,
                         int64_t cols_per_sys, int ibytes, const Context& ctx, const TuneParams& tune);

@@ -279,6 +279,24 @@ constexpr bool sub_tiles_ok(int rpt)
     return rpt * int(sizeof(VT)) == 8 && rpt * int(sizeof(IdxT)) <= 4;
 }
 
+// The stored-index tile kernel of a plan: over long tiles, or by its shape; f
+// receives the kernel and its threads per block.
+template <class VT, int RPT, class IdxT, class Epi, class F>
+void with_stored_tile(const GatherPlan& gp, F&& f)
+{
+    if constexpr (std::is_same_v<IdxT, uint16_t> && RPT == (sizeof(VT) == 8 ? 2 : 8)) {
+        constexpr int B = sizeof(VT), L = long_rpt(B);
+        if (gp.runs == 1) return f(k_gather_long<VT, L, IdxT, Epi, 1, long_wide_slots(B, 1)>, kTileBlock);
+        if (gp.runs == 2) return f(k_gather_long<VT, L, IdxT, Epi, 2, long_wide_slots(B, 2)>, kTileBlock);
+        if constexpr (long_max_runs(B) > 2)
+            if (gp.runs == 3) return f(k_gather_long<VT, L, IdxT, Epi, 3, long_wide_slots(B, 3)>, kTileBlock);
+    }
+    with_tile_shape<sub_tiles_ok<VT, IdxT>(RPT)>(gp.bs, gp.sub, [&](auto bc, auto sc) {
+        constexpr int BS = decltype(bc)::value;
+        f(k_gather_tile<VT, RPT, IdxT, Epi, BS, decltype(sc)::value>, BS);
+    });
+}
+
 // The row blocks a gather launches: the tile plan's or the grid plan's (all
 // systems), or those of an ActiveLists built for this value size.
 struct RowList {
@@ -295,7 +313,7 @@ RowList row_list(cad_matrix* m, const ActiveLists* al)
         const GridSys base = gp.ok && !al->row_kernel ? gp.sys() : m->grid.row_sys();
         return RowList{al->tiles.as<RowWork>(), al->ntiles,
                        GridSys{al->tfirst.as<int32_t>(), al->tcount.as<int32_t>(), base.counters,
-                               al->row_kernel ? al->gpart.as<double>() : base.partials}};
+                               al->gpart.as<double>()}};
     }
     if (gp.ok) return RowList{gp.d_tiles.as<RowWork>(), int(gp.tiles.size()), gp.sys()};
     return RowList{m->grid.d_rows.as<RowWork>(), int(m->grid.rows.size()), m->grid.row_sys()};
@@ -327,11 +345,9 @@ void gather(cad_matrix* m, const VT* x, Epi epi, hipStream_t s, const ActiveList
                                        m->d_sys_col.as<uint32_t>(), gp.d_steps.as<GatherStep>(),
                                        int(gp.steps.size()), gp.d_phases.as<PhaseSeg>(), gp.wmax, x, epi, rl.sys);
                 } else {
-                    with_tile_shape<sub_tiles_ok<VT, IdxT>(RPT)>(gp.bs, gp.sub, [&](auto bc, auto sc) {
-                        constexpr int BS = decltype(bc)::value;
-                        auto kern = k_gather_tile<VT, RPT, IdxT, Epi, BS, decltype(sc)::value>;
+                    with_stored_tile<VT, RPT, IdxT, Epi>(gp, [&](auto kern, int bs) {
                         allow_lds(kern, lds);
-                        hipLaunchKernelGGL(kern, dim3(unsigned(rl.n)), dim3(BS), lds, s, view, rl.p,
+                        hipLaunchKernelGGL(kern, dim3(unsigned(rl.n)), dim3(unsigned(bs)), lds, s, view, rl.p,
                                            m->d_sys_col.as<uint32_t>(), gp.d_steps.as<GatherStep>(),
                                            int(gp.steps.size()), gp.d_phases.as<PhaseSeg>(), gp.wmax, x, epi,
                                            rl.sys);
@@ -585,9 +601,11 @@ static void build_active(cad_matrix* m, ActiveLists& al, const std::vector<int>&
                     fine.push_back(RowWork{r, std::min(m->sys_row_begin[i + 1], r + int64_t(kRowBlock)), i, 0});
             fine_count[i] = int32_t(fine.size()) - fine_first[i];
         }
-    const std::vector<RowWork>& tiles = al.row_kernel ? fine : gp.tiles;
-    const std::vector<int32_t>& tf = al.row_kernel ? fine_first : gp.first;
-    const std::vector<int32_t>& tc = al.row_kernel ? fine_count : gp.count;
+    // the staged kernel's tiles, cut anew for the running systems
+    if (!al.row_kernel) cut_tiles(m, gp, &on, fine, fine_first, fine_count);
+    const std::vector<RowWork>& tiles = fine;
+    const std::vector<int32_t>& tf = fine_first;
+    const std::vector<int32_t>& tc = fine_count;
     std::vector<RowWork> t;
     std::vector<int32_t> t_first(n, 0), t_count(n, 0);
     std::vector<ColWork> cw;
@@ -614,7 +632,7 @@ static void build_active(cad_matrix* m, ActiveLists& al, const std::vector<int>&
     al.nreduce = int(sub.reduce.size());
     al.ncols = int(cw.size());
     al.tiles = to_device(t, s);
-    if (al.row_kernel) al.gpart = DBuf(2 * sizeof(double) * std::max<size_t>(1, t.size()));
+    al.gpart = DBuf(2 * sizeof(double) * std::max<size_t>(1, t.size()));
     al.tfirst = to_device(t_first, s);
     al.tcount = to_device(t_count, s);
     al.scatter = to_device(sub.work, s);
@@ -664,10 +682,8 @@ static void prepare_gather(cad_matrix* m)
             if constexpr (std::is_void_v<IdxT>)
                 allow_lds(k_gather_tile_mf<VT, RPT, Epi>, size_t(gp.lds_elems) * sizeof(VT));
             else
-                with_tile_shape<sub_tiles_ok<VT, IdxT>(RPT)>(gp.bs, gp.sub, [&](auto bc, auto sc) {
-                    allow_lds(k_gather_tile<VT, RPT, IdxT, Epi, decltype(bc)::value, decltype(sc)::value>,
-                              size_t(gp.lds_elems) * sizeof(VT));
-                });
+                with_stored_tile<VT, RPT, IdxT, Epi>(
+                    gp, [&](auto kern, int) { allow_lds(kern, size_t(gp.lds_elems) * sizeof(VT)); });
         });
     });
 }
