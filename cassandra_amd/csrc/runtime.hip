@@ -31,17 +31,23 @@ DBuf::DBuf(size_t n) : bytes(n)
     }
 }
 
+DBuf::DBuf(std::shared_ptr<DBuf> whole, size_t at, size_t n)
+    : p(static_cast<uint8_t*>(whole->p) + at), bytes(n), part(std::move(whole))
+{
+}
+
 DBuf::~DBuf()
 {
-    if (p) (void)hipFree(p);
+    if (p && !part) (void)hipFree(p);
 }
 
 DBuf& DBuf::operator=(DBuf&& o) noexcept
 {
     if (this != &o) {
-        if (p) (void)hipFree(p);
+        if (p && !part) (void)hipFree(p);
         p = o.p;
         bytes = o.bytes;
+        part = std::move(o.part);
         o.p = nullptr;
         o.bytes = 0;
     }
@@ -52,6 +58,37 @@ void DBuf::upload(const void* h, size_t n, hipStream_t s)
 {
     CAD_HIP(hipMemcpyAsync(p, h, n, hipMemcpyHostToDevice, s));
     CAD_HIP(hipStreamSynchronize(s));
+}
+
+namespace {
+constexpr size_t kPieceAlign = 256;
+size_t piece(size_t n) { return (n + kPieceAlign - 1) / kPieceAlign * kPieceAlign; }
+}  // namespace
+
+void Uploads::put_bytes(DBuf& dst, const void* src, size_t bytes, size_t least)
+{
+    const size_t at = piece(host.size());
+    host.resize(at + std::max(bytes, least), 0);
+    if (bytes) std::memcpy(host.data() + at, src, bytes);
+    items.push_back(Item{&dst, at, std::max(bytes, least), true});
+}
+
+void Uploads::reserve(DBuf& dst, size_t bytes)
+{
+    items.push_back(Item{&dst, reserved, bytes, false});
+    reserved += piece(bytes);
+}
+
+void Uploads::flush(hipStream_t s)
+{
+    if (items.empty()) return;
+    const size_t copied = piece(host.size());
+    auto whole = std::make_shared<DBuf>(std::max<size_t>(1, copied + reserved));
+    if (!host.empty()) whole->upload(host.data(), host.size(), s);
+    for (const Item& i : items) *i.dst = DBuf(whole, i.copied ? i.at : copied + i.at, i.bytes);
+    items.clear();
+    host.clear();
+    reserved = 0;
 }
 
 Context::~Context()
@@ -299,13 +336,19 @@ void make_scatter_lists_xcd(const ScatterPlan& sp, const std::vector<int64_t>& s
     L.part_elems = off;
 }
 
-// Scatter tiles of (system rows) x (group window).  The number of row chunks
-// of a window is set by its share of the work (about two tiles per CU in
-// total), capped so that the partial slices (written and read once) stay near
-// 10% of the window's index traffic.
+// Scatter tiles of (system rows) x (group window): every window of a system
+// gets row chunks by its time (win_cost), so that the tiles -- about target of
+// them -- take equally long; a window's chunks are limited by its partial
+// slices (written and read once): partial_cap of its index traffic, or the
+// floor bytes a window where that leaves CUs idle -- small_floor (8 MB by
+// default) for a small system (at most kRowKernelRows rows, whose tiles are
+// latency-bound: a 100k-row PCG iteration 47 -> 42 µs), 2 MB for a large one --
+// and to kScatterBlock rows.  Rounding each window's share by itself, and the
+// floor, made 263 tiles for 256 CUs at 5M rows of FIT8: seven in a second wave,
+// 197 µs where 256 take 127.
 void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_rows,
                         const std::vector<uint32_t>& sys_col, int64_t cols_per_sys, uint32_t wmax, int vbytes,
-                        int ibytes, int cus, const TuneParams& tune, ScatterLists& L,
+                        int ibytes, int cus, const TuneParams& tune, bool fp32, ScatterLists& L,
                         const std::vector<uint8_t>* on = nullptr)
 {
     L.work.clear();
@@ -314,12 +357,15 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
     pack_groups(sp, wmax, tune.pack_slots, L);
     const int nsys = int(sys_col.size());
     auto in = [&](int s) { return !on || (*on)[size_t(s)] != 0; };
-    // Work of a window per row: its slot loads, and its atomics -- the share
-    // of the group's entries that fall into the window, taken as its share of
-    // the group's columns.  scatter_balance weighs the two (1: loads only).
+    // Time of a window per row, in units of one slot's loads.  Measured (cycles
+    // a tile per 64 rows): FP32 windows take 32 for the row and 7.8 + 2 f a
+    // slot, f the window's share of the group's columns (66 to 111 for 4 to 8
+    // slots), FP64 ones 18 and 6 + 17.5 f (62 to 206: their adds are slower).
+    // Other values of scatter_balance weigh the slot loads (1: loads only)
+    // against the entries that fall into the window.  Matrix-free: a slot's
+    // columns are computed whether or not they fall into the window
+    // (ScatterPlan::slot_cost), after the row's digits (row_cost).
     const double lam = std::min(1.0, std::max(0.0, tune.scatter_balance));
-    // (Matrix-free: a slot's columns are computed whether or not they fall into
-    // the window, ScatterPlan::slot_cost, after the row's digits, row_cost.)
     auto win_cost = [&](const SlotGroup& g, uint32_t W) {
         if (!sp.slot_cost.empty() && vbytes == 8) {
             double c = sp.row_cost;
@@ -327,92 +373,107 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
             return c;
         }
         const double frac = double(W) / double(std::max<uint32_t>(1, g.col_hi - g.col_lo));
+        if (lam == 1.0 && vbytes == 8) return fp32 ? 4.1 + g.nslots * (1.0 + 0.26 * frac) : 3.0 + g.nslots * (1.0 + 2.9 * frac);
         return g.nslots * (lam + (1.0 - lam) * frac);
     };
-    double total = 0;
     int nrun = 0;  // systems planned here that have rows: their windows run side by side
-    for (int s = 0; s < nsys; s++) {
-        if (!in(s)) continue;
-        const int64_t R = sys_rows[s + 1] - sys_rows[s];
-        nrun += R > 0;
-        for (auto& g : L.groups)
-            for (uint32_t wl = g.col_lo; wl < g.col_hi; wl += wmax)
-                total += double(R) * win_cost(g, std::min(g.col_hi, wl + wmax) - wl);
-    }
-    // several systems side by side have tiles of very different sizes (their
-    // row counts differ): more tiles a CU let the launch balance them
-    const double target = tune.blocks_per_cu * std::max(cus, 1) * (nrun > 1 ? kMultiSystemTiles : 1.0);
+    for (int s = 0; s < nsys; s++) nrun += in(s) && sys_rows[s + 1] > sys_rows[s];
     int windows = 0;
     for (auto& g : L.groups) windows += int((g.col_hi - g.col_lo + wmax - 1) / wmax);
+    // several systems whose windows outnumber the CUs have tiles of very
+    // different sizes (their row counts differ): more tiles a CU let the launch
+    // balance them
+    const double share = tune.blocks_per_cu * std::max(cus, 1);
+    const double target = share * (nrun > 1 && double(windows) * nrun > 0.75 * share ? kMultiSystemTiles : 1.0);
     int64_t off = 0;
     if (tune.scatter_order == 1) {
         make_scatter_lists_xcd(sp, sys_rows, sys_col, cols_per_sys, wmax, vbytes, ibytes, target, cus, tune, L, on);
         return;
     }
+    // the windows of every system, and their chunks
+    struct Win {
+        uint32_t lo, hi;
+        int s, group;
+        int64_t rows, chunks, most;
+        double time;
+    };
+    std::vector<Win> wins;
+    double total = 0;
     for (int s = 0; s < nsys; s++) {
         if (!in(s)) continue;
         const int64_t R = sys_rows[s + 1] - sys_rows[s];
-        std::vector<std::pair<uint32_t, uint32_t>> covered;
         for (size_t gi = 0; gi < L.groups.size(); gi++) {
             const SlotGroup& g = L.groups[gi];
             for (uint32_t wl = g.col_lo; wl < g.col_hi; wl += wmax) {
-                const uint32_t wh = std::min(g.col_hi, wl + wmax);
-                const uint32_t W = wh - wl;
-                covered.push_back({wl, wh});
-                L.widest = std::max(L.widest, W);
-                int64_t C = 0;
-                if (R > 0) {
-                    const double share = total > 0 ? double(R) * win_cost(g, W) / total : 1.0;
-                    const double cap = tune.partial_cap * double(R) * g.nslots * ibytes / (2.0 * W * vbytes);
-                    C = window_chunks(R, target * share, cap, cus, windows * std::max(1, nrun), W, vbytes,
-                                      tune.small_floor_bytes);
-                    const int64_t chunk = (R + C - 1) / C;
-                    C = (R + chunk - 1) / chunk;
-                    for (int64_t c = 0; c < C; c++) {
-                        ScatterWork w;
-                        w.row_begin = sys_rows[s] + c * chunk;
-                        w.row_end = sys_rows[s] + std::min(R, (c + 1) * chunk);
-                        w.part_off = off + c * int64_t(W);
-                        w.win_lo = sys_col[s] + wl;
-                        w.win_hi = sys_col[s] + wh;
-                        w.group = int32_t(gi);
-                        w.sys = s;
-                        L.work.push_back(w);
-                    }
-                }
-                // one column per thread of a reduce block (kReduceCols), so the
-                // reduce launches enough blocks to cover the CUs
-                for (uint32_t c0 = wl; c0 < wh; c0 += kReduceCols) {
-                    ReduceWork r;
-                    r.col_begin = int64_t(sys_col[s]) + c0;
-                    r.col_end = int64_t(sys_col[s]) + std::min(wh, c0 + kReduceCols);
-                    r.part_off = off + (c0 - wl);
-                    r.nchunk = int32_t(C);
-                    r.stride = W;
-                    r.sys = s;
-                    r.pad = 0;
-                    L.reduce.push_back(r);
-                }
-                off += C * int64_t(W);
+                const uint32_t wh = std::min(g.col_hi, wl + wmax), W = wh - wl;
+                const double slice = 2.0 * double(W) * vbytes;
+                const double cap = tune.partial_cap * double(R) * g.nslots * ibytes / slice;
+                const double floor_c = (R <= kRowKernelRows ? tune.small_floor_bytes : kPartialFloorBytes) / slice;
+                Win w{wl, wh, s, int(gi), R, 0, 0, double(R) * win_cost(g, W)};
+                w.most = std::max<int64_t>(1, std::min<int64_t>(int64_t(std::max(cap, floor_c)),
+                                                                (R + kScatterBlock - 1) / kScatterBlock));
+                total += w.time;
+                wins.push_back(w);
             }
+        }
+    }
+    // whole shares, then one chunk more wherever the tiles are longest
+    int64_t tiles = 0;
+    std::vector<std::pair<double, size_t>> longest;  // a heap by tile time
+    for (size_t i = 0; i < wins.size(); i++) {
+        Win& w = wins[i];
+        if (w.rows <= 0) continue;
+        w.chunks = std::max<int64_t>(1, std::min<int64_t>(w.most, int64_t(target * w.time / total)));
+        tiles += w.chunks;
+        if (w.chunks < w.most) longest.push_back({w.time / double(w.chunks), i});
+    }
+    std::make_heap(longest.begin(), longest.end());
+    while (tiles < int64_t(target) && !longest.empty()) {
+        std::pop_heap(longest.begin(), longest.end());
+        Win& w = wins[longest.back().second];
+        longest.pop_back();
+        w.chunks++;
+        tiles++;
+        if (w.chunks < w.most) {
+            longest.push_back({w.time / double(w.chunks), size_t(&w - wins.data())});
+            std::push_heap(longest.begin(), longest.end());
+        }
+    }
+    size_t at = 0;
+    for (int s = 0; s < nsys; s++) {
+        if (!in(s)) continue;
+        std::vector<std::pair<uint32_t, uint32_t>> covered;
+        for (; at < wins.size() && wins[at].s == s; at++) {
+            const Win& wn = wins[at];
+            const uint32_t W = wn.hi - wn.lo;
+            covered.push_back({wn.lo, wn.hi});
+            L.widest = std::max(L.widest, W);
+            int64_t C = 0;
+            if (wn.rows > 0) {
+                const int64_t chunk = (wn.rows + wn.chunks - 1) / wn.chunks;
+                C = (wn.rows + chunk - 1) / chunk;
+                for (int64_t c = 0; c < C; c++) {
+                    ScatterWork w;
+                    w.row_begin = sys_rows[s] + c * chunk;
+                    w.row_end = sys_rows[s] + std::min(wn.rows, (c + 1) * chunk);
+                    w.part_off = off + c * int64_t(W);
+                    w.win_lo = sys_col[s] + wn.lo;
+                    w.win_hi = sys_col[s] + wn.hi;
+                    w.group = int32_t(wn.group);
+                    w.sys = s;
+                    L.work.push_back(w);
+                }
+            }
+            push_reduce(L, s, sys_col[s], wn.lo, wn.hi, off, C);
+            off += C * int64_t(W);
         }
         // columns outside every window are written as zeros
         std::sort(covered.begin(), covered.end());
         covered.push_back({uint32_t(cols_per_sys), uint32_t(cols_per_sys)});
-        uint32_t at = 0;
+        uint32_t next = 0;
         for (auto& iv : covered) {
-            for (uint32_t c0 = at; c0 < iv.first; c0 += kReduceCols) {
-                ReduceWork r;
-                r.col_begin = int64_t(sys_col[s]) + c0;
-                r.col_end = int64_t(sys_col[s]) + std::min(iv.first, c0 + kReduceCols);
-                r.part_off = 0;
-                r.nchunk = 0;
-                r.stride = 0;
-                r.sys = s;
-                r.pad = 0;
-                L.reduce.push_back(r);
-            }
-            at = std::max(at, iv.second);
+            if (next < iv.first) push_reduce(L, s, sys_col[s], next, iv.first, 0, 0);
+            next = std::max(next, iv.second);
         }
     }
     L.part_elems = off;
@@ -537,7 +598,8 @@ GridSys GatherPlan::sys() const
 
 void build_scatter_plan(ScatterPlan& sp, const std::vector<uint32_t>& lo, const std::vector<uint32_t>& hi,
                         const std::vector<int64_t>& sys_rows, const std::vector<uint32_t>& sys_col,
-                        int64_t cols_per_sys, int ibytes, const Context& ctx, const TuneParams& tune)
+                        int64_t cols_per_sys, int ibytes, const Context& ctx, const TuneParams& tune, bool fp32,
+                        Uploads& up)
 {
     make_groups(lo, hi, sp);
     const size_t lds = lds_budget(ctx);
@@ -549,37 +611,35 @@ void build_scatter_plan(ScatterPlan& sp, const std::vector<uint32_t>& lo, const 
     t4.partial_cap = 1.0;
     t4.scatter_balance = 1.0;
     t4.pack_slots = kMaxSegSlots;  // (the count kernel holds a group's slots in registers)
-    make_scatter_lists(sp, sys_rows, sys_col, cols_per_sys, uint32_t(lds / 4), 4, ibytes, ctx.cus, t4, sp.f4);
-    make_scatter_lists(sp, sys_rows, sys_col, cols_per_sys, uint32_t(lds / 8), 8, ibytes, ctx.cus, tune, sp.f8);
     const int nsys = int(sys_rows.size()) - 1;
-    finish_lists(sp.f4, nsys);
-    finish_lists(sp.f8, nsys);
-    sp.d_groups = to_device(sp.groups, ctx.stream);
-    // slot lists padded to whole 32-bit words (the kernels read them as words)
-    auto padded = [](std::vector<uint16_t> v) {
-        if (v.size() % 2) v.push_back(0);
-        return v;
+    auto build = [&](ScatterLists& L, int wbytes, const TuneParams& t, bool f32) {
+        make_scatter_lists(sp, sys_rows, sys_col, cols_per_sys, uint32_t(lds / wbytes), wbytes, ibytes, ctx.cus, t,
+                           f32, L);
+        finish_lists(L, nsys);
+        // slot lists padded to whole 32-bit words (the kernels read them as words)
+        std::vector<uint16_t> padded = L.slot_list;
+        if (padded.size() % 2) padded.push_back(0);
+        up.put(L.d_groups, L.groups);
+        up.put(L.d_slot_list, padded);
+        up.put(L.d_work, L.work);
+        up.put(L.d_reduce, L.reduce);
+        up.put(L.d_red_first, L.red_first);
+        up.put(L.d_red_count, L.red_count);
+        up.put(L.d_red_counters, std::vector<unsigned>(size_t(std::max(1, nsys)), 0u));
+        up.reserve(L.d_red_partials, 2 * sizeof(double) * std::max<size_t>(1, L.reduce.size()));
+        L.part = DBuf();
     };
-    sp.d_slot_list = to_device(padded(sp.slot_list), ctx.stream);
-    for (ScatterLists* L : {&sp.f4, &sp.f8}) {
-        L->d_groups = to_device(L->groups, ctx.stream);
-        L->d_slot_list = to_device(padded(L->slot_list), ctx.stream);
-        L->d_work = to_device(L->work, ctx.stream);
-        L->d_reduce = to_device(L->reduce, ctx.stream);
-        L->d_red_first = to_device(L->red_first, ctx.stream);
-        L->d_red_count = to_device(L->red_count, ctx.stream);
-        L->d_red_counters = to_device(std::vector<unsigned>(size_t(std::max(1, nsys)), 0u), ctx.stream);
-        L->d_red_partials = DBuf(2 * sizeof(double) * std::max<size_t>(1, L->reduce.size()));
-        L->part = DBuf();
-    }
+    build(sp.f4, 4, t4, false);
+    build(sp.f8, 8, tune, false);
+    if (fp32) build(sp.f8s, 8, tune, true);
 }
 
 void plan_scatter_subset(const ScatterPlan& sp, const std::vector<int64_t>& sys_rows,
                          const std::vector<uint32_t>& sys_col, int64_t cols_per_sys, int ibytes, const Context& ctx,
-                         const TuneParams& tune, const std::vector<uint8_t>& on, ScatterLists& L)
+                         const TuneParams& tune, const std::vector<uint8_t>& on, bool fp32, ScatterLists& L)
 {
-    make_scatter_lists(sp, sys_rows, sys_col, cols_per_sys, uint32_t(lds_budget(ctx) / 8), 8, ibytes, ctx.cus, tune, L,
-                       &on);
+    make_scatter_lists(sp, sys_rows, sys_col, cols_per_sys, uint32_t(lds_budget(ctx) / 8), 8, ibytes, ctx.cus, tune,
+                       fp32, L, &on);
     finish_lists(L, int(sys_rows.size()) - 1);
 }
 
@@ -643,7 +703,7 @@ void cut_tiles(const cad_matrix* m, const GatherPlan& gp, const std::vector<int>
 // slots that follow each other in slot order (true for pattern matrices, whose
 // groups are the patterns); groups wider than the LDS may hold at most
 // kMaxSegSlots slots.
-void build_gather_plan(cad_matrix* m, GatherPlan& gp, int vbytes, int rpt, int bs, int sub)
+void build_gather_plan(cad_matrix* m, GatherPlan& gp, int vbytes, int rpt, int bs, int sub, Uploads& up)
 {
     const Context& ctx = *m->ctx;
     const ScatterPlan& sp = m->splan;
@@ -760,14 +820,13 @@ void build_gather_plan(cad_matrix* m, GatherPlan& gp, int vbytes, int rpt, int b
         }
     }
     cut_tiles(m, gp, nullptr, gp.tiles, gp.first, gp.count);
-    gp.d_segs = to_device(gp.segs, ctx.stream);
-    gp.d_steps = to_device(gp.steps, ctx.stream);
-    gp.d_phases = to_device(gp.phases, ctx.stream);
-    gp.d_tiles = to_device(gp.tiles, ctx.stream);
-    gp.d_first = to_device(gp.first, ctx.stream);
-    gp.d_count = to_device(gp.count, ctx.stream);
-    gp.d_counters = to_device(std::vector<unsigned>(std::max(1, m->nsys), 0u), ctx.stream);
-    gp.d_partials = DBuf(2 * sizeof(double) * std::max<size_t>(1, gp.tiles.size()));
+    up.put(gp.d_steps, gp.steps);
+    up.put(gp.d_phases, gp.phases);
+    up.put(gp.d_tiles, gp.tiles);
+    up.put(gp.d_first, gp.first);
+    up.put(gp.d_count, gp.count);
+    up.put(gp.d_counters, std::vector<unsigned>(size_t(std::max(1, m->nsys)), 0u));
+    up.reserve(gp.d_partials, 2 * sizeof(double) * std::max<size_t>(1, gp.tiles.size()));
     gp.ok = true;
 }
 
@@ -781,12 +840,13 @@ void build_plans(cad_matrix* m)
         m->sys_col = {0};
         m->cols_per_sys = m->cols;
     }
-    m->d_sys_col = to_device(m->sys_col, ctx.stream);
+    Uploads up;
+    up.put(m->d_sys_col, m->sys_col);
     // (a matrix-free matrix sizes its scatter partials as a u16 matrix would)
     build_scatter_plan(m->splan, m->slot_lo, m->slot_hi, m->sys_row_begin, m->sys_col, m->cols_per_sys,
-                       m->mf ? 2 : m->ibytes, ctx, m->tune);
-    build_gather_plan(m, m->gplan4, 4, m->tune.rpt4, m->tune.bs4, m->tune.sub4);
-    build_gather_plan(m, m->gplan8, 8, m->tune.rpt8, m->tune.bs8, m->tune.sub8);
+                       m->mf ? 2 : m->ibytes, ctx, m->tune, true, up);
+    build_gather_plan(m, m->gplan4, 4, m->tune.rpt4, m->tune.bs4, m->tune.sub4, up);
+    build_gather_plan(m, m->gplan8, 8, m->tune.rpt8, m->tune.bs8, m->tune.sub8, up);
 
     GridPlan& g = m->grid;
     g.rows.clear();
@@ -809,19 +869,20 @@ void build_plans(cad_matrix* m)
         for (int64_t c = c0; c < c1; c += cchunk) g.cols.push_back(ColWork{c, std::min(c1, c + cchunk), s, c == c0});
         g.col_count[s] = int32_t(g.cols.size()) - g.col_first[s];
     }
-    g.d_rows = to_device(g.rows, ctx.stream);
-    g.d_cols = to_device(g.cols, ctx.stream);
-    g.d_row_first = to_device(g.row_first, ctx.stream);
-    g.d_row_count = to_device(g.row_count, ctx.stream);
-    g.d_col_first = to_device(g.col_first, ctx.stream);
-    g.d_col_count = to_device(g.col_count, ctx.stream);
+    up.put(g.d_rows, g.rows);
+    up.put(g.d_cols, g.cols);
+    up.put(g.d_row_first, g.row_first);
+    up.put(g.d_row_count, g.row_count);
+    up.put(g.d_col_first, g.col_first);
+    up.put(g.d_col_count, g.col_count);
     std::vector<unsigned> zeros(std::max(1, m->nsys), 0u);
-    g.d_row_counters = to_device(zeros, ctx.stream);
-    g.d_col_counters = to_device(zeros, ctx.stream);
-    g.d_partials = DBuf(2 * sizeof(double) * std::max<size_t>(1, std::max(g.rows.size(), g.cols.size())));
+    up.put(g.d_row_counters, zeros);
+    up.put(g.d_col_counters, zeros);
+    up.reserve(g.d_partials, 2 * sizeof(double) * std::max<size_t>(1, std::max(g.rows.size(), g.cols.size())));
     // max |y| per row block and per system, for the fixed-point FP32 scatter
-    m->splan.d_ymax_part = DBuf(sizeof(unsigned) * std::max<size_t>(1, g.rows.size()));
-    m->splan.d_ymax = DBuf(sizeof(unsigned) * size_t(std::max(1, m->nsys)));
+    up.reserve(m->splan.d_ymax_part, sizeof(unsigned) * std::max<size_t>(1, g.rows.size()));
+    up.reserve(m->splan.d_ymax, sizeof(unsigned) * size_t(std::max(1, m->nsys)));
+    up.flush(ctx.stream);
 }
 
 }  // namespace cad

@@ -24,16 +24,18 @@ void hip_check(hipError_t e, const char* what);
 
 struct Context;
 
-// Owning device buffer.
+// Owning device buffer, or (part set) a piece of one that all its pieces keep.
 struct DBuf {
     void* p = nullptr;
     size_t bytes = 0;
+    std::shared_ptr<DBuf> part;
     DBuf() = default;
     explicit DBuf(size_t n);
+    DBuf(std::shared_ptr<DBuf> whole, size_t at, size_t n);
     ~DBuf();
     DBuf(const DBuf&) = delete;
     DBuf& operator=(const DBuf&) = delete;
-    DBuf(DBuf&& o) noexcept : p(o.p), bytes(o.bytes) { o.p = nullptr; o.bytes = 0; }
+    DBuf(DBuf&& o) noexcept : p(o.p), bytes(o.bytes), part(std::move(o.part)) { o.p = nullptr; o.bytes = 0; }
     DBuf& operator=(DBuf&& o) noexcept;
     template <class T> T* as() const { return static_cast<T*>(p); }
     void upload(const void* h, size_t n, hipStream_t s);
@@ -46,6 +48,30 @@ DBuf to_device(const std::vector<T>& v, hipStream_t s)
     if (!v.empty()) b.upload(v.data(), v.size() * sizeof(T), s);
     return b;
 }
+
+// The buffers of a plan, in one allocation with one copy: a matrix has about 40
+// of them, and an allocation, a copy and a wait each took 0.7 ms of the 1.4 ms
+// of a fit of 100,000 rows.  The destinations are set by flush.
+struct Uploads {
+    template <class T>
+    void put(DBuf& dst, const std::vector<T>& v)
+    {
+        put_bytes(dst, v.data(), v.size() * sizeof(T), sizeof(T));
+    }
+    void reserve(DBuf& dst, size_t bytes);  // contents undefined
+    void flush(hipStream_t s);              // waits for the copy
+
+private:
+    struct Item {
+        DBuf* dst;
+        size_t at, bytes;
+        bool copied;
+    };
+    void put_bytes(DBuf& dst, const void* src, size_t bytes, size_t least);
+    std::vector<uint8_t> host;
+    std::vector<Item> items;
+    size_t reserved = 0;
+};
 
 // Appends list l of a ternary-word program (DevTern): the squares src[j] of a
 // base-3 number sum_j 3^j (P[src_j] + 2 O[src_j]) as entries {2 (q mod 16),
@@ -99,8 +125,10 @@ struct ScatterLists {
 struct ScatterPlan {
     std::vector<SlotGroup> groups;
     std::vector<uint16_t> slot_list;
-    DBuf d_groups, d_slot_list;
-    ScatterLists f4, f8;  // float and double (and uint32 counts) windows
+    // 4-byte windows (the u32 counts), 8-byte windows of FP64 products and of
+    // FP32 ones in fixed point (the same windows, their row chunks by the time
+    // that either takes); the evaluator's plan has no f8s
+    ScatterLists f4, f8, f8s;
     // a window's time per row, where it is not the number of its slots
     // (matrix-free): of each slot, and of the row itself
     std::vector<double> slot_cost;
@@ -124,7 +152,7 @@ struct GatherPlan {
     std::vector<PhaseSeg> phases;
     std::vector<RowWork> tiles;
     std::vector<int32_t> first, count;
-    DBuf d_segs, d_steps, d_phases, d_tiles, d_first, d_count, d_counters, d_partials;
+    DBuf d_steps, d_phases, d_tiles, d_first, d_count, d_counters, d_partials;
     GridSys sys() const;
 };
 
@@ -274,14 +302,15 @@ struct cad_matrix {
 
 namespace cad {
 void build_plans(cad_matrix* m);
-void build_gather_plan(cad_matrix* m, GatherPlan& gp, int vbytes, int rpt, int bs, int sub);
+void build_gather_plan(cad_matrix* m, GatherPlan& gp, int vbytes, int rpt, int bs, int sub, Uploads& up);
 // The row tiles of a gather plan for the systems in `on` (null: all): each
 // system's range of them in first / count.
 void cut_tiles(const cad_matrix* m, const GatherPlan& gp, const std::vector<int>* on, std::vector<RowWork>& tiles,
                std::vector<int32_t>& first, std::vector<int32_t>& count);
 void build_scatter_plan(ScatterPlan& sp, const std::vector<uint32_t>& lo, const std::vector<uint32_t>& hi,
                         const std::vector<int64_t>& sys_rows, const std::vector<uint32_t>& sys_col,
-                        int64_t cols_per_sys, int ibytes, const Context& ctx, const TuneParams& tune);
+                        int64_t cols_per_sys, int ibytes, const Context& ctx, const TuneParams& tune, bool fp32,
+                        Uploads& up);
 // The 8-byte window lists of the systems in `on` alone (host vectors only:
 // work, reduce items ordered by system with each system's range, part_elems,
 // cbits), their row chunks set for the windows those systems run side by
@@ -289,6 +318,6 @@ void build_scatter_plan(ScatterPlan& sp, const std::vector<uint32_t>& lo, const 
 // groups and slot lists serve the work items.
 void plan_scatter_subset(const ScatterPlan& sp, const std::vector<int64_t>& sys_rows,
                          const std::vector<uint32_t>& sys_col, int64_t cols_per_sys, int ibytes, const Context& ctx,
-                         const TuneParams& tune, const std::vector<uint8_t>& on, ScatterLists& L);
+                         const TuneParams& tune, const std::vector<uint8_t>& on, bool fp32, ScatterLists& L);
 void set_error(const std::string& s);
 }  // namespace cad

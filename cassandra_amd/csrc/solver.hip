@@ -60,23 +60,21 @@ void allow_lds(K kernel, size_t bytes)
 }
 
 // The scatter windows: every real-valued scatter accumulates in 8-byte LDS
-// words (FP64, or the 64-bit fixed point of the FP32 stored-index scatter), so
-// it uses the 8-byte windows whatever its value type (f4 serves the u32
-// multiplicity counts of the Jacobi diagonal).
+// words (FP64, or the 64-bit fixed point of the FP32 scatter), each value type
+// with row chunks of its own (f4 serves the u32 multiplicity counts of the
+// Jacobi diagonal).
 template <class VT>
 ScatterLists& lists(ScatterPlan& sp)
 {
-    return sp.f8;
+    return sizeof(VT) == 4 ? sp.f8s : sp.f8;
 }
 
-// The partial buffer of a scatter list, sized for 8-byte elements whatever PT
-// is: FP32 and FP64 scatters share the list, and a buffer grown for one
-// precision would free the one a captured graph of the other still uses.
-// (Allocated outside graph capture: every solver calls prepare_scatter first.)
+// The partial buffer of a scatter list (allocated outside graph capture: every
+// solver calls prepare_scatter first).
 template <class PT>
 PT* partials(ScatterLists& L)
 {
-    const size_t bytes = sizeof(double) * size_t(std::max<int64_t>(1, L.part_elems));
+    const size_t bytes = sizeof(PT) * size_t(std::max<int64_t>(1, L.part_elems));
     if (L.part.bytes < bytes) L.part = DBuf(bytes);
     return L.part.as<PT>();
 }
@@ -626,7 +624,7 @@ static void build_active(cad_matrix* m, ActiveLists& al, const std::vector<int>&
     // side (few in the tail of a batch, where the systems left are small)
     ScatterLists sub;
     plan_scatter_subset(m->splan, m->sys_row_begin, m->sys_col, m->cols_per_sys, m->mf ? 2 : m->ibytes, *m->ctx,
-                        m->tune, al.on, sub);
+                        m->tune, al.on, sizeof(VT) == 4, sub);
     al.ntiles = int(t.size());
     al.nscatter = int(sub.work.size());
     al.nreduce = int(sub.reduce.size());
@@ -1437,17 +1435,20 @@ void set_schedule(cad_matrix* m, const TuneParams& tp)
     drop_graphs(m);
     const TuneParams keep = m->tune;
     m->tune = tp;
-    build_gather_plan(m, m->gplan4, 4, tp.rpt4, tp.bs4, tp.sub4);
-    build_gather_plan(m, m->gplan8, 8, tp.rpt8, tp.bs8, tp.sub8);
+    Uploads up;
+    build_gather_plan(m, m->gplan4, 4, tp.rpt4, tp.bs4, tp.sub4, up);
+    build_gather_plan(m, m->gplan8, 8, tp.rpt8, tp.bs8, tp.sub8, up);
     if ((tp.rpt4 > 0 && !m->gplan4.ok) || (tp.rpt8 > 0 && !m->gplan8.ok)) {
         m->tune = keep;
-        build_gather_plan(m, m->gplan4, 4, keep.rpt4, keep.bs4, keep.sub4);
-        build_gather_plan(m, m->gplan8, 8, keep.rpt8, keep.bs8, keep.sub8);
+        Uploads back;
+        build_gather_plan(m, m->gplan4, 4, keep.rpt4, keep.bs4, keep.sub4, back);
+        build_gather_plan(m, m->gplan8, 8, keep.rpt8, keep.bs8, keep.sub8, back);
+        back.flush(m->ctx->stream);
         throw Error(CAD_ERR_ARGUMENT, "this matrix cannot use the tile gather");
     }
     build_scatter_plan(m->splan, m->slot_lo, m->slot_hi, m->sys_row_begin, m->sys_col, m->cols_per_sys,
-                       m->mf ? 2 : m->ibytes, *m->ctx, tp);
-    CAD_HIP(hipStreamSynchronize(m->ctx->stream));
+                       m->mf ? 2 : m->ibytes, *m->ctx, tp, true, up);
+    up.flush(m->ctx->stream);
 }
 
 void kernel_times(cad_matrix* m, int reps, double* us, int n)
@@ -1512,7 +1513,9 @@ std::string autotune(cad_matrix* m)
         GShape best{rpt, bs, sub};
         double best_us = 1e300;
         for (const GShape& c : cands) {
-            build_gather_plan(m, gp, vbytes, c.rpt, c.bs, c.sub);
+            Uploads up;
+            build_gather_plan(m, gp, vbytes, c.rpt, c.bs, c.sub, up);
+            up.flush(s);
             if (c.rpt > 0 && !gp.ok) continue;
             const double us = t.us(run, s);
             std::snprintf(line, sizeof line, "gather f%d rpt %d block %d sub %d: %.1f us\n", 8 * vbytes, c.rpt, c.bs,
@@ -1523,7 +1526,9 @@ std::string autotune(cad_matrix* m)
         rpt = best.rpt;
         bs = best.bs;
         sub = best.sub;
-        build_gather_plan(m, gp, vbytes, rpt, bs, sub);
+        Uploads up;
+        build_gather_plan(m, gp, vbytes, rpt, bs, sub, up);
+        up.flush(s);
     };
     tune_gather(4, (!m->mf && m->ibytes == 2) ? std::vector<int>{4, 8, 2, 0} : std::vector<int>{4, 2, 0}, tp.rpt4,
                 tp.bs4, tp.sub4, [&] { spmv<float>(m, x4.as<float>(), y4.as<float>(), s); });
@@ -1550,13 +1555,15 @@ std::string autotune(cad_matrix* m)
             tp.blocks_per_cu = c.bpc;
             tp.partial_cap = c.cap;
             tp.scatter_balance = c.bal;
+            Uploads up;
             build_scatter_plan(m->splan, m->slot_lo, m->slot_hi, m->sys_row_begin, m->sys_col, m->cols_per_sys,
-                               m->mf ? 2 : m->ibytes, *m->ctx, tp);
+                               m->mf ? 2 : m->ibytes, *m->ctx, tp, true, up);
+            up.flush(s);
             const double us =
                 t.us([&] { scatter<float, float, float>(m, y4.as<float>(), nullptr, z4.as<float>(), s); }, s);
             std::snprintf(line, sizeof line,
                           "scatter f32 order %d rpt %d blocks/CU %.0f cap %.2f balance %.2f (%zu tiles): %.1f us\n",
-                          c.order, c.srpt, c.bpc, c.cap, c.bal, m->splan.f8.work.size(), us);
+                          c.order, c.srpt, c.bpc, c.cap, c.bal, m->splan.f8s.work.size(), us);
             log += line;
             // a later candidate must win by 2 %, and a per-window (order 0)
             // one over the chunk-shared XCD-major order, which comes first, by
@@ -1573,8 +1580,10 @@ std::string autotune(cad_matrix* m)
         tp.blocks_per_cu = best.bpc;
         tp.partial_cap = best.cap;
         tp.scatter_balance = best.bal;
+        Uploads up;
         build_scatter_plan(m->splan, m->slot_lo, m->slot_hi, m->sys_row_begin, m->sys_col, m->cols_per_sys,
-                           m->mf ? 2 : m->ibytes, *m->ctx, tp);
+                           m->mf ? 2 : m->ibytes, *m->ctx, tp, true, up);
+        up.flush(s);
     }
     CAD_HIP(hipStreamSynchronize(s));
     m->tuned = true;
