@@ -270,8 +270,10 @@ const ScatterPlan& eval_plan(cad_patterns* p, int64_t B)
 
 // The backward's first stage (B > 0): the window tiles of the evaluator's
 // scatter plan into its partial slices; returns the plan's lists and slices.
-template <class VT, class View>
-ScatterLists& eval_backward_windows(cad_patterns* p, const View& view, int64_t B, const VT* g, VT*& part)
+// Entry (r, s) is idx[r * row_stride + s * slot_stride].
+template <class VT>
+ScatterLists& eval_backward_windows(cad_patterns* p, const int32_t* idx, int64_t row_stride, int64_t slot_stride,
+                                    int64_t B, const VT* g, VT*& part)
 {
     hipStream_t s = p->ctx->stream;
     ScatterPlan& sp = const_cast<ScatterPlan&>(eval_plan(p, B));
@@ -281,21 +283,20 @@ ScatterLists& eval_backward_windows(cad_patterns* p, const View& view, int64_t B
     part = L.part.as<VT>();
     if (!L.work.empty()) {
         const size_t lds = size_t(L.widest) * sizeof(double);
-        auto kern = k_scatter_part<VT, VT, View>;
+        auto kern = k_scatter_part<VT>;
         if (lds > 64 * 1024)
             (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
-        hipLaunchKernelGGL(kern, dim3(unsigned(L.work.size())), dim3(kScatterBlock), lds, s,
-                           view, L.d_work.as<ScatterWork>(), L.d_groups.as<SlotGroup>(),
-                           L.d_slot_list.as<uint16_t>(), p->d_syscol0.as<uint32_t>(), g,
-                           (LsqrScalars*)nullptr, kScatterAll, FixedScale{nullptr, 0}, 0, part, GridSys{});
+        hipLaunchKernelGGL(kern, dim3(unsigned(L.work.size())), dim3(kScatterBlock), lds, s, idx, row_stride,
+                           slot_stride, L.d_work.as<ScatterWork>(), L.d_groups.as<SlotGroup>(),
+                           L.d_slot_list.as<uint16_t>(), g, part);
         CAD_HIP(hipGetLastError());
     }
     return L;
 }
 
-template <class VT, class View>
-void eval_backward_view(cad_patterns* p, const View& view, int64_t B, const VT* g, VT* grad)
+template <class VT>
+void eval_backward(cad_patterns* p, const int32_t* idx, int64_t B, const VT* g, VT* grad)
 {
     hipStream_t s = p->ctx->stream;
     const int64_t C = int64_t(p->group->cols());
@@ -305,17 +306,15 @@ void eval_backward_view(cad_patterns* p, const View& view, int64_t B, const VT* 
         return;
     }
     VT* part = nullptr;
-    ScatterLists& L = eval_backward_windows<VT>(p, view, B, g, part);
+    ScatterLists& L = eval_backward_windows<VT>(p, idx, p->group->k(), 1, B, g, part);
     hipLaunchKernelGGL((k_scatter_reduce<VT, VT>), dim3(unsigned(L.reduce.size())), dim3(kRowBlock), 0, s,
                        L.d_reduce.as<ReduceWork>(), (const VT*)part, grad, (const LsqrScalars*)nullptr, kScatterAll);
     CAD_HIP(hipGetLastError());
 }
 
-template <class VT>
-void eval_backward(cad_patterns* p, const int32_t* idx, int64_t B, const VT* g, VT* grad)
-{
-    eval_backward_view<VT>(p, RowMajor32{idx, p->group->k()}, B, g, grad);
-}
+// Rows of k entries that start at multiples of 8 bytes (their entries can be
+// read in pairs).
+bool pair_rows(const int32_t* idx, int k) { return k % 2 == 0 && reinterpret_cast<uintptr_t>(idx) % 8 == 0; }
 
 // One Adam step of the Huber-loss fit on the minibatch rows sel[0..B): the
 // forward with the loss and its gradient (which also copies the minibatch's
@@ -342,18 +341,18 @@ void train_step(cad_patterns* p, const int32_t* idx, const float* target, const 
     int32_t* rows = p->d_train_rows.as<int32_t>();
     const AdamStep a{lr, b1, b2, eps, 1.0f - std::pow(b1, float(step)), std::sqrt(1.0f - std::pow(b2, float(step)))};
     if (B > 0) {
-        hipLaunchKernelGGL(k_train_forward, dim3(nblk), dim3(kRowBlock), 0, s, idx, sel, B, k, w, uint32_t(C), target,
-                           delta, g, part, rows);
-        // the backward's window tiles over the contiguous copy of the
+        hipLaunchKernelGGL(pair_rows(idx, k) ? k_train_forward<2> : k_train_forward<1>, dim3(nblk), dim3(kRowBlock), 0,
+                           s, idx, sel, B, k, w, uint32_t(C), target, delta, g, part, rows);
+        // the backward's window tiles over the slot-major copy of the
         // minibatch's rows, then their column sums with the Adam update
         float* gpart = nullptr;
-        ScatterLists& L = eval_backward_windows<float>(p, RowMajor32{rows, k}, B, g, gpart);
+        ScatterLists& L = eval_backward_windows<float>(p, rows, 1, B, B, g, gpart);
         hipLaunchKernelGGL(k_adam_reduce, dim3(unsigned(L.reduce.size())), dim3(kRowBlock), 0, s,
                            L.d_reduce.as<ReduceWork>(), (const float*)gpart, w, m, v, a, (const double*)part, nblk, B,
                            loss);
     } else {
         // no rows: a zero gradient (Adam still moves the weights by its moments)
-        eval_backward_view<float>(p, RowMajor32{rows, k}, B, g, grad);
+        eval_backward<float>(p, rows, B, g, grad);
         hipLaunchKernelGGL(k_adam, dim3(grid1(C, kRowBlock)), dim3(kRowBlock), 0, s, w, (const float*)grad, m, v, C, a,
                            (const double*)part, 0, int64_t(1), loss);
     }
@@ -364,8 +363,10 @@ template <class VT>
 void eval_forward(cad_patterns* p, const int32_t* idx, int64_t B, const VT* w, VT* out)
 {
     if (B <= 0) return;
-    hipLaunchKernelGGL(k_eval_forward<VT>, dim3(grid1(B, kRowBlock)), dim3(kRowBlock), 0, p->ctx->stream, idx, B,
-                       p->group->k(), w, uint32_t(p->group->cols()), out);
+    const int k = p->group->k();
+    auto kern = pair_rows(idx, k) ? k_eval_forward<VT, 2> : k_eval_forward<VT, 1>;
+    hipLaunchKernelGGL(kern, dim3(grid1(B, kRowBlock)), dim3(kRowBlock), 0, p->ctx->stream, idx, B, k, w,
+                       uint32_t(p->group->cols()), out);
     CAD_HIP(hipGetLastError());
 }
 

@@ -83,8 +83,7 @@ PT* partials(ScatterLists& L)
 // column reduction in chunk order (which writes every column of z).
 // The first-stage scatter kernel of a view: vector loads of rpt (4, or 8 for
 // u16 indices) consecutive rows for stored indices, two runs of 64 rows a wave
-// and step for a matrix-free matrix, one row per step otherwise; f receives the
-// kernel.  beta: the instantiation that forms an LSQR iteration's beta itself;
+// and step for a matrix-free matrix; f receives the kernel.  beta: the instantiation that forms an LSQR iteration's beta itself;
 // ymax: the instantiation that forms each system's max |y| from the row-block
 // maxima (FixedScale::ypart), used by FP32 PCG.
 template <class VT, class YT, class View, class F>
@@ -97,10 +96,8 @@ void with_scatter_kernel(int rpt, bool beta, bool ymax, F&& f)
             return f(k_scatter_tile<VT, YT, uint16_t, 4, B, Y>);
         } else if constexpr (std::is_same_v<View, SlotMajor<uint32_t>>) {
             return f(k_scatter_tile<VT, YT, uint32_t, 4, B, Y>);
-        } else if constexpr (std::is_same_v<View, PositionsView>) {
-            return f(k_scatter_tile_mf<VT, YT, 2, B, Y>);
         } else {
-            return f(k_scatter_part<VT, YT, View, B>);
+            return f(k_scatter_tile_mf<VT, YT, 2, B, Y>);
         }
     };
     if (beta) return pick(std::true_type{}, std::false_type{});
