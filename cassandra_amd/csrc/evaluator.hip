@@ -1,8 +1,8 @@
 // The expanded-table evaluator on the device: expansion of compact weights
 // into one table of 3^n floats per variation (ScoreEstimator's constructor,
 // Pattern/Evaluator.cpp:11-29), compaction back (ScoreEstimator::Weights,
-// Pattern/Evaluator.cpp:56-73), and a resident evaluator that keeps the
-// tables in HBM and scores batches of positions (ScoreEstimator::Eval,
+// Pattern/Evaluator.cpp:56-73), and a resident evaluator that keeps its
+// weights in HBM and scores batches of positions (ScoreEstimator::Eval,
 // Pattern/Evaluator.cpp:48-54, for the leaves of a search).
 #include "evaluator.hpp"
 
@@ -107,43 +107,141 @@ __global__ __launch_bounds__(256) void k_compact_write(const EvalSlot* __restric
 
 // Eval for every position: the sum over the variations of table_i[FastIndex(
 // pos, mask_i)], in variation order from 0.0f (bit-identical to
-// ScoreEstimator::Eval and to (A x)[row]).  A thread scores kEvalRows
-// positions (r, r + 256, ...) from their ternary words; each variation's
-// FastIndex is its ternary-word program (the variation's squares in
-// ascending order), read once for all of them.  The descriptors are the same
-// for the whole wave.
-constexpr int kEvalRows = 4;
+// ScoreEstimator::Eval and to (A x)[row]).  The evaluator keeps the compact
+// weights, not the expanded tables: every variation of a pattern reads the
+// same columns, which an index tile computes for 64 positions and four
+// variations with four matrix instructions; 52 slots of 12 patterns read 0.7 MB
+// where their tables are 5.4 MB.
+constexpr int kEvalBlock = 1024;
 
-__global__ __launch_bounds__(256) void k_eval_tables(const uint64_t* __restrict__ pos, int64_t n,
-                                                     const EvalSlot* __restrict__ es,
-                                                     const DevTern* __restrict__ ts,
-                                                     const uint32_t* __restrict__ tern, int k,
-                                                     const float* __restrict__ tables, float* __restrict__ out)
+// Small batches: a block takes 64 positions, a wave of it one index tile, and
+// the values meet in LDS, where wave 0 adds them in slot order (0.0f for the
+// slots a tile does not have: no partial sum is -0.0f).  Walking the slots in
+// one thread took a dependent chain of descriptor, program and table loads per
+// slot: 64 positions x 52 slots 16.4 µs against 3.8 here, 65,536 12.0 (4
+// patterns, 18 slots: 5.6, slot by slot 15.8).  Bound by latency, and above
+// 30,000 positions by the columns' lines in L1.
+__global__ __launch_bounds__(kEvalBlock) void k_eval_block(const uint64_t* __restrict__ pos, int64_t n, TileView tv,
+                                                           const float* __restrict__ w, uint32_t cols,
+                                                           float* __restrict__ out)
 {
-    const int64_t r0 = blockIdx.x * int64_t(256 * kEvalRows) + threadIdx.x;
-    if (r0 >= n) return;
-    uint32_t T[kEvalRows][4];
-    bool ok[kEvalRows];
-    float sum[kEvalRows];
+    __shared__ uint32_t words[64 * 4];
+    __shared__ float vals[kEvalBlock / 64][4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = int(blockDim.x) >> 6;
+    const int64_t base = blockIdx.x * int64_t(64);
+    TileRegs next = load_tile(tv, min(wave, tv.n - 1));
+    if (wave == 0) {
+        const int64_t r = min(base + lane, n - 1);
+        uint32_t T[4];
+        ternary_words(pos[2 * r], pos[2 * r + 1], T);
 #pragma unroll
-    for (int i = 0; i < kEvalRows; i++) {
-        const int64_t r = r0 + int64_t(i) * 256;
-        ok[i] = r < n;
-        const int64_t rr = ok[i] ? r : r0;  // a valid row's words for the lanes past the end
-        ternary_words(pos[2 * rr], pos[2 * rr + 1], T[i]);
-        sum[i] = 0.0f;
+        for (int i = 0; i < 4; i++) words[4 * lane + i] = T[i];
     }
-    for (int s = 0; s < k; s++) {
-        const EvalSlot e = uniform_load(es + s);
-        const DevTern t = uniform_load(ts + s);
-        uint32_t v[kEvalRows];
-        tern_values<kEvalRows>(tern, t.off[0], t.nent[0], T, v);
+    __syncthreads();
+    Int4 b[4];
 #pragma unroll
-        for (int i = 0; i < kEvalRows; i++) sum[i] += tables[e.table_offset + v[i]];
+    for (int p = 0; p < 4; p++) b[p] = expand_digits(words[4 * (16 * p + (lane & 15)) + (lane >> 4)]);
+    float sum = 0.0f;
+    for (int t0 = 0; t0 < tv.n; t0 += nw) {
+        const int t = t0 + wave;
+        if (t < tv.n) {
+            const TileRegs cur = next;
+            const IndexTile tl = cur.tile();
+            next = load_tile(tv, min(t + nw, tv.n - 1));
+            uint32_t ci[4];
+            tile_columns(tl, t, tv, cur.weights, b, ci);
+            transpose_groups(ci);
+            float x[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = w[min(tl.col_offset + ci[j], cols - 1)];
+#pragma unroll
+            for (int j = 0; j < 4; j++) vals[wave][j][lane] = j < tl.nslots ? x[j] : 0.0f;
+        }
+        __syncthreads();
+        if (wave == 0) {
+            const int m = min(nw, tv.n - t0);
+            for (int i = 0; i < m; i++) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) sum += vals[i][j][lane];
+            }
+        }
+        if (t0 + nw < tv.n) __syncthreads();
     }
+    if (wave == 0 && base + lane < n) out[base + lane] = sum;
+}
+
+// Large batches: one block a CU keeps the weights of the patterns with the
+// most variations a column in LDS (EvalPlan) and its waves walk the positions,
+// 64 C at a time; the other patterns' weights come through L1, where a wave's
+// load of 64 columns takes as many lines, and which bounds the kernel (20 of the
+// 52 slots of 12 patterns: 64 x 20 lines a wave are about 0.85 of its time).
+// 1M positions of 12 patterns: 59 µs, 85 from the expanded tables, 135 with no
+// weights in LDS; of 4 patterns 40 (52 with none).  Two runs of positions a wave
+// share a tile's weights and hide each other's latency (1M: 64 µs with one);
+// where one run a wave covers the batch, one is faster (262,144: 22 against 29).
+// A second phase of staging in place of the L1 loads would cost what it saves:
+// 160 KB for each CU take as long as 4 slots of its 4,000 positions.
+template <int C>
+__global__ __launch_bounds__(kEvalBlock) void k_eval_staged(const uint64_t* __restrict__ pos, int64_t n, TileView tv,
+                                                            const int32_t* __restrict__ tile_lds,
+                                                            const PhaseSeg* __restrict__ segs, int nsegs,
+                                                            const float* __restrict__ w, uint32_t cols,
+                                                            float* __restrict__ out)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    float* xs = reinterpret_cast<float*>(smem_raw);
+    for (int s = 0; s < nsegs; s++) {
+        const PhaseSeg ps = uniform_load(segs + s);
+        stage_direct<float, kEvalBlock>(xs + ps.lds_off, w + ps.col_lo, ps.width);
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t step = int64_t(gridDim.x) * (kEvalBlock * C);
+    for (int64_t base = (blockIdx.x * int64_t(kEvalBlock / 64) + wave) * (64 * C); base < n; base += step) {
+        Int4 b[C][4];
+        float sum[C];
 #pragma unroll
-    for (int i = 0; i < kEvalRows; i++)
-        if (ok[i]) out[r0 + int64_t(i) * 256] = sum[i];
+        for (int c = 0; c < C; c++) {
+            sum[c] = 0.0f;
+#pragma unroll
+            for (int p = 0; p < 4; p++)
+                b[c][p] = digits_of_position(pos, min(base + 64 * c + 16 * p + (lane & 15), n - 1));
+        }
+        TileRegs next = load_tile(tv, 0);
+        int next_lds = tile_lds[0];
+        for (int t = 0; t < tv.n; t++) {
+            const TileRegs cur = next;
+            const IndexTile tl = cur.tile();
+            const int at = __builtin_amdgcn_readfirstlane(next_lds);
+            const int nt = min(t + 1, tv.n - 1);
+            next = load_tile(tv, nt);
+            next_lds = tile_lds[nt];
+            float x[C][4];
+#pragma unroll
+            for (int c = 0; c < C; c++) {
+                uint32_t ci[4];
+                tile_columns(tl, t, tv, cur.weights, b[c], ci);
+                transpose_groups(ci);
+                if (at >= 0) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) x[c][j] = xs[uint32_t(at) + ci[j]];
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) x[c][j] = w[min(tl.col_offset + ci[j], cols - 1)];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (j < tl.nslots) {
+#pragma unroll
+                    for (int c = 0; c < C; c++) sum[c] += x[c][j];
+                }
+        }
+#pragma unroll
+        for (int c = 0; c < C; c++)
+            if (base + 64 * c + lane < n) out[base + 64 * c + lane] = sum[c];
+    }
 }
 
 int blocks_for(uint64_t n, int cap = 4096)
@@ -152,6 +250,13 @@ int blocks_for(uint64_t n, int cap = 4096)
 }
 
 }  // namespace
+
+// Positions a CU from which a batch is scored from LDS: the staging costs about
+// 6 µs and a pass of the staged block is long (131,072 positions on 256 CUs,
+// block / staged: 12 patterns of 52 slots 21.4 / 18.4 µs, of 54 slots 21.3 /
+// 20.3, 46 slots 15.2 / 16.4, 4 patterns 9.4 / 11.3; twice as many: 38.7 / 21.7,
+// 38.2 / 23.1, 27.5 / 17.2, 16.2 / 13.6).
+constexpr int64_t kEvalStagedRows = 512;
 
 // Per-slot table layout of a pattern group (variation after variation, in
 // slot order), uploaded once per pattern group.
@@ -181,21 +286,9 @@ const ExpandedLayout& expanded_layout(cad_patterns* p)
         }
     }
     if (slot != g.k()) throw Error(CAD_ERR_PATTERN, "variation count differs from the slot count");
-    // each variation's FastIndex as a ternary-word program (list 0)
-    std::vector<DevTern> ts;
-    std::vector<uint32_t> tern;
-    for (const EvalSlot& e : es) {
-        DevTern t;
-        std::memset(&t, 0, sizeof(t));
-        append_ternary_list(e.sq, int(e.n), tern, t, 0);
-        ts.push_back(t);
-    }
-    tern.insert(tern.end(), kTernPadding, 0u);
     L->slots = es;
     L->size = int64_t(off);
     hipStream_t s = p->ctx->stream;
-    L->d_tslots = to_device(ts, s);
-    L->d_tern = to_device(tern, s);
     L->d_slots = to_device(es, s);
     L->d_first_slot = to_device(L->first_slot, s);
     CAD_HIP(hipStreamSynchronize(s));  // the host vectors are uploaded
@@ -236,14 +329,98 @@ void weights_compact(cad_patterns* p, const float* tables, float* w)
     CAD_HIP(hipStreamSynchronize(s));  // the key buffer is freed on return
 }
 
-void eval_tables(cad_patterns* p, const float* tables, const uint64_t* pos, int64_t n, float* out)
+const EvalPlan& eval_weights_plan(cad_patterns* p)
+{
+    if (p->eval_plan) return *p->eval_plan;
+    std::unique_ptr<EvalPlan> E(new EvalPlan);
+    const PatternGroup& g = *p->group;
+    for (const PatternInfo& pi : g.patterns)
+        if (__builtin_popcountll(pi.mask) > 16)
+            throw Error(CAD_ERR_PATTERN, "expanded tables need patterns of at most 16 squares");
+    // the patterns with the fewest columns a variation first
+    std::vector<size_t> order(g.patterns.size());
+    for (size_t i = 0; i < order.size(); i++) order[i] = i;
+    std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) {
+        const PatternInfo &x = g.patterns[a], &y = g.patterns[b];
+        return uint64_t(x.size) * y.variations.size() < uint64_t(y.size) * x.variations.size();
+    });
+    const uint64_t room = std::min<size_t>(p->ctx->max_lds, 160 * 1024) / sizeof(float);
+    std::vector<PhaseSeg> segs;
+    std::vector<int32_t> pattern_lds(g.patterns.size(), -1), tile_lds(size_t(std::max(1, p->ntiles)), -1);
+    uint64_t used = 0;
+    for (size_t i : order) {
+        // a segment keeps its columns' places within a 16-byte line
+        const PatternInfo& pi = g.patterns[i];
+        const uint32_t head = pi.offset & 3u;
+        const uint64_t need = (uint64_t(head) + pi.size + 3) & ~uint64_t(3);
+        if (used + need > room) continue;
+        segs.push_back(PhaseSeg{pi.offset, pi.size, uint32_t(used), 0});
+        pattern_lds[i] = int32_t(used + head);
+        used += need;
+    }
+    int slot = 0;
+    for (size_t i = 0; i < g.patterns.size(); i++)
+        for (size_t v = 0; v < g.patterns[i].variations.size(); v++)
+            tile_lds[p->slot_tile[size_t(slot++)]] = pattern_lds[i];
+    if (slot != g.k()) throw Error(CAD_ERR_PATTERN, "variation count differs from the slot count");
+    E->nsegs = int(segs.size());
+    E->lds = size_t(used) * sizeof(float);
+    hipStream_t s = p->ctx->stream;
+    E->d_segs = to_device(segs, s);
+    E->d_tile_lds = to_device(tile_lds, s);
+    CAD_HIP(hipStreamSynchronize(s));  // the host vectors are uploaded
+    p->eval_plan = std::move(E);
+    return *p->eval_plan;
+}
+
+void eval_weights(cad_patterns* p, const float* w, const uint64_t* pos, int64_t n, float* out)
 {
     if (n <= 0) return;
-    const ExpandedLayout& L = expanded_layout(p);
-    hipLaunchKernelGGL(k_eval_tables, dim3(unsigned((n + 256 * kEvalRows - 1) / (256 * kEvalRows))), dim3(256), 0,
-                       p->ctx->stream, pos, n, L.d_slots.as<EvalSlot>(), L.d_tslots.as<DevTern>(),
-                       L.d_tern.as<uint32_t>(), int(L.slots.size()), tables, out);
+    const EvalPlan& E = eval_weights_plan(p);
+    const TileView tv = p->tiles();
+    const uint32_t cols = uint32_t(p->group->cols());
+    hipStream_t s = p->ctx->stream;
+    if (tv.n == 0) {
+        hipLaunchKernelGGL(k_fill<float>, dim3(unsigned(blocks_for(uint64_t(n)))), dim3(256), 0, s, out, n, 0.0f);
+    } else if (E.nsegs > 0 && n >= kEvalStagedRows * p->ctx->cus) {
+        const int C = n <= int64_t(p->ctx->cus) * kEvalBlock ? 1 : 2;
+        auto kern = C == 1 ? k_eval_staged<1> : k_eval_staged<2>;
+        if (E.lds > 64 * 1024)
+            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      int(E.lds));
+        const int64_t blocks = std::min<int64_t>(p->ctx->cus, (n + kEvalBlock * C - 1) / (kEvalBlock * C));
+        hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(kEvalBlock), E.lds, s, pos, n, tv,
+                           E.d_tile_lds.as<int32_t>(), E.d_segs.as<PhaseSeg>(), E.nsegs, w, cols, out);
+    } else {
+        const int waves = std::min(kEvalBlock / 64, tv.n);
+        hipLaunchKernelGGL(k_eval_block, dim3(unsigned((n + 63) / 64)), dim3(unsigned(64 * waves)), 0, s, pos, n, tv, w,
+                           cols, out);
+    }
     CAD_HIP(hipGetLastError());
 }
 
 }  // namespace cad
+
+void cad_evaluator::pin(int64_t n)
+{
+    if (n <= pinned) return;
+    CAD_HIP(hipStreamSynchronize(ctx->stream));
+    const int64_t m = std::max(n, 2 * pinned);  // (a search's batches grow in small steps)
+    uint64_t* a = nullptr;
+    float* b = nullptr;
+    CAD_HIP(hipHostMalloc(reinterpret_cast<void**>(&a), sizeof(uint64_t) * 2 * size_t(m), hipHostMallocDefault));
+    const hipError_t rc = hipHostMalloc(reinterpret_cast<void**>(&b), sizeof(float) * size_t(m), hipHostMallocDefault);
+    if (rc != hipSuccess) (void)hipHostFree(a);
+    CAD_HIP(rc);
+    if (h_pos) (void)hipHostFree(h_pos);
+    if (h_out) (void)hipHostFree(h_out);
+    h_pos = a;
+    h_out = b;
+    pinned = m;
+}
+
+cad_evaluator::~cad_evaluator()
+{
+    if (h_pos) (void)hipHostFree(h_pos);
+    if (h_out) (void)hipHostFree(h_out);
+}

@@ -224,7 +224,15 @@ struct ExpandedLayout {
     std::vector<int32_t> first_slot;  // first slot (variation 0) of each pattern
     int64_t size = 0;                 // floats of all tables
     DBuf d_slots, d_first_slot;
-    DBuf d_tslots, d_tern;            // FastIndex of every variation as a ternary-word program
+};
+
+// The weights the evaluator of a pattern group keeps in LDS: the column ranges
+// of whole patterns, and for every index tile the LDS place of its pattern's
+// first column (-1: not in LDS).
+struct EvalPlan {
+    DBuf d_segs, d_tile_lds;
+    int nsegs = 0;
+    size_t lds = 0;  // bytes
 };
 
 struct Context {
@@ -254,20 +262,27 @@ struct cad_patterns {
     std::map<int64_t, std::unique_ptr<cad::ScatterPlan>> eval_plans;
     cad::DBuf d_base0, d_syscol0;            // zeros
     std::unique_ptr<cad::ExpandedLayout> layout;  // expanded tables (built on first use)
+    std::unique_ptr<cad::EvalPlan> eval_plan;     // the evaluator's (built on first use)
     // the training step's buffers: per-row gradient of the loss, the weight
     // gradient, the forward's block sums of the loss, the minibatch's index
     // rows made contiguous (grown on demand)
     cad::DBuf d_train_g, d_train_grad, d_train_part, d_train_rows;
 };
 
-// A resident evaluator: the expanded tables of one weight vector in HBM and
-// staging for host batches (ScoreEstimator on the device).
+// A resident evaluator: one weight vector in HBM and staging for host batches
+// (ScoreEstimator on the device).
 struct cad_evaluator {
     cad_context* ctx = nullptr;        // the pattern group's context
     cad_patterns* patterns = nullptr;
-    cad::DBuf tables;
+    cad::DBuf weights;
     cad::DBuf d_pos, d_out;     // staging of cad_evaluator_eval_host
     int64_t staged = 0;         // rows the staging holds
+    // the same in pinned host memory, for small batches (grown on demand)
+    uint64_t* h_pos = nullptr;
+    float* h_out = nullptr;
+    int64_t pinned = 0;
+    void pin(int64_t n);
+    ~cad_evaluator();
 };
 
 struct cad_matrix {
