@@ -870,6 +870,22 @@ __global__ __launch_bounds__(kRowBlock) void k_epi_finish(Epi epi, GridSys g)
     if (threadIdx.x == 0) epi.finish(sys, s);
 }
 
+// One block per system: the sums of both slots of the system's block partials
+// handed to f, in the order of the last-block ticket's sums.  For the column
+// kernels at a solve's start and end, whose tickets' fences (an L2 write-back
+// and invalidate a block) took most of their time: 16 systems of 102,222
+// columns, |z|^2 76 -> 6 + 5 µs, the start of PCG 130 -> 12 + 5; one such
+// system 8.6 -> 3 + 3.
+template <class F>
+__global__ __launch_bounds__(kRowBlock) void k_system_finish(F f, GridSys g)
+{
+    __shared__ double sh[kRowBlock / 64];
+    if (!f.begin(blockIdx.x)) return;
+    double s0, s1;
+    system_sum2<kRowBlock>(g, blockIdx.x, sh, s0, s1);
+    if (threadIdx.x == 0) f.finish(blockIdx.x, s0, s1);
+}
+
 template <class VT, class View>
 __device__ __forceinline__ VT row_sum(const View& m, int k, int64_t r, uint32_t cb, const VT* __restrict__ x)
 {
@@ -1683,35 +1699,6 @@ __global__ __launch_bounds__(kTileBlock) void k_gather_tile_mf(PositionsView m, 
     reduce_tail<kTileBlock>(epi, red, w.sys, g);
 }
 
-// Rows init of LSQR: u_raw = src (converted), beta = |src| (FP64).
-template <class VT>
-__global__ __launch_bounds__(kRowBlock) void k_lsqr_init_u(const RowWork* __restrict__ work,
-                                                           const double* __restrict__ src, VT* __restrict__ u,
-                                                           GridSys g, LsqrScalars* scal)
-{
-    __shared__ double sh[kRowBlock / 64];
-    const RowWork w = work[blockIdx.x];
-    LsqrScalars* st = &scal[w.sys];
-    if (!st->active) return;
-    double acc = 0.0;
-    for (int64_t r = w.row_begin + threadIdx.x; r < w.row_end; r += kRowBlock) {
-        const double v = src[r];
-        u[r] = VT(v);
-        acc += v * v;
-    }
-    acc = block_sum<kRowBlock>(acc, sh);
-    if (threadIdx.x == 0) g.partials[2 * blockIdx.x] = acc;
-    if (arrive_last(&g.counters[w.sys], g.blk_count[w.sys])) {
-        double s = 0.0;
-        for (int i = threadIdx.x; i < g.blk_count[w.sys]; i += kRowBlock) s += g.partials[2 * (g.blk_first[w.sys] + i)];
-        s = block_sum<kRowBlock>(s, sh);
-        if (threadIdx.x == 0) {
-            st->beta = sqrt(s);
-            st->anorm2 = 0.0;
-        }
-    }
-}
-
 // ------------------------------------------------------------ scatter ------
 // Which systems a scatter serves, and its scale:
 //   kScatterAll      every system, scale 1 (plain products)
@@ -2487,11 +2474,11 @@ __global__ __launch_bounds__(kRowBlock) void k_lsqr_step(const ColWork* __restri
 template <class ZT>
 __global__ __launch_bounds__(kRowBlock) void k_lsqr_init_v(const ColWork* __restrict__ work,
                                                            const double* __restrict__ D, const ZT* __restrict__ z,
-                                                           double* __restrict__ v, GridSys g, LsqrScalars* scal)
+                                                           double* __restrict__ v, GridSys g, const LsqrScalars* scal)
 {
     __shared__ double sh[kRowBlock / 64];
     const ColWork w = work[blockIdx.x];
-    LsqrScalars* st = &scal[w.sys];
+    const LsqrScalars* st = &scal[w.sys];
     if (!st->active || !st->restart) return;
     const double ib = st->beta != 0.0 ? 1.0 / st->beta : 0.0;
     double a0 = 0.0, a1 = 0.0;
@@ -2508,29 +2495,27 @@ __global__ __launch_bounds__(kRowBlock) void k_lsqr_init_v(const ColWork* __rest
         g.partials[2 * blockIdx.x] = a0;
         g.partials[2 * blockIdx.x + 1] = a1;
     }
-    if (arrive_last(&g.counters[w.sys], g.blk_count[w.sys])) {
-        double s0 = 0.0, s1 = 0.0;
-        for (int i = threadIdx.x; i < g.blk_count[w.sys]; i += kRowBlock) {
-            s0 += g.partials[2 * (g.blk_first[w.sys] + i)];
-            s1 += g.partials[2 * (g.blk_first[w.sys] + i) + 1];
-        }
-        s0 = block_sum<kRowBlock>(s0, sh);
-        s1 = block_sum<kRowBlock>(s1, sh);
-        if (threadIdx.x == 0) {
-            const double alpha = sqrt(s0);
-            st->alpha = alpha;
-            st->rhobar = alpha;
-            st->phibar = st->beta;
-            st->nres0 = alpha * st->beta;
-            st->nres = st->nres0;
-            st->rnorm = st->beta;
-            st->anorm2 = s0 + st->beta * 0.0;
-            st->reduce_b = s1;
-            st->iters = 0;
-            st->stop = 0;
-        }
-    }
 }
+
+struct FinishLsqrInit {
+    LsqrScalars* scal;
+    __device__ bool begin(int sys) const { return scal[sys].active && scal[sys].restart; }
+    __device__ void finish(int sys, double s0, double s1) const
+    {
+        LsqrScalars* st = &scal[sys];
+        const double alpha = sqrt(s0);
+        st->alpha = alpha;
+        st->rhobar = alpha;
+        st->phibar = st->beta;
+        st->nres0 = alpha * st->beta;
+        st->nres = st->nres0;
+        st->rnorm = st->beta;
+        st->anorm2 = s0 + st->beta * 0.0;
+        st->reduce_b = s1;
+        st->iters = 0;
+        st->stop = 0;
+    }
+};
 
 // v = vbar/alpha, vd = D v, w = v, y = 0.
 template <class VT>
@@ -2695,29 +2680,32 @@ __global__ void k_lsmr_init(int nsys, const LsqrScalars* scal, LsmrState* lsmr)
     ls->k_hb = ls->k_x = ls->k_h = 0.0;
 }
 
-// |z|^2 per system into reduce_b (used for |A^T b| and |A^T r|).
+// |z|^2 per system into reduce_b (used for |A^T b| and |A^T r|): the block
+// partials (slot 0; slot 1 is cleared), summed by FinishNorm2.
 template <class ZT>
 __global__ __launch_bounds__(kRowBlock) void k_cols_norm2(const ColWork* __restrict__ work, const ZT* __restrict__ z,
-                                                          GridSys g, LsqrScalars* scal)
+                                                          GridSys g, const LsqrScalars* scal)
 {
     __shared__ double sh[kRowBlock / 64];
     const ColWork w = work[blockIdx.x];
-    LsqrScalars* st = &scal[w.sys];
-    if (!st->active) return;
+    if (!scal[w.sys].active) return;
     double acc = 0.0;
     for (int64_t c = w.col_begin + threadIdx.x; c < w.col_end; c += kRowBlock) {
         const double zc = double(z[c]);
         acc += zc * zc;
     }
     acc = block_sum<kRowBlock>(acc, sh);
-    if (threadIdx.x == 0) g.partials[2 * blockIdx.x] = acc;
-    if (arrive_last(&g.counters[w.sys], g.blk_count[w.sys])) {
-        double s = 0.0;
-        for (int i = threadIdx.x; i < g.blk_count[w.sys]; i += kRowBlock) s += g.partials[2 * (g.blk_first[w.sys] + i)];
-        s = block_sum<kRowBlock>(s, sh);
-        if (threadIdx.x == 0) st->reduce_b = s;
+    if (threadIdx.x == 0) {
+        g.partials[2 * blockIdx.x] = acc;
+        g.partials[2 * blockIdx.x + 1] = 0.0;
     }
 }
+
+struct FinishNorm2 {
+    LsqrScalars* scal;
+    __device__ bool begin(int sys) const { return scal[sys].active; }
+    __device__ void finish(int sys, double s0, double) const { scal[sys].reduce_b = s0; }
+};
 
 // out = D y (the unscaled solution of a column-scaled LSQR).
 __global__ void k_scale_mul(const double* __restrict__ D, const double* __restrict__ y, int64_t n,
@@ -2797,11 +2785,10 @@ __global__ __launch_bounds__(kRowBlock) void k_pcg_update(const ColWork* __restr
 }
 
 // rz' (slot 0 of k_pcg_update's partials), rr (slot 1), beta = rz' / rz;
-// p = zz + beta p; q = 0 for the next scatter.
+// p = zz + beta p (k_pcg_reduce_q writes every column of q).
 template <class VT>
 __global__ __launch_bounds__(kRowBlock) void k_pcg_p(const ColWork* __restrict__ work, const VT* __restrict__ zz,
-                                                     VT* __restrict__ p, VT* __restrict__ q, GridSys g,
-                                                     PcgScalars* scal)
+                                                     VT* __restrict__ p, GridSys g, PcgScalars* scal)
 {
     __shared__ double sh[kRowBlock / 64];
     const ColWork w = work[blockIdx.x];
@@ -2819,21 +2806,19 @@ __global__ __launch_bounds__(kRowBlock) void k_pcg_p(const ColWork* __restrict__
     const VT b = VT(beta);
     for (int64_t c = w.col_begin + threadIdx.x; c < w.col_end; c += kRowBlock) {
         p[c] = zz[c] + b * p[c];
-        q[c] = VT(0);
     }
 }
 
-// PCG start: r = rhs (A^T b, x0 = 0), zz = P r, p = zz, rz = r.zz, q = 0.
+// PCG start: r = rhs (A^T b, x0 = 0), zz = P r, p = zz, the partials of
+// rz = r.zz and r.r (FinishPcgInit).
 template <class VT>
 __global__ __launch_bounds__(kRowBlock) void k_pcg_init(const ColWork* __restrict__ work, const VT* __restrict__ P,
-                                                        VT* __restrict__ rhs_r, VT* __restrict__ zz, VT* __restrict__ p,
-                                                        VT* __restrict__ x, VT* __restrict__ q, GridSys g,
-                                                        PcgScalars* scal)
+                                                        const VT* __restrict__ rhs_r, VT* __restrict__ zz, VT* __restrict__ p,
+                                                        VT* __restrict__ x, GridSys g, const PcgScalars* scal)
 {
     __shared__ double sh[kRowBlock / 64];
     const ColWork w = work[blockIdx.x];
-    PcgScalars* st = &scal[w.sys];
-    if (!st->active) return;
+    if (!scal[w.sys].active) return;
     double a0 = 0.0, a1 = 0.0;
     for (int64_t c = w.col_begin + threadIdx.x; c < w.col_end; c += kRowBlock) {
         const VT rc = rhs_r[c];
@@ -2841,7 +2826,6 @@ __global__ __launch_bounds__(kRowBlock) void k_pcg_init(const ColWork* __restric
         zz[c] = zc;
         p[c] = zc;
         x[c] = VT(0);
-        q[c] = VT(0);
         a0 += double(rc) * double(zc);
         a1 += double(rc) * double(rc);
     }
@@ -2851,21 +2835,18 @@ __global__ __launch_bounds__(kRowBlock) void k_pcg_init(const ColWork* __restric
         g.partials[2 * blockIdx.x] = a0;
         g.partials[2 * blockIdx.x + 1] = a1;
     }
-    if (arrive_last(&g.counters[w.sys], g.blk_count[w.sys])) {
-        double s0 = 0.0, s1 = 0.0;
-        for (int i = threadIdx.x; i < g.blk_count[w.sys]; i += kRowBlock) {
-            s0 += g.partials[2 * (g.blk_first[w.sys] + i)];
-            s1 += g.partials[2 * (g.blk_first[w.sys] + i) + 1];
-        }
-        s0 = block_sum<kRowBlock>(s0, sh);
-        s1 = block_sum<kRowBlock>(s1, sh);
-        if (threadIdx.x == 0) {
-            st->rz = s0;
-            st->rr = s1;
-            st->iters = 0;
-        }
-    }
 }
+
+struct FinishPcgInit {
+    PcgScalars* scal;
+    __device__ bool begin(int sys) const { return scal[sys].active; }
+    __device__ void finish(int sys, double s0, double s1) const
+    {
+        scal[sys].rz = s0;
+        scal[sys].rr = s1;
+        scal[sys].iters = 0;
+    }
+};
 
 // DiagonalPreconditioner (Math/Solver.h:29-34): non-normal entries become 1.
 template <class VT>

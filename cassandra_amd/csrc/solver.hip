@@ -487,6 +487,14 @@ static void column_scaling(cad_matrix* m, double* D, bool on, hipStream_t s)
     }
 }
 
+// The column blocks' partials of each system, summed and handed to f.
+template <class F>
+static void system_finish(cad_matrix* m, F f, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_system_finish<F>, dim3(unsigned(m->nsys)), dim3(kRowBlock), 0, s, f, m->grid.col_sys());
+    CAD_HIP(hipGetLastError());
+}
+
 // Explicit FP64 |A^T(b - A x)| and |b - A x| per system (one FP64 SpMV and one
 // FP64 scatter).  Uses its own scalar block so that solver state is untouched.
 static void explicit_residual(cad_matrix* m, Workspace& ws, const double* x, const double* b,
@@ -502,8 +510,8 @@ static void explicit_residual(cad_matrix* m, Workspace& ws, const double* x, con
     gather<double>(m, x, EpiResidual<double>{b, ws.r64.as<double>(), nullptr, sc}, s);
     scatter<double, double, double>(m, ws.r64.as<double>(), nullptr, ws.z64.as<double>(), s);
     hipLaunchKernelGGL(k_cols_norm2<double>, dim3(unsigned(g.cols.size())), dim3(kRowBlock), 0, s,
-                       g.d_cols.as<ColWork>(), ws.z64.as<double>(), g.col_sys(), sc);
-    CAD_HIP(hipGetLastError());
+                       g.d_cols.as<ColWork>(), ws.z64.as<double>(), g.col_sys(), (const LsqrScalars*)sc);
+    system_finish(m, FinishNorm2{sc}, s);
     const LsqrScalars* h = read_scalars<LsqrScalars>(m, ws, ws.scal_chk, s);
     nres.resize(m->nsys);
     rnorm.resize(m->nsys);
@@ -523,8 +531,9 @@ static std::vector<double> atb_norms(cad_matrix* m, Workspace& ws, const double*
     set_active(m, ws, ws.scal_chk, act, s);
     scatter<double, double, double>(m, b, nullptr, ws.z64.as<double>(), s);
     hipLaunchKernelGGL(k_cols_norm2<double>, dim3(unsigned(g.cols.size())), dim3(kRowBlock), 0, s,
-                       g.d_cols.as<ColWork>(), ws.z64.as<double>(), g.col_sys(), ws.scal_chk.as<LsqrScalars>());
-    CAD_HIP(hipGetLastError());
+                       g.d_cols.as<ColWork>(), ws.z64.as<double>(), g.col_sys(),
+                       (const LsqrScalars*)ws.scal_chk.as<LsqrScalars>());
+    system_finish(m, FinishNorm2{ws.scal_chk.as<LsqrScalars>()}, s);
     const LsqrScalars* h = read_scalars<LsqrScalars>(m, ws, ws.scal_chk, s);
     std::vector<double> out(m->nsys);
     for (int i = 0; i < m->nsys; i++) out[i] = std::sqrt(h[i].reduce_b);
@@ -726,7 +735,8 @@ static void lsqr_start_from_residual(cad_matrix* m, Workspace& ws, const double*
     scatter_restart<double, double, double>(m, ws.r64.as<double>(), sc, ws.z64.as<double>(), s);
     hipLaunchKernelGGL(k_lsqr_init_v<double>, dim3(unsigned(g.cols.size())), dim3(kRowBlock), 0, s,
                        g.d_cols.as<ColWork>(), ws.D.as<double>(), ws.z64.as<double>(), ws.v.as<double>(), g.col_sys(),
-                       sc);
+                       (const LsqrScalars*)sc);
+    system_finish(m, FinishLsqrInit{sc}, s);
     hipLaunchKernelGGL(k_lsqr_init_w<VT>, dim3(unsigned(g.cols.size())), dim3(kRowBlock), 0, s,
                        g.d_cols.as<ColWork>(), ws.D.as<double>(), ws.v.as<double>(), ws.vd.as<VT>(),
                        ws.w.as<double>(), ws.y.as<double>(), (const LsqrScalars*)sc);
@@ -1115,7 +1125,7 @@ static void pcg_iteration(cad_matrix* m, Workspace& ws, hipStream_t s)
                        g.d_cols.as<ColWork>(), ws.P.as<VT>(), ws.p.as<VT>(), ws.q.as<VT>(), ws.xr.as<VT>(),
                        ws.rr.as<VT>(), ws.zz.as<VT>(), L.reduce_sys(), g.col_sys(), sc);
     hipLaunchKernelGGL(k_pcg_p<VT>, dim3(unsigned(g.cols.size())), dim3(kRowBlock), 0, s, g.d_cols.as<ColWork>(),
-                       ws.zz.as<VT>(), ws.p.as<VT>(), ws.q.as<VT>(), g.col_sys(), sc);
+                       ws.zz.as<VT>(), ws.p.as<VT>(), g.col_sys(), sc);
     CAD_HIP(hipGetLastError());
 }
 
@@ -1154,9 +1164,9 @@ static void pcg_solve(cad_matrix* m, const double* b, double* x, const cad_solve
     // rhs = A^T b into rr (x0 = 0 so r = rhs)
     scatter<VT, VT, VT>(m, ws.bvt.as<VT>(), nullptr, ws.rr.as<VT>(), s);
     hipLaunchKernelGGL(k_pcg_init<VT>, dim3(unsigned(g.cols.size())), dim3(kRowBlock), 0, s, g.d_cols.as<ColWork>(),
-                       ws.P.as<VT>(), ws.rr.as<VT>(), ws.zz.as<VT>(), ws.p.as<VT>(), ws.xr.as<VT>(), ws.q.as<VT>(),
-                       g.col_sys(), ws.pscal.as<PcgScalars>());
-    CAD_HIP(hipGetLastError());
+                       ws.P.as<VT>(), (const VT*)ws.rr.as<VT>(), ws.zz.as<VT>(), ws.p.as<VT>(), ws.xr.as<VT>(), g.col_sys(),
+                       (const PcgScalars*)ws.pscal.as<PcgScalars>());
+    system_finish(m, FinishPcgInit{ws.pscal.as<PcgScalars>()}, s);
     const int batch = std::max(1, o.check_every);
     int it = 0;
     while (it < o.max_iterations) {
