@@ -341,8 +341,8 @@ void train_step(cad_patterns* p, const int32_t* idx, const float* target, const 
     int32_t* rows = p->d_train_rows.as<int32_t>();
     const AdamStep a{lr, b1, b2, eps, 1.0f - std::pow(b1, float(step)), std::sqrt(1.0f - std::pow(b2, float(step)))};
     if (B > 0) {
-        hipLaunchKernelGGL(pair_rows(idx, k) ? k_train_forward<2> : k_train_forward<1>, dim3(nblk), dim3(kRowBlock), 0,
-                           s, idx, sel, B, k, w, uint32_t(C), target, delta, g, part, rows);
+        hipLaunchKernelGGL(k_train_forward, dim3(nblk), dim3(kRowBlock), 0, s, idx, sel, B, k, w, uint32_t(C), target,
+                           delta, g, part, rows);
         // the backward's window tiles over the slot-major copy of the
         // minibatch's rows, then their column sums with the Adam update
         float* gpart = nullptr;

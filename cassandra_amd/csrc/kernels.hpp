@@ -2861,13 +2861,12 @@ __global__ void k_precond_from_jacobi(const float* __restrict__ jac, int64_t n, 
 // ------------------------------------------------------------ evaluator ----
 // sum_s w[idx[s]] of one row's k consecutive entries, in slot order from zero
 // (Pattern/Evaluator.cpp:48-54 sums the same terms in the same order; entries
-// outside [0, cols) add nothing), put(s, entry) for each of them.  A thread
-// takes a row: kGatherAhead entries and then their weights are loaded together
+// outside [0, cols) add nothing).  A thread takes a row: kGatherAhead entries and then their weights are loaded together
 // (V = 2: pairs, for an even k and rows aligned to 8 bytes).
 constexpr int kGatherAhead = 20;
-template <class VT, int V, class Put>
+template <class VT, int V>
 __device__ __forceinline__ VT row_gather(const int32_t* __restrict__ row, int k, const VT* __restrict__ w,
-                                         uint32_t cols, Put&& put)
+                                         uint32_t cols)
 {
     VT acc = VT(0);
     for (int s0 = 0; s0 < k; s0 += kGatherAhead) {
@@ -2888,10 +2887,7 @@ __device__ __forceinline__ VT row_gather(const int32_t* __restrict__ row, int k,
         for (int j = 0; j < kGatherAhead; j++) x[j] = w[min(uint32_t(c[j]), cols - 1)];
 #pragma unroll
         for (int j = 0; j < kGatherAhead; j++) {
-            if (s0 + j < k) {
-                acc = uint32_t(c[j]) < cols ? acc + x[j] : acc;
-                put(s0 + j, c[j]);
-            }
+            if (s0 + j < k) acc = uint32_t(c[j]) < cols ? acc + x[j] : acc;
         }
     }
     return acc;
@@ -2906,7 +2902,7 @@ __global__ __launch_bounds__(kRowBlock) void k_eval_forward(const int32_t* __res
 {
     const int64_t r = blockIdx.x * int64_t(kRowBlock) + threadIdx.x;
     if (r >= B) return;
-    out[r] = row_gather<VT, V>(idx + r * k, k, w, cols, [](int, int32_t) {});
+    out[r] = row_gather<VT, V>(idx + r * k, k, w, cols);
 }
 
 // The Huber loss of d = pred - target (0.5 d^2 inside [-delta, delta],
@@ -2923,9 +2919,15 @@ __device__ __forceinline__ double huber_term(float d, float delta, int64_t B, fl
 // the prediction (the evaluator's gather-sum, slot order from zero), the loss
 // and g[b] (huber_term); the block sums of the losses (FP64) go to
 // part[blockIdx.x], and the entries to rows[s * B + b] -- slot-major, so that
-// both these stores and the backward's loads are whole lines.  65,536 rows of
-// FIT4 out of 5M: 12.9 µs (16.5 with three pairs of entries at a time).
-template <int V>
+// both these stores and the backward's loads are whole lines.
+// A wave takes 64 rows, up to kTrainChunk slots at a time: its lanes load the
+// entries as they lie in memory (row after row, so that a load touches the
+// lines of a few rows and not of 64) into the wave's part of the LDS, from
+// which each lane takes its row.  65,536 rows of FIT4 out of 5M: 11.4 µs (12.2
+// with a lane loading its own row, 16.5 three pairs of entries at a time), with
+// one wave a SIMD the latency of its loads one after the other: the shuffled
+// order, the rows, the weights.
+constexpr int kTrainChunk = 32;
 __global__ __launch_bounds__(kRowBlock) void k_train_forward(const int32_t* __restrict__ idx,
                                                              const int64_t* __restrict__ sel, int64_t B, int k,
                                                              const float* __restrict__ w, uint32_t cols,
@@ -2933,17 +2935,60 @@ __global__ __launch_bounds__(kRowBlock) void k_train_forward(const int32_t* __re
                                                              float* __restrict__ g, double* __restrict__ part,
                                                              int32_t* __restrict__ rows)
 {
-    __shared__ double sh[kRowBlock / 64];
-    const int64_t b = blockIdx.x * int64_t(kRowBlock) + threadIdx.x;
+    constexpr int kWaves = kRowBlock / 64, kPitch = kTrainChunk + 1, kAhead = 16;
+    __shared__ double sh[kWaves];
+    __shared__ int64_t at[kWaves][64];            // first entry of each row
+    __shared__ int32_t ent[kWaves][64 * kPitch];  // entry (row, slot of the chunk)
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t b = blockIdx.x * int64_t(kRowBlock) + threadIdx.x, wave0 = b - lane;
     double loss = 0.0;
-    if (b < B) {
-        const int64_t r = sel[b];
+    if (wave0 < B) {
+        const int64_t r = sel[min(b, B - 1)];
         const float t = target[r];
+        at[wave][lane] = r * k;
         int32_t* __restrict__ dst = rows + b;
-        const float acc = row_gather<float, V>(idx + r * k, k, w, cols, [&](int s, int32_t c) { dst[s * B] = c; });
-        float gr;
-        loss = huber_term(acc - t, delta, B, gr);
-        g[b] = gr;
+        float acc = 0.0f;
+        for (int s0 = 0; s0 < k; s0 += kTrainChunk) {
+            const int nc = min(kTrainChunk, k - s0);
+            // e / nc for e < 64 nc, exact for nc <= 32
+            const uint32_t inv = (65536u + uint32_t(nc) - 1u) / uint32_t(nc);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            for (int i0 = 0; i0 < nc; i0 += kAhead) {
+                int32_t c[kAhead];
+                int place[kAhead];
+#pragma unroll
+                for (int i = 0; i < kAhead; i++) {
+                    const uint32_t e = uint32_t(lane + 64 * min(i0 + i, nc - 1));
+                    const uint32_t row = (e * inv) >> 16, s = e - row * uint32_t(nc);
+                    place[i] = int(row) * kPitch + int(s);
+                    c[i] = idx[at[wave][row] + s0 + int(s)];
+                }
+#pragma unroll
+                for (int i = 0; i < kAhead; i++) ent[wave][place[i]] = c[i];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            for (int j0 = 0; j0 < nc; j0 += kAhead) {
+                int32_t c[kAhead];
+                float x[kAhead];
+#pragma unroll
+                for (int j = 0; j < kAhead; j++) c[j] = ent[wave][lane * kPitch + min(j0 + j, nc - 1)];
+#pragma unroll
+                for (int j = 0; j < kAhead; j++) x[j] = w[min(uint32_t(c[j]), cols - 1)];
+#pragma unroll
+                for (int j = 0; j < kAhead; j++)
+                    if (j0 + j < nc) {
+                        acc = uint32_t(c[j]) < cols ? acc + x[j] : acc;
+                        if (b < B) dst[(s0 + j0 + j) * B] = c[j];
+                    }
+            }
+        }
+        if (b < B) {
+            float gr;
+            loss = huber_term(acc - t, delta, B, gr);
+            g[b] = gr;
+        }
     }
     loss = block_sum<kRowBlock>(loss, sh);
     if (threadIdx.x == 0) part[blockIdx.x] = loss;
