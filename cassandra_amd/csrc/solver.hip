@@ -1199,12 +1199,10 @@ static void pcg_solve(cad_matrix* m, const double* b, double* x, const cad_solve
     int it = 0;
     while (it < o.max_iterations) {
         const int n = std::min(batch, o.max_iterations - it);
-        // a graph is captured where it will be replayed: with two batches left,
-        // or once this workspace has run one (capturing and instantiating ten
-        // iterations takes longer than launching them once: FitWeights of
-        // 100,000 rows 1030 µs with it, 928 without)
-        const bool replayed = ws.exec != nullptr || ws.ran_batch || o.max_iterations - it >= 2 * batch;
-        ws.ran_batch = true;
+        // a graph is captured where it will be replayed: capturing and
+        // instantiating takes longer than launching once (FitWeights of 100,000
+        // rows, one batch of ten iterations: 1,030 µs with it, 928 without)
+        const bool replayed = ws.exec != nullptr || o.max_iterations - it >= 2 * batch;
         if (o.use_graph && batch > 1 && n == batch && s != nullptr && replayed) {
             // `batch` iterations captured once per workspace, replayed
             if (!ws.exec || ws.graph_iters != batch) {

@@ -37,7 +37,6 @@ struct Workspace {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     int graph_iters = 0, graph_prec = 0;
-    bool ran_batch = false;   // PCG: a batch of iterations has been launched with these buffers
     int graph_gen = -1;       // ActiveLists generation the graph was captured with (-1: full lists)
     ActiveLists active;
     bool use_active = false;  // iterations launch the active lists
