@@ -456,7 +456,7 @@ def leg_evaluator(ctx):
     bwd_ms = event_time_ms(ctx, lambda: L.cad_eval_backward_f32(P.h, hp(sub), B, hp(g), hp(grad)), reps)
     bwd_na_ms = event_time_ms(ctx, lambda: L.cad_eval_backward_f32_noalloc(P.h, hp(sub), B, hp(g), hp(grad)), reps)
     nbytes = B * (4 * P.k + 4) + 4 * P.cols
-    # the resident evaluator (expanded tables kept on the device): positions
+    # the resident evaluator (weights kept on the device): positions
     # in, scores out -- on device positions, and host batches with the copies
     E = P.evaluator(w)
     pos_b = pos[:B].contiguous()

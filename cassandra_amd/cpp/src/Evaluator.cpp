@@ -69,8 +69,7 @@ std::vector<float> ScoreEstimator::Weights() const
     return out;
 }
 
-// The pattern group and the expanded tables of one ScoreEstimator on the
-// device; calls on one estimator take turns (its staging buffers are shared).
+// The pattern group and the weights of one ScoreEstimator on the device; calls on one estimator take turns (its staging buffers are shared).
 struct ScoreEstimatorDevice {
     std::mutex mu;
     cad_patterns* patterns = nullptr;

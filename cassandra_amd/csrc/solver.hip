@@ -1201,7 +1201,7 @@ static void pcg_solve(cad_matrix* m, const double* b, double* x, const cad_solve
         const int n = std::min(batch, o.max_iterations - it);
         // a graph is captured where it will be replayed: capturing and
         // instantiating takes longer than launching once (FitWeights of 100,000
-        // rows, one batch of ten iterations: 1,030 µs with it, 928 without)
+        // rows, one batch of ten iterations: 1,030 µs with it, 840 without)
         const bool replayed = ws.exec != nullptr || o.max_iterations - it >= 2 * batch;
         if (o.use_graph && batch > 1 && n == batch && s != nullptr && replayed) {
             // `batch` iterations captured once per workspace, replayed

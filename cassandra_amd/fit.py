@@ -197,7 +197,7 @@ class Patterns:
 
 
 class Evaluator:
-    """A resident evaluator: the expanded tables of one weight vector kept on
+    """A resident evaluator: one weight vector kept on
     the device (ScoreEstimator::Eval for batches of positions)."""
 
     def __init__(self, patterns: Patterns, w: torch.Tensor):

@@ -297,17 +297,18 @@ int cad_weights_compact(cad_patterns* p, const float* d_tables, float* d_w);
 /* ---- resident evaluator (ScoreEstimator::Eval, Pattern/Evaluator.cpp:48-54;
  * the batched form of the leaf evaluations of
  * Search/PrincipalVariation.cpp:224-229) --------------------------------------
- * Holds the expanded tables of one compact weight vector in device memory,
+ * Holds one compact weight vector in device memory (all variations of a pattern
+ * read the same columns, so it needs no expanded tables),
  * so that batches of positions are scored without re-uploading anything.
  * Every score is the float sum over the variations in order from 0, the same
  * bits as ScoreEstimator::Eval.  The pattern group must outlive it. */
 int cad_evaluator_create(cad_patterns* p, const float* d_w, cad_evaluator** out);
 int cad_evaluator_destroy(cad_evaluator* e);
-/* New compact weights (d_w: cols floats), expanded on the device. */
+/* New compact weights (d_w: cols floats), copied on the device. */
 int cad_evaluator_set_weights(cad_evaluator* e, const float* d_w);
 /* d_out[r] = Eval(position r) for n device positions (enqueued on the stream). */
 int cad_evaluator_eval(cad_evaluator* e, const uint64_t* d_positions, int64_t n, float* d_out);
-/* The same for host positions and scores (staged through buffers the
+/* The same for host positions and scores (through buffers, pinned for small batches, that the
  * evaluator keeps; synchronises the stream). */
 int cad_evaluator_eval_host(cad_evaluator* e, const uint64_t* h_positions, int64_t n, float* h_out);
 
