@@ -1850,6 +1850,7 @@ __device__ __forceinline__ void store_window(const double* __restrict__ win, uin
 // max |VT(y)| as float bits (non-negative floats order as unsigned integers;
 // NaN and inf above every finite value), the ymax of FixedScale, in two
 // launches without atomics: one value per row block, then one per system.
+// 5M rows: 7.1 µs, 10.5 with one row a thread at a time.
 template <class YT>
 __global__ __launch_bounds__(kRowBlock) void k_absmax_blocks(const RowWork* __restrict__ work,
                                                              const YT* __restrict__ y, unsigned* __restrict__ part)
@@ -1857,8 +1858,14 @@ __global__ __launch_bounds__(kRowBlock) void k_absmax_blocks(const RowWork* __re
     __shared__ unsigned sh[kRowBlock / 64];
     const RowWork w = work[blockIdx.x];
     unsigned mb = 0;
-    for (int64_t r = w.row_begin + threadIdx.x; r < w.row_end; r += kRowBlock)
-        mb = max(mb, __float_as_uint(fabsf(float(y[r]))));
+    // four rows a thread in flight (the last row again past the end)
+    for (int64_t r = w.row_begin + threadIdx.x; r < w.row_end; r += 4 * kRowBlock) {
+        YT t[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) t[i] = y[min(r + i * kRowBlock, w.row_end - 1)];
+#pragma unroll
+        for (int i = 0; i < 4; i++) mb = max(mb, __float_as_uint(fabsf(float(t[i]))));
+    }
     for (int o = 32; o > 0; o >>= 1) mb = max(mb, unsigned(__shfl_xor(int(mb), o, 64)));
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = mb;
     __syncthreads();
@@ -1876,7 +1883,16 @@ __global__ __launch_bounds__(kRowBlock) void k_absmax_systems(const int32_t* __r
     __shared__ unsigned sh[kRowBlock / 64];
     const int s = blockIdx.x;
     unsigned mb = 0;
-    for (int i = threadIdx.x; i < count[s]; i += kRowBlock) mb = max(mb, part[first[s] + i]);
+    const int n = count[s];
+    const unsigned* __restrict__ p = part + first[s];
+    // eight in flight (the last again past the end): 20M rows took 19 µs with one
+    for (int i = threadIdx.x; i < n; i += 8 * kRowBlock) {
+        unsigned v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = p[min(i + j * kRowBlock, n - 1)];
+#pragma unroll
+        for (int j = 0; j < 8; j++) mb = max(mb, v[j]);
+    }
     for (int o = 32; o > 0; o >>= 1) mb = max(mb, unsigned(__shfl_xor(int(mb), o, 64)));
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = mb;
     __syncthreads();
