@@ -365,6 +365,11 @@ const EvalPlan& eval_weights_plan(cad_patterns* p)
     if (slot != g.k()) throw Error(CAD_ERR_PATTERN, "variation count differs from the slot count");
     E->nsegs = int(segs.size());
     E->lds = size_t(used) * sizeof(float);
+    // the kernels' LDS limit is set here, so that a launch is all a batch needs
+    // (also while a stream is captured); the same limit for every pattern group
+    for (auto kern : {k_eval_staged<1>, k_eval_staged<2>})
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  int(room * sizeof(float)));
     hipStream_t s = p->ctx->stream;
     E->d_segs = to_device(segs, s);
     E->d_tile_lds = to_device(tile_lds, s);
@@ -385,9 +390,6 @@ void eval_weights(cad_patterns* p, const float* w, const uint64_t* pos, int64_t 
     } else if (E.nsegs > 0 && n >= kEvalStagedRows * p->ctx->cus) {
         const int C = n <= int64_t(p->ctx->cus) * kEvalBlock ? 1 : 2;
         auto kern = C == 1 ? k_eval_staged<1> : k_eval_staged<2>;
-        if (E.lds > 64 * 1024)
-            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      int(E.lds));
         const int64_t blocks = std::min<int64_t>(p->ctx->cus, (n + kEvalBlock * C - 1) / (kEvalBlock * C));
         hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(kEvalBlock), E.lds, s, pos, n, tv,
                            E.d_tile_lds.as<int32_t>(), E.d_segs.as<PhaseSeg>(), E.nsegs, w, cols, out);
