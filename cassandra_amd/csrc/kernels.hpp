@@ -2150,23 +2150,24 @@ __global__ __launch_bounds__(kScatterBlock) void k_scatter_tile(SlotMajor<IdxT> 
 // Stage 1 for a matrix-free matrix: as k_scatter_tile, with every slot's column
 // computed by its index tile.  A wave takes RPT runs of 64 rows a step; the
 // columns turn from one slot per 16-lane group to one row per lane.  A group's
-// slots are runs of whole patterns, so its tiles follow each other.  FP32
-// windows accumulate in fixed point as k_scatter_tile's do.  20M rows of
-// FIT12: 1,430 µs (2,537 with the lists evaluated digit by digit into FP64
-// windows), bound by vector issue: a tile of a 32-slot group takes 395 cycles
-// of a SIMD per 64 rows, about 75 instructions.
-template <class VT, class YT, int RPT, bool kBeta = false, bool kYmax = false>
+// slots are runs of whole patterns, so its tiles follow each other.  The windows
+// are FP64 whatever VT is: the terms of up to 32 slots and a million rows meet
+// in one window, and a fixed-point word with room for that many terms resolves
+// no more than 2^-39 of max |y|.  20M rows of FIT12: 1,745 µs (2,570 with the
+// lists evaluated digit by digit); a window of 32 slots takes 1,099 cycles per
+// 64 rows, where fixed point, whose adds are faster, took 790.
+template <class VT, class YT, int RPT, bool kBeta = false>
 __global__ __launch_bounds__(kScatterBlock) void k_scatter_tile_mf(PositionsView m,
                                                                    const ScatterWork* __restrict__ work,
                                                                    const SlotGroup* __restrict__ groups,
                                                                    const uint16_t* __restrict__ slot_list,
                                                                    const uint32_t* __restrict__ sys_col,
                                                                    const YT* __restrict__ y, LsqrScalars* div,
-                                                                   int mode, FixedScale fx, int y_padded,
+                                                                   int mode, FixedScale, int,
                                                                    VT* __restrict__ part, GridSys bsum)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    double* win = reinterpret_cast<double*>(smem_raw);  // 8-byte window words (FP64 or fixed point)
+    double* win = reinterpret_cast<double*>(smem_raw);
     const ScatterWork w = uniform_load(work + blockIdx.x);
     if (!scatter_selected(div, mode, w.sys)) return;
     const uint32_t W = w.win_hi - w.win_lo;
@@ -2175,89 +2176,76 @@ __global__ __launch_bounds__(kScatterBlock) void k_scatter_tile_mf(PositionsView
     const SlotGroup gr = uniform_load(groups + w.group);
     const uint32_t cb = sys_col[w.sys];
     const VT sc = scatter_scale<VT, kScatterBlock, kBeta>(div, mode, w.sys, bsum);
-    const double fscale = window_scale<VT, kScatterBlock, kYmax>(fx, w.sys, sc);
     // the group's tiles: ntile of them, gr.nslots slots in all
     const int first = uniform_u16(slot_list, gr.first);
     const int tile0 = m.slot_tile(first), ntile = m.slot_tile(first + gr.nslots - 1) - tile0 + 1;
     const int lane = threadIdx.x & 63;
-    auto rows = [&](auto* wn) {
-        using WT = std::remove_pointer_t<decltype(wn)>;
-        // Run c of a step: the wave's rows a + c kScatterBlock + [0, 64).  The
-        // next step's words and y load while this one is added.
-        uint32_t tn[RPT][4];
-        YT yn[RPT];
-        auto load = [&](int64_t a) {
-            const uint32_t* __restrict__ tw = reinterpret_cast<const uint32_t*>(m.tw + a);
-            const YT* __restrict__ ya = y + a;
-            const int last = int(min<int64_t>(w.row_end - a, int64_t(RPT) * kScatterBlock)) - 1;
-            if (last >= (RPT - 1) * kScatterBlock + 63) {
-#pragma unroll
-                for (int c = 0; c < RPT; c++) {
-#pragma unroll
-                    for (int p = 0; p < 4; p++)
-                        tn[c][p] = tw[uint32_t(4 * (lane & 15) + (lane >> 4)) + uint32_t(4 * (c * kScatterBlock + 16 * p))];
-                    yn[c] = ya[uint32_t(lane) + uint32_t(c * kScatterBlock)];
-                }
-            } else {
-#pragma unroll
-                for (int c = 0; c < RPT; c++) {
-#pragma unroll
-                    for (int p = 0; p < 4; p++)
-                        tn[c][p] = tw[4 * min(c * kScatterBlock + 16 * p + (lane & 15), last) + (lane >> 4)];
-                    yn[c] = ya[min(c * kScatterBlock + lane, last)];
-                }
-            }
-        };
-        // (the wave's rows through scalar registers: its addresses are a
-        // scalar base and one offset)
-        int64_t a = w.row_begin + __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u);
-        if (a >= w.row_end) return;
-        load(a);
-        TileRegs tr = load_tile(m.tiles, tile0);
-        int at = 0;
-        for (; a < w.row_end; a += RPT * kScatterBlock) {
-            Int4 b[RPT][4];
-            WT yv[RPT];
-            bool ok[RPT];
+    // Run c of a step: the wave's rows a + c kScatterBlock + [0, 64).  The
+    // next step's words and y load while this one is added.
+    uint32_t tn[RPT][4];
+    YT yn[RPT];
+    auto load = [&](int64_t a) {
+        const uint32_t* __restrict__ tw = reinterpret_cast<const uint32_t*>(m.tw + a);
+        const YT* __restrict__ ya = y + a;
+        const int last = int(min<int64_t>(w.row_end - a, int64_t(RPT) * kScatterBlock)) - 1;
+        if (last >= (RPT - 1) * kScatterBlock + 63) {
 #pragma unroll
             for (int c = 0; c < RPT; c++) {
 #pragma unroll
-                for (int p = 0; p < 4; p++) b[c][p] = expand_digits(tn[c][p]);
-                ok[c] = a + c * kScatterBlock + lane < w.row_end;
-                yv[c] = window_term<WT>(double(VT(yn[c]) * sc), fscale);
+                for (int p = 0; p < 4; p++)
+                    tn[c][p] = tw[uint32_t(4 * (lane & 15) + (lane >> 4)) + uint32_t(4 * (c * kScatterBlock + 16 * p))];
+                yn[c] = ya[uint32_t(lane) + uint32_t(c * kScatterBlock)];
             }
-            if (a + RPT * kScatterBlock < w.row_end) load(a + RPT * kScatterBlock);
-            for (int t = 0; t < ntile; t++) {
-                const IndexTile tl = tr.tile();
-                const Int4 wt = tr.weights;
-                const int number = tile0 + at;
-                at = at + 1 < ntile ? at + 1 : 0;
-                tr = load_tile(m.tiles, tile0 + at);
-                const uint32_t off = cb + tl.col_offset - w.win_lo;
+        } else {
 #pragma unroll
-                for (int c = 0; c < RPT; c++) {
-                    uint32_t ci[4];
-                    tile_columns(tl, number, m.tiles, wt, b[c], ci);
-                    transpose_groups(ci);
+            for (int c = 0; c < RPT; c++) {
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const uint32_t uc = off + ci[j];
-                        if (j < tl.nslots && ok[c] && uc < W) atomicAdd(&wn[uc], yv[c]);
-                    }
-                }
+                for (int p = 0; p < 4; p++)
+                    tn[c][p] = tw[4 * min(c * kScatterBlock + 16 * p + (lane & 15), last) + (lane >> 4)];
+                yn[c] = ya[min(c * kScatterBlock + lane, last)];
             }
         }
     };
-    if constexpr (std::is_same_v<VT, float>) {
-        if (fscale > 0.0)
-            rows(reinterpret_cast<unsigned long long*>(win));
-        else
-            rows(win);
-    } else {
-        rows(win);
+    // (the wave's rows through scalar registers: its addresses are a
+    // scalar base and one offset)
+    int64_t a = w.row_begin + __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u);
+    if (a < w.row_end) load(a);
+    TileRegs tr = load_tile(m.tiles, tile0);
+    int at = 0;
+    for (; a < w.row_end; a += RPT * kScatterBlock) {
+        Int4 b[RPT][4];
+        double yv[RPT];
+        bool ok[RPT];
+#pragma unroll
+        for (int c = 0; c < RPT; c++) {
+#pragma unroll
+            for (int p = 0; p < 4; p++) b[c][p] = expand_digits(tn[c][p]);
+            ok[c] = a + c * kScatterBlock + lane < w.row_end;
+            yv[c] = double(VT(yn[c]) * sc);
+        }
+        if (a + RPT * kScatterBlock < w.row_end) load(a + RPT * kScatterBlock);
+        for (int t = 0; t < ntile; t++) {
+            const IndexTile tl = tr.tile();
+            const Int4 wt = tr.weights;
+            const int number = tile0 + at;
+            at = at + 1 < ntile ? at + 1 : 0;
+            tr = load_tile(m.tiles, tile0 + at);
+            const uint32_t off = cb + tl.col_offset - w.win_lo;
+#pragma unroll
+            for (int c = 0; c < RPT; c++) {
+                uint32_t ci[4];
+                tile_columns(tl, number, m.tiles, wt, b[c], ci);
+                transpose_groups(ci);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const uint32_t uc = off + ci[j];
+                    if (j < tl.nslots && ok[c] && uc < W) atomicAdd(&win[uc], yv[c]);
+                }
+            }
+        }
     }
     __syncthreads();
-    store_window<VT>(win, W, fscale, part + w.part_off);
+    store_window<VT>(win, W, 0.0, part + w.part_off);
 }
 
 // Stage 2: z[c] = sum of the window's chunk slices, in chunk order

@@ -188,11 +188,13 @@ struct TuneParams {
 // expanded once for all of them.
 constexpr int kPackSlotsMf = 32;
 
-// Time of a matrix-free scatter window per row, in units of one slot: a group
-// of 32 slots took 24.7 cycles per 64 rows and slot, one of 8 slots 29, of 4
-// slots 44, and one with two slots of dense tables (a lookup each) 48 for 6.
-// With windows weighed by their slots alone the longest tile took 4.68 million
-// cycles and the mean 3.05 (20M rows of FIT12).
+// Time of a matrix-free scatter window per row, in units of one slot.  Measured
+// (cycles per 64 rows): 4 slots 170 to 181, 8 slots 230 to 248 with a third of
+// their entries in the window, 6 slots with two of dense tables (a lookup each)
+// 304, 18 with two 683; 32 slots, all their entries in the window, 1,099, which
+// these weights take for 880: the longest tile is 1.23 of the mean (20M rows of
+// FIT12; 1.53 with the slots alone for weights).  Weighing the entries too made
+// FP32 2 % faster and FP64 4 % slower.
 constexpr double kMfRowCost = 3.5, kMfDenseCost = 2.5;
 
 // A matrix (or, in a batch, the systems still iterating) of at most this many

@@ -97,7 +97,7 @@ void with_scatter_kernel(int rpt, bool beta, bool ymax, F&& f)
         } else if constexpr (std::is_same_v<View, SlotMajor<uint32_t>>) {
             return f(k_scatter_tile<VT, YT, uint32_t, 4, B, Y>);
         } else {
-            return f(k_scatter_tile_mf<VT, YT, 2, B, Y>);
+            return f(k_scatter_tile_mf<VT, YT, 2, B>);
         }
     };
     if (beta) return pick(std::true_type{}, std::false_type{});
@@ -112,8 +112,7 @@ template <class VT, class View>
 constexpr bool fixed_point_scatter()
 {
     return std::is_same_v<VT, float> &&
-           (std::is_same_v<View, SlotMajor<uint16_t>> || std::is_same_v<View, SlotMajor<uint32_t>> ||
-            std::is_same_v<View, PositionsView>);
+           (std::is_same_v<View, SlotMajor<uint16_t>> || std::is_same_v<View, SlotMajor<uint32_t>>);
 }
 
 template <class YT>
@@ -178,14 +177,12 @@ void launch_scatter(ScatterPlan& sp, const View& view, int rpt, const uint32_t* 
                     const LsqrScalars* div, int mode, ZT* z, const GridPlan& g, int nsys, hipStream_t s,
                     bool y_padded = false)
 {
-    // a stored matrix's window tiles take the row blocks' maxima themselves, a
+    // the fixed-point window tiles take the row blocks' maxima themselves, a
     // launch less (A x and A^T y of 5M rows of FIT8 279 -> 274 µs, of 50,001
-    // rows of FIT4 57.7 -> 55.5); the matrix-free tiles have no registers to
-    // spare for it
+    // rows of FIT4 57.7 -> 55.5)
     if (fixed_point_scatter<VT, View>() && mode != kScatterLsqr && !lists<VT>(sp).work.empty())
-        launch_absmax(sp, y, g, nsys, s, std::is_same_v<View, PositionsView>);
-    launch_scatter_tiles<VT, YT>(sp, view, rpt, sys_col, y, div, mode, s, y_padded, nullptr, GridSys{},
-                                 std::is_same_v<View, PositionsView> ? nullptr : &g);
+        launch_absmax(sp, y, g, nsys, s, false);
+    launch_scatter_tiles<VT, YT>(sp, view, rpt, sys_col, y, div, mode, s, y_padded, nullptr, GridSys{}, &g);
     launch_scatter_reduce<VT>(sp, div, mode, z, s);
 }
 
