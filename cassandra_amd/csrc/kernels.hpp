@@ -2252,9 +2252,13 @@ __global__ __launch_bounds__(kScatterBlock) void k_scatter_tile_mf(PositionsView
 // (the order of the slices is fixed; the sums inside a slice took the LDS
 // atomics' arrival order); columns outside every window get 0.
 // Column c's sum over the slices of its window: integer counts stay
-// integer; real sums add up in FP64, in chunk order, sixteen slices
+// integer; real sums add up in FP64, in chunk order, up to sixteen slices
 // loaded ahead of their additions (a load's latency, not the bytes, is what a
-// column of 20 to 60 slices waits for).
+// column of 20 to 60 slices waits for).  Whole sixteens, then the smallest step
+// that holds the rest: a batch's columns have one slice or a few, and sixteen
+// loads (with a 64-bit multiply each for the address) for those took 17.8 µs
+// where one takes 7.3 (30 systems of 102,222 columns); 100,000 rows, 25 to 38
+// slices a column, 4.5 -> 2.7, 1M rows 5.0 -> 3.3.
 template <class T>
 __device__ __forceinline__ std::conditional_t<std::is_integral_v<T>, T, double>
 reduce_column(const T* __restrict__ part, const ReduceWork& w, int64_t c)
@@ -2262,15 +2266,27 @@ reduce_column(const T* __restrict__ part, const ReduceWork& w, int64_t c)
     using AccT = std::conditional_t<std::is_integral_v<T>, T, double>;
     const T* __restrict__ p = part + w.part_off + (c - w.col_begin);
     AccT s = AccT(0);
-    constexpr int kAhead = 16;
-    for (int j = 0; j < w.nchunk; j += kAhead) {
+    int left = w.nchunk;
+    if (left == 1) return s + AccT(*p);
+    // the next `ahead` slices (the last one again past the end)
+    auto step = [&](auto ahead, auto whole) {
+        constexpr int kAhead = decltype(ahead)::value;
         T t[kAhead];
 #pragma unroll
-        for (int q = 0; q < kAhead; q++) t[q] = p[int64_t(min(j + q, w.nchunk - 1)) * w.stride];
+        for (int q = 0; q < kAhead; q++) {
+            t[q] = *p;
+            if (decltype(whole)::value || q + 1 < left) p += w.stride;
+        }
 #pragma unroll
         for (int q = 0; q < kAhead; q++)
-            if (j + q < w.nchunk) s += AccT(t[q]);
-    }
+            if (decltype(whole)::value || q < left) s += AccT(t[q]);
+        left -= kAhead;
+    };
+    while (left >= 16) step(std::integral_constant<int, 16>{}, std::true_type{});
+    if (left > 8) step(std::integral_constant<int, 16>{}, std::false_type{});
+    else if (left > 4) step(std::integral_constant<int, 8>{}, std::false_type{});
+    else if (left > 2) step(std::integral_constant<int, 4>{}, std::false_type{});
+    else if (left > 0) step(std::integral_constant<int, 2>{}, std::false_type{});
     return s;
 }
 
