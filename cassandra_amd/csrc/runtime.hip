@@ -339,13 +339,16 @@ void make_scatter_lists_xcd(const ScatterPlan& sp, const std::vector<int64_t>& s
 // Scatter tiles of (system rows) x (group window): every window of a system
 // gets row chunks by its time (win_cost), so that the tiles -- about target of
 // them -- take equally long; a window's chunks are limited by its partial
-// slices (written and read once): partial_cap of its index traffic, or the
-// floor bytes a window where that leaves CUs idle -- small_floor (8 MB by
-// default) for a small system (at most kRowKernelRows rows, whose tiles are
-// latency-bound: a 100k-row PCG iteration 47 -> 42 µs), 2 MB for a large one --
-// and to kScatterBlock rows.  Rounding each window's share by itself, and the
-// floor, made 263 tiles for 256 CUs at 5M rows of FIT8: seven in a second wave,
-// 197 µs where 256 take 127.
+// slices (written and read once): partial_cap of its index traffic, or, where
+// every window could be cut in two and until there are as many tiles as CUs,
+// the floor bytes a window -- small_floor (8 MB by default) for a small system
+// (at most kRowKernelRows rows, whose tiles are latency-bound: a 100k-row PCG
+// iteration 47 -> 42 µs), 2 MB for a large one -- and to kScatterBlock rows.
+// Rounding each window's share by itself, and the floor, made 263 tiles for 256
+// CUs at 5M rows of FIT8: seven in a second wave, 197 µs where 256 take 127.
+// The floor for a batch whose windows fill the CUs by themselves left mostly
+// slices to write and sum: 100 iterations of FP64 PCG over 50 systems 28.9 ms
+// against 19.5, the mixed fit of the 50 336 against 317.
 void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_rows,
                         const std::vector<uint32_t>& sys_col, int64_t cols_per_sys, uint32_t wmax, int vbytes,
                         int ibytes, int cus, const TuneParams& tune, bool fp32, ScatterLists& L,
@@ -394,11 +397,13 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
     struct Win {
         uint32_t lo, hi;
         int s, group;
-        int64_t rows, chunks, most;
+        int64_t rows, chunks, cap, most;  // most: the limit while CUs are idle
         double time;
     };
     std::vector<Win> wins;
     double total = 0;
+    const double wave = std::max(cus, 1);
+    const bool idle = 2.0 * windows * nrun <= wave;  // every window could be cut in two
     for (int s = 0; s < nsys; s++) {
         if (!in(s)) continue;
         const int64_t R = sys_rows[s + 1] - sys_rows[s];
@@ -409,35 +414,45 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
                 const double slice = 2.0 * double(W) * vbytes;
                 const double cap = tune.partial_cap * double(R) * g.nslots * ibytes / slice;
                 const double floor_c = (R <= kRowKernelRows ? tune.small_floor_bytes : kPartialFloorBytes) / slice;
-                Win w{wl, wh, s, int(gi), R, 0, 0, double(R) * win_cost(g, W)};
-                w.most = std::max<int64_t>(1, std::min<int64_t>(int64_t(std::max(cap, floor_c)),
-                                                                (R + kScatterBlock - 1) / kScatterBlock));
+                auto limit = [&](double c) {
+                    return std::max<int64_t>(1, std::min<int64_t>(int64_t(c), (R + kScatterBlock - 1) / kScatterBlock));
+                };
+                Win w{wl, wh, s, int(gi), R, 0, limit(cap), 0, double(R) * win_cost(g, W)};
+                w.most = idle ? std::max(w.cap, limit(floor_c)) : w.cap;
                 total += w.time;
                 wins.push_back(w);
             }
         }
     }
-    // whole shares, then one chunk more wherever the tiles are longest
+    // whole shares, then one chunk more wherever the tiles are longest; tiles
+    // of one wave last as long as their longest, so that nothing is gained by
+    // more once that one cannot be cut
+    const double share0 = idle ? std::min(target, wave) : target;
     int64_t tiles = 0;
+    double stuck = 0;  // the longest tile of a window at its limit
     std::vector<std::pair<double, size_t>> longest;  // a heap by tile time
     for (size_t i = 0; i < wins.size(); i++) {
         Win& w = wins[i];
         if (w.rows <= 0) continue;
-        w.chunks = std::max<int64_t>(1, std::min<int64_t>(w.most, int64_t(target * w.time / total)));
+        w.chunks = std::max<int64_t>(1, std::min<int64_t>(w.most, int64_t(share0 * w.time / total)));
         tiles += w.chunks;
-        if (w.chunks < w.most) longest.push_back({w.time / double(w.chunks), i});
+        longest.push_back({w.time / double(w.chunks), i});
     }
     std::make_heap(longest.begin(), longest.end());
     while (tiles < int64_t(target) && !longest.empty()) {
         std::pop_heap(longest.begin(), longest.end());
+        const double time = longest.back().first;
         Win& w = wins[longest.back().second];
         longest.pop_back();
+        if (target <= wave && time <= stuck) break;
+        if (w.chunks >= (double(tiles) < wave ? w.most : w.cap)) {
+            stuck = std::max(stuck, time);
+            continue;
+        }
         w.chunks++;
         tiles++;
-        if (w.chunks < w.most) {
-            longest.push_back({w.time / double(w.chunks), size_t(&w - wins.data())});
-            std::push_heap(longest.begin(), longest.end());
-        }
+        longest.push_back({w.time / double(w.chunks), size_t(&w - wins.data())});
+        std::push_heap(longest.begin(), longest.end());
     }
     size_t at = 0;
     for (int s = 0; s < nsys; s++) {
