@@ -138,6 +138,9 @@ int64_t window_chunks(int64_t R, double share_chunks, double cap_chunks, int cus
     return std::max<int64_t>(1, std::min<int64_t>(C, (R + kScatterBlock - 1) / kScatterBlock));
 }
 
+// Slots of fewer columns than this take longer the fewer they are (win_cost).
+constexpr double kNarrowSlot = 1024;
+
 // Group slots whose column ranges overlap (transitively).
 void make_groups(const std::vector<uint32_t>& lo, const std::vector<uint32_t>& hi, ScatterPlan& sp)
 {
@@ -147,6 +150,7 @@ void make_groups(const std::vector<uint32_t>& lo, const std::vector<uint32_t>& h
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return lo[a] < lo[b]; });
     sp.groups.clear();
     sp.slot_list.clear();
+    sp.narrow.assign(size_t(k), 0.0);
     int i = 0;
     while (i < k) {
         uint32_t glo = lo[order[i]], ghi = hi[order[i]];
@@ -156,7 +160,11 @@ void make_groups(const std::vector<uint32_t>& lo, const std::vector<uint32_t>& h
             j++;
         }
         std::vector<uint16_t> members;
-        for (int t = i; t < j; t++) members.push_back(uint16_t(order[t]));
+        for (int t = i; t < j; t++) {
+            members.push_back(uint16_t(order[t]));
+            const uint32_t width = std::max<uint32_t>(1, hi[order[t]] - lo[order[t]]);
+            sp.narrow[size_t(order[t])] = std::max(0.0, std::log2(kNarrowSlot / width));
+        }
         std::sort(members.begin(), members.end());  // keep slot order inside a group
         SlotGroup g;
         g.col_lo = glo;
@@ -363,7 +371,10 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
     // Time of a window per row, in units of one slot's loads.  Measured (cycles
     // a tile per 64 rows): FP32 windows take 32 for the row and 7.8 + 2 f a
     // slot, f the window's share of the group's columns (66 to 111 for 4 to 8
-    // slots), FP64 ones 18 and 6 + 17.5 f (62 to 206: their adds are slower).
+    // slots), FP64 ones 18 and 6 + 17.5 f (62 to 206: their adds are slower).  A
+    // slot of few columns adds to the same ones over and over: 4 slots of 1,134
+    // columns take 74 (FP64 116), 8 of 378 and 1,134 165 (272), 8 of 45 and 135
+    // columns 205 (318), where 8 wide ones take 145 (245) of the same rows.
     // Other values of scatter_balance weigh the slot loads (1: loads only)
     // against the entries that fall into the window.  Matrix-free: a slot's
     // columns are computed whether or not they fall into the window
@@ -376,7 +387,12 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
             return c;
         }
         const double frac = double(W) / double(std::max<uint32_t>(1, g.col_hi - g.col_lo));
-        if (lam == 1.0 && vbytes == 8) return fp32 ? 4.1 + g.nslots * (1.0 + 0.26 * frac) : 3.0 + g.nslots * (1.0 + 2.9 * frac);
+        if (lam == 1.0 && vbytes == 8) {
+            double narrow = 0;
+            for (int j = 0; j < g.nslots; j++) narrow += sp.narrow[L.slot_list[size_t(g.first + j)]];
+            return fp32 ? 4.1 + g.nslots * (1.0 + 0.26 * frac) + 0.32 * narrow
+                        : 3.0 + g.nslots * (1.0 + 2.9 * frac) + 0.45 * narrow;
+        }
         return g.nslots * (lam + (1.0 - lam) * frac);
     };
     int nrun = 0;  // systems planned here that have rows: their windows run side by side
@@ -424,9 +440,10 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
             }
         }
     }
-    // whole shares, then one chunk more wherever the tiles are longest; tiles
-    // of one wave last as long as their longest, so that nothing is gained by
-    // more once that one cannot be cut
+    // whole shares, then one chunk more wherever the tiles are longest: in one
+    // wave until those cannot be cut (more of the shorter ones gain nothing), in
+    // several until they are a quarter of those (the Jacobi counts of 500,000
+    // rows of 46 slots 33 -> 28 µs, of 100,000 16 -> 13)
     const double share0 = idle ? std::min(target, wave) : target;
     int64_t tiles = 0;
     double stuck = 0;  // the longest tile of a window at its limit
@@ -444,7 +461,7 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
         const double time = longest.back().first;
         Win& w = wins[longest.back().second];
         longest.pop_back();
-        if (target <= wave && time <= stuck) break;
+        if (time <= (target <= wave ? stuck : 0.25 * stuck)) break;
         if (w.chunks >= (double(tiles) < wave ? w.most : w.cap)) {
             stuck = std::max(stuck, time);
             continue;

@@ -125,6 +125,7 @@ struct ScatterLists {
 struct ScatterPlan {
     std::vector<SlotGroup> groups;
     std::vector<uint16_t> slot_list;
+    std::vector<double> narrow;  // per slot: log2 of how far its columns are below kNarrowSlot
     // 4-byte windows (the u32 counts), 8-byte windows of FP64 products and of
     // FP32 ones in fixed point (the same windows, their row chunks by the time
     // that either takes); the evaluator's plan has no f8s
