@@ -259,6 +259,7 @@ const ScatterPlan& eval_plan(cad_patterns* p, int64_t B)
     TuneParams tp;
     tp.partial_cap = 8.0;
     tp.small_floor_bytes = 2.0 * 1024 * 1024;
+    tp.weigh_narrow = false;
     Uploads up;
     build_scatter_plan(*sp, p->slot_lo, p->slot_hi, std::vector<int64_t>{0, B}, std::vector<uint32_t>{0u},
                        int64_t(p->group->cols()), 4, *p->ctx, tp, false, up);

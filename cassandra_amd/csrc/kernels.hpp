@@ -1907,11 +1907,14 @@ __global__ __launch_bounds__(kRowBlock) void k_absmax_systems(const int32_t* __r
 // adds on doubles run several times faster than on floats on this GPU, and the
 // sums are exact for integer data either way) and stores the window to its
 // slice of the partial buffer -- no global atomics.  Entry (r, s) is
-// idx[r row_stride + s slot_stride].  A chunk is one or two rows a thread,
-// so the kernel is a chain of latencies: the first two rows' entries and g are on their way before the
-// window is cleared, all of a row's entries together.  65,536 rows of FIT4:
-// 10.0 µs slot-major (14.3 reading slot after slot from row-major rows), 14.5
-// row-major (15.7), where every lane's entries lie in lines of their own.
+// idx[r row_stride + s slot_stride].  A chunk is one or two rows a thread, so
+// the kernel is a chain of latencies: the first two rows' entries and g are on
+// their way before the window is cleared, all of a row's entries together -- as
+// many as a group of up to four slots or of up to eight has, and no second row
+// where there is none (4,096 rows of 4 slots 8.3 µs with eight loads for each of
+// two rows, 7.0 so, both with the column sums; 65,536 rows of FIT4 21.1 and 17.5).
+// Row-major rows are the slower ones: every lane's entries lie in lines of their
+// own.
 // Groups are runs of at most kMaxSegSlots consecutive slots.
 template <class VT>
 __global__ __launch_bounds__(kScatterBlock) void k_scatter_part(const int32_t* __restrict__ idx, int64_t row_stride,
@@ -1927,35 +1930,43 @@ __global__ __launch_bounds__(kScatterBlock) void k_scatter_part(const int32_t* _
     const SlotGroup gr = constant_load(groups + w.group);
     const int ns = gr.nslots, s0 = uniform_u16(slot_list, gr.first);
     const uint32_t W = w.win_hi - w.win_lo;
-    constexpr int kRows = 2;
-    int32_t c[kRows][kMaxSegSlots];
-    VT y[kRows];
-    auto load = [&](int64_t r0) {
+    auto rows = [&](auto slots) {
+        constexpr int NS = decltype(slots)::value, kRows = 2;
+        int32_t c[kRows][NS];
+        VT y[kRows];
+        // rows a + threadIdx.x and, if the chunk has any, the kScatterBlock rows after
+        auto load = [&](int64_t a) {
 #pragma unroll
-        for (int u = 0; u < kRows; u++) {
-            const int64_t r = min(r0 + u * kScatterBlock, w.row_end - 1);
-            const int32_t* __restrict__ row = idx + r * row_stride + s0 * slot_stride;
+            for (int u = 0; u < kRows; u++) {
+                if (a + u * kScatterBlock >= w.row_end) break;
+                const int64_t r = min(a + u * kScatterBlock + threadIdx.x, w.row_end - 1);
+                const int32_t* __restrict__ row = idx + r * row_stride + s0 * slot_stride;
 #pragma unroll
-            for (int j = 0; j < kMaxSegSlots; j++) c[u][j] = row[min(j, ns - 1) * slot_stride];
-            y[u] = g[r];
+                for (int j = 0; j < NS; j++) c[u][j] = row[min(j, ns - 1) * slot_stride];
+                y[u] = g[r];
+            }
+        };
+        load(w.row_begin);
+        for (uint32_t i = threadIdx.x; i < W; i += kScatterBlock) win[i] = 0.0;
+        __syncthreads();
+        for (int64_t a = w.row_begin; a < w.row_end; a += kRows * kScatterBlock) {
+#pragma unroll
+            for (int u = 0; u < kRows; u++) {
+                if (a + u * kScatterBlock >= w.row_end) break;
+                const bool ok = a + u * kScatterBlock + threadIdx.x < w.row_end;
+#pragma unroll
+                for (int j = 0; j < NS; j++) {
+                    const uint32_t uc = uint32_t(c[u][j]) - w.win_lo;
+                    if (j < ns && ok && uc < W) atomicAdd(&win[uc], double(y[u]));
+                }
+            }
+            load(a + kRows * kScatterBlock);
         }
     };
-    int64_t r0 = w.row_begin + threadIdx.x;
-    load(r0);
-    for (uint32_t i = threadIdx.x; i < W; i += kScatterBlock) win[i] = 0.0;
-    __syncthreads();
-    for (; r0 < w.row_end; r0 += kRows * kScatterBlock) {
-#pragma unroll
-        for (int u = 0; u < kRows; u++) {
-            const bool ok = r0 + u * kScatterBlock < w.row_end;
-#pragma unroll
-            for (int j = 0; j < kMaxSegSlots; j++) {
-                const uint32_t uc = uint32_t(c[u][j]) - w.win_lo;
-                if (j < ns && ok && uc < W) atomicAdd(&win[uc], double(y[u]));
-            }
-        }
-        if (r0 + kRows * kScatterBlock < w.row_end) load(r0 + kRows * kScatterBlock);
-    }
+    if (ns <= kMaxSegSlots / 2)
+        rows(std::integral_constant<int, kMaxSegSlots / 2>{});
+    else
+        rows(std::integral_constant<int, kMaxSegSlots>{});
     __syncthreads();
     store_window<VT>(win, W, 0.0, part + w.part_off);
 }

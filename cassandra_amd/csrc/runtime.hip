@@ -389,7 +389,7 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
         const double frac = double(W) / double(std::max<uint32_t>(1, g.col_hi - g.col_lo));
         if (lam == 1.0 && vbytes == 8) {
             double narrow = 0;
-            for (int j = 0; j < g.nslots; j++) narrow += sp.narrow[L.slot_list[size_t(g.first + j)]];
+            for (int j = 0; j < g.nslots && tune.weigh_narrow; j++) narrow += sp.narrow[L.slot_list[size_t(g.first + j)]];
             return fp32 ? 4.1 + g.nslots * (1.0 + 0.26 * frac) + 0.32 * narrow
                         : 3.0 + g.nslots * (1.0 + 2.9 * frac) + 0.45 * narrow;
         }

@@ -183,6 +183,7 @@ struct TuneParams {
     double scatter_balance = 1.0; // order 0: weight of slot loads against atomics in a window's work (1: loads)
     int pack_slots = kMaxSegSlots; // most slots of narrow groups that share a window
     double small_floor_bytes = 8.0 * 1024 * 1024;  // partial slices a window may take to spread a small system
+    bool weigh_narrow = true;   // slots of few columns weigh more (not the evaluator's, whose loads take longest)
 };
 
 // Most slots sharing a window of a matrix-free scatter: its rows' digits are
