@@ -202,14 +202,15 @@ void upload_programs(cad_patterns* p)
 }
 
 // Rows a wave of the slot-major extraction takes at a time, per lane: four
-// (8-byte stores of u16 entries) where that still gives every SIMD two waves.
+// (8-byte stores of aligned u16 entries) where that still gives every SIMD two
+// waves.
 template <class OutT>
 void extract_slots(hipStream_t s, const TileView& v, const uint64_t* pos, int64_t n, OutT* out, int64_t ld,
                    int64_t nstore, int local, int cus)
 {
     auto launch = [&](auto cc) {
         constexpr int C = decltype(cc)::value;
-        const bool vec = reinterpret_cast<uintptr_t>(out) % (C * sizeof(OutT)) == 0 && ld % C == 0;
+        const bool vec = sizeof(OutT) == 2 && reinterpret_cast<uintptr_t>(out) % (C * sizeof(OutT)) == 0 && ld % C == 0;
         hipLaunchKernelGGL((k_index_extract<OutT, C>), dim3(unsigned(grid1(nstore, kRowBlock * C))), dim3(kRowBlock),
                            0, s, pos, n, nstore, v, out, ld, local, int(vec));
     };

@@ -499,11 +499,13 @@ __device__ __forceinline__ TileRegs load_tile(const TileView& tv, int t)
 
 // Pattern/Indexer.cpp InsertIndices for every row, slot-major: out[s * ld + r]
 // = (local ? 0 : col_offset) + column, rows [n, nstore) as zeros.  A wave takes
-// 64 C rows, lane l the C consecutive rows from its first + l C on, so that
-// a slot's stores are C entries wide (vec: every such run is aligned to its
-// size).  Bound by the stores: 5M rows of FIT8 as u16 take 159 µs for 420 MB,
-// 240 µs (with the clear of the whole matrix that the padding rows cost)
-// digit by digit; 100,000 rows of FIT4 8 µs against 36.
+// 64 C rows: where 2-byte entries are aligned in runs of C (vec), lane l has the
+// C consecutive rows from its first + l C on, so that a slot's stores are C
+// entries wide; else row l of each 64, a store's entries side by side (4-byte
+// entries C apart or in runs took 1M rows of 4 slots 21 and 19 µs, 9.4 so).
+// Bound by the stores: 5M rows of FIT8 as u16 take 124 µs for 420 MB, 240 (with
+// the clear of the whole matrix that the padding rows cost) digit by digit;
+// 100,000 rows of FIT4 8 against 36.
 template <class OutT, int C>
 __global__ __launch_bounds__(kRowBlock) void k_index_extract(const uint64_t* __restrict__ pos, int64_t n,
                                                              int64_t nstore, TileView tv, OutT* __restrict__ out,
@@ -512,13 +514,22 @@ __global__ __launch_bounds__(kRowBlock) void k_index_extract(const uint64_t* __r
     const int lane = threadIdx.x & 63;
     const int64_t base = (blockIdx.x * int64_t(kRowBlock / 64) + (threadIdx.x >> 6)) * (64 * C);
     if (base >= nstore) return;
+    // row c of lane l: l per_lane + c per_row from the wave's first
+    const int per_lane = vec ? C : 1, per_row = vec ? 1 : 64;
     Int4 b[C][4];
+    const int64_t r0 = base + int64_t(lane) * per_lane;
+    // every lane loads its own rows' positions; the transposition hands word g of
+    // the row of lane 16 p + n to lane (n, g) (each lane loading the 16 bits of
+    // its words: 5M rows of FIT8 156 µs, of 4 slots 79 against 30)
 #pragma unroll
-    for (int c = 0; c < C; c++)
+    for (int c = 0; c < C; c++) {
+        const int64_t r = min(r0 + c * per_row, n - 1);
+        uint32_t T[4];
+        ternary_words(pos[2 * r], pos[2 * r + 1], T);
+        transpose_groups(T);
 #pragma unroll
-        for (int p = 0; p < 4; p++)
-            b[c][p] = digits_of_position(pos, min(base + (16 * p + (lane & 15)) * C + c, n - 1));
-    const int64_t r0 = base + int64_t(lane) * C;
+        for (int p = 0; p < 4; p++) b[c][p] = expand_digits(T[p]);
+    }
     for (int t = 0; t < tv.n; t++) {
         const IndexTile tl = constant_load(tv.tiles + t);
         const Int4 wt = *tile_weights(t, tv);
@@ -534,7 +545,7 @@ __global__ __launch_bounds__(kRowBlock) void k_index_extract(const uint64_t* __r
             if (j >= tl.nslots) break;
             OutT o[C];
 #pragma unroll
-            for (int c = 0; c < C; c++) o[c] = r0 + c < n ? OutT(off + v[c][j]) : OutT(0);
+            for (int c = 0; c < C; c++) o[c] = r0 + c * per_row < n ? OutT(off + v[c][j]) : OutT(0);
             OutT* __restrict__ dst = out + int64_t(tl.slot_first + j) * ld + r0;
             if (vec && r0 + C <= nstore) {
                 struct alignas(sizeof(OutT) * C) Run {
@@ -546,7 +557,7 @@ __global__ __launch_bounds__(kRowBlock) void k_index_extract(const uint64_t* __r
             } else {
 #pragma unroll
                 for (int c = 0; c < C; c++)
-                    if (r0 + c < nstore) dst[c] = o[c];
+                    if (r0 + c * per_row < nstore) dst[c * per_row] = o[c];
             }
         }
     }
