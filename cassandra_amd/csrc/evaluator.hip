@@ -204,9 +204,7 @@ __global__ __launch_bounds__(kEvalBlock) void k_eval_staged(const uint64_t* __re
 #pragma unroll
         for (int c = 0; c < C; c++) {
             sum[c] = 0.0f;
-#pragma unroll
-            for (int p = 0; p < 4; p++)
-                b[c][p] = digits_of_position(pos, min(base + 64 * c + 16 * p + (lane & 15), n - 1));
+            digits_of_rows(pos, min(base + 64 * c + lane, n - 1), b[c]);
         }
         TileRegs next = load_tile(tv, 0);
         int next_lds = tile_lds[0];

@@ -371,16 +371,7 @@ __device__ __forceinline__ Int4 expand_digits(uint32_t t)
                 int((t >> 6) & 0x03030303u)};
 }
 
-// Lane (n, g)'s digits of row r, read from the positions (word g: 16-bit
-// group g of P and of O).
-__device__ __forceinline__ Int4 digits_of_position(const uint64_t* __restrict__ pos, int64_t r)
-{
-    const int g = (threadIdx.x >> 4) & 3;
-    const uint16_t* __restrict__ h = reinterpret_cast<const uint16_t*>(pos + 2 * r);
-    return expand_digits(spread16(h[g]) | (spread16(h[4 + g]) << 1));
-}
-
-// The same from the rows' ternary words, tw[r].
+// Lane (n, g)'s digits of row r, from the rows' ternary words tw[r] (word g).
 __device__ __forceinline__ Int4 digits_of_words(const uint4* __restrict__ tw, int64_t r)
 {
     return expand_digits(reinterpret_cast<const uint32_t*>(tw + r)[(threadIdx.x >> 4) & 3]);
@@ -401,9 +392,20 @@ __device__ __forceinline__ void transpose_groups(uint32_t (&r)[4])
     r[3] = b[1];
 }
 
-// The pattern-local column of slot g of the tile for the four position sets
-// b[0..4) (idx[p]: lane (n, g) holds slot g of position n of set p; lanes of
-// slots past the tile's hold column 0 of some configuration).
+// The digits of the wave's 64 rows, lane l's row r: every lane loads its own
+// position, and the transposition hands word g of lane 16 p + n's row to lane (n, g)
+// of set p (each lane loading the 16 bits of its words: extraction of 5M rows of
+// FIT8 156 µs against 124, of 4 slots 79 against 30; 300,000 positions scored
+// with 4 slots 7.6 against 5.3, with 18 slots 19.0 against 16.3).
+__device__ __forceinline__ void digits_of_rows(const uint64_t* __restrict__ pos, int64_t r, Int4 (&b)[4])
+{
+    uint32_t T[4];
+    ternary_words(pos[2 * r], pos[2 * r + 1], T);
+    transpose_groups(T);
+#pragma unroll
+    for (int p = 0; p < 4; p++) b[p] = expand_digits(T[p]);
+}
+
 // Tile t's weights (two blocks of 64 a tile, the second for wide pairs with a
 // diagonal).
 __device__ __forceinline__ const Int4* tile_weights(int t, const TileView& tv)
@@ -411,6 +413,9 @@ __device__ __forceinline__ const Int4* tile_weights(int t, const TileView& tv)
     return reinterpret_cast<const Int4*>(tv.weights) + (128 * t + int(threadIdx.x & 63));
 }
 
+// The pattern-local column of slot g of the tile for the four position sets
+// b[0..4) (idx[p]: lane (n, g) holds slot g of position n of set p; lanes of
+// slots past the tile's hold column 0 of some configuration).
 __device__ __forceinline__ void tile_columns(const IndexTile& t, int number, const TileView& tv, const Int4& w,
                                              const Int4 (&b)[4], uint32_t (&idx)[4])
 {
@@ -518,18 +523,8 @@ __global__ __launch_bounds__(kRowBlock) void k_index_extract(const uint64_t* __r
     const int per_lane = vec ? C : 1, per_row = vec ? 1 : 64;
     Int4 b[C][4];
     const int64_t r0 = base + int64_t(lane) * per_lane;
-    // every lane loads its own rows' positions; the transposition hands word g of
-    // the row of lane 16 p + n to lane (n, g) (each lane loading the 16 bits of
-    // its words: 5M rows of FIT8 156 µs, of 4 slots 79 against 30)
 #pragma unroll
-    for (int c = 0; c < C; c++) {
-        const int64_t r = min(r0 + c * per_row, n - 1);
-        uint32_t T[4];
-        ternary_words(pos[2 * r], pos[2 * r + 1], T);
-        transpose_groups(T);
-#pragma unroll
-        for (int p = 0; p < 4; p++) b[c][p] = expand_digits(T[p]);
-    }
+    for (int c = 0; c < C; c++) digits_of_rows(pos, min(r0 + c * per_row, n - 1), b[c]);
     for (int t = 0; t < tv.n; t++) {
         const IndexTile tl = constant_load(tv.tiles + t);
         const Int4 wt = *tile_weights(t, tv);
@@ -582,8 +577,7 @@ __global__ __launch_bounds__(kRowBlock) void k_index_extract_rows(const uint64_t
     if (base >= n) return;
     const int rows = int(min<int64_t>(64, n - base));
     Int4 b[4];
-#pragma unroll
-    for (int p = 0; p < 4; p++) b[p] = digits_of_position(pos, min<int64_t>(base + 16 * p + (lane & 15), n - 1));
+    digits_of_rows(pos, min<int64_t>(base + lane, n - 1), b);
     uint32_t* __restrict__ dst = out + base * k;
     int first = 0;  // first slot of the chunk
     for (int t = 0; t < tv.n; t++) {
