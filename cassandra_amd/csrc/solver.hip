@@ -1198,8 +1198,14 @@ static void pcg_solve(cad_matrix* m, const double* b, double* x, const cad_solve
         const int n = std::min(batch, o.max_iterations - it);
         // a graph is captured where it will be replayed: capturing and
         // instantiating takes longer than launching once (FitWeights of 100,000
-        // rows, one batch of ten iterations: 1,030 µs with it, 840 without)
-        const bool replayed = ws.exec != nullptr || o.max_iterations - it >= 2 * batch;
+        // rows, one batch of ten iterations: 1,030 µs with it, 928 without).  It
+        // costs about what kDirectBatches replays gain (3,000 rows, 100
+        // iterations: 2.92 ms a solve against 3.07), so solves of one long batch
+        // get one after that many on the same matrix; of ten iterations a replay
+        // takes as long as their launches (20,000 rows 551 µs against 541).
+        constexpr int kDirectBatches = 12, kLongBatch = 32;
+        const bool replayed = ws.exec != nullptr || o.max_iterations - it >= 2 * batch ||
+                              (batch >= kLongBatch && ws.direct_batches >= kDirectBatches);
         if (o.use_graph && batch > 1 && n == batch && s != nullptr && replayed) {
             // `batch` iterations captured once per workspace, replayed
             if (!ws.exec || ws.graph_iters != batch) {
@@ -1219,6 +1225,7 @@ static void pcg_solve(cad_matrix* m, const double* b, double* x, const cad_solve
             CAD_HIP(hipGraphLaunch(ws.exec, s));
         } else {
             for (int i = 0; i < n; i++) pcg_iteration<VT>(m, ws, s);
+            ws.direct_batches += n == batch;
         }
         it += n;
         const PcgScalars* h = read_scalars<PcgScalars>(m, ws, ws.pscal, s);

@@ -37,6 +37,7 @@ struct Workspace {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     int graph_iters = 0, graph_prec = 0;
+    int direct_batches = 0;   // whole batches launched without a graph (PCG)
     int graph_gen = -1;       // ActiveLists generation the graph was captured with (-1: full lists)
     ActiveLists active;
     bool use_active = false;  // iterations launch the active lists
