@@ -225,9 +225,15 @@ void extract_rows(cad_patterns* p, const uint64_t* pos, int64_t n, uint32_t* out
     const int chunk = std::min(k, kExtractChunk);
     const int pitch = chunk == k ? k : chunk | 1;
     const size_t lds = size_t(kRowBlock) * size_t(pitch) * sizeof(uint32_t);
-    hipLaunchKernelGGL(k_index_extract_rows, dim3(unsigned(grid1(n, kRowBlock))), dim3(kRowBlock), lds,
-                       p->ctx->stream, pos, n, p->tiles(), k, chunk, pitch, out,
-                       int(reinterpret_cast<uintptr_t>(out) % 16 == 0));
+    // (a launch holds fewer than 2^32 threads, one a row)
+    constexpr int64_t kPart = int64_t(1) << 31;
+    for (int64_t a = 0; a < n; a += kPart) {
+        const int64_t m = std::min(kPart, n - a);
+        uint32_t* dst = out + a * k;
+        hipLaunchKernelGGL(k_index_extract_rows, dim3(unsigned(grid1(m, kRowBlock))), dim3(kRowBlock), lds,
+                           p->ctx->stream, pos + 2 * a, m, p->tiles(), k, chunk, pitch, dst,
+                           int(reinterpret_cast<uintptr_t>(dst) % 16 == 0));
+    }
     CAD_HIP(hipGetLastError());
 }
 

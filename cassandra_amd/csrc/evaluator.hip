@@ -255,6 +255,8 @@ int blocks_for(uint64_t n, int cap = 4096)
 // 20.3, 46 slots 15.2 / 16.4, 4 patterns 9.4 / 11.3; twice as many: 38.7 / 21.7,
 // 38.2 / 23.1, 27.5 / 17.2, 16.2 / 13.6).
 constexpr int64_t kEvalStagedRows = 512;
+// Most positions of one launch of the block kernel.
+constexpr int64_t kEvalBlockRows = int64_t(1) << 26;
 
 // Per-slot table layout of a pattern group (variation after variation, in
 // slot order), uploaded once per pattern group.
@@ -393,8 +395,12 @@ void eval_weights(cad_patterns* p, const float* w, const uint64_t* pos, int64_t 
                            E.d_tile_lds.as<int32_t>(), E.d_segs.as<PhaseSeg>(), E.nsegs, w, cols, out);
     } else {
         const int waves = std::min(kEvalBlock / 64, tv.n);
-        hipLaunchKernelGGL(k_eval_block, dim3(unsigned((n + 63) / 64)), dim3(unsigned(64 * waves)), 0, s, pos, n, tv, w,
-                           cols, out);
+        // (a launch holds fewer than 2^32 threads: 2^28 positions of 16 waves)
+        for (int64_t a = 0; a < n; a += kEvalBlockRows) {
+            const int64_t m = std::min(kEvalBlockRows, n - a);
+            hipLaunchKernelGGL(k_eval_block, dim3(unsigned((m + 63) / 64)), dim3(unsigned(64 * waves)), 0, s,
+                               pos + 2 * a, m, tv, w, cols, out + a);
+        }
     }
     CAD_HIP(hipGetLastError());
 }
