@@ -157,19 +157,6 @@ void upload_programs(cad_patterns* p)
         d.dense_offset = s.dense_offset;
         slots.push_back(d);
     }
-    // the ternary-word programs: per list, its entries {2 (q mod 16), 3^j}
-    // grouped by the word q / 16; three zero entries end the array (the
-    // kernels load four entries at a time, also at a list's last entry)
-    std::vector<DevTern> tslots;
-    std::vector<uint32_t> tern;
-    for (const SlotProgram& s : g.slots) {
-        DevTern t;
-        std::memset(&t, 0, sizeof(t));
-        for (int l = 0; l < 3; l++)
-            append_ternary_list(s.list[l].src.data(), int(s.list[l].src.size()), tern, t, l);
-        tslots.push_back(t);
-    }
-    tern.insert(tern.end(), kTernPadding, 0u);
     // the index tiles, pattern after pattern
     IndexTiles it;
     int slot = 0;
@@ -184,8 +171,6 @@ void upload_programs(cad_patterns* p)
     for (size_t t = 0; t < it.tiles.size(); t++) p->slot_tile.insert(p->slot_tile.end(), it.tiles[t].nslots, uint32_t(t));
     p->d_tiles = to_device(it.tiles, st);
     p->d_weights = to_device(it.weights, st);
-    p->d_tslots = to_device(tslots, st);
-    p->d_tern = to_device(tern, st);
     p->d_slots = to_device(slots, st);
     sq.resize((sq.size() + 7) / 4 * 4, 0);  // the kernels read the squares as whole 32-bit words
     p->d_sq = to_device(sq, st);
@@ -196,9 +181,6 @@ void upload_programs(cad_patterns* p)
         p->slot_lo.push_back(s.col_offset);
         p->slot_hi.push_back(s.col_offset + s.block_size);
     }
-    std::vector<uint32_t> zeros(std::max<size_t>(1, g.slots.size()), 0u);
-    p->d_base0 = to_device(zeros, st);
-    p->d_syscol0 = to_device(std::vector<uint32_t>{0u}, st);
 }
 
 // Rows a wave of the slot-major extraction takes at a time, per lane: four
@@ -676,8 +658,6 @@ int cad_matrix_from_positions_mf(cad_patterns* p, const uint64_t* d_pos, int64_t
         m->ntiles = p->ntiles;
         m->slot_tile = p->slot_tile;
         m->d_slot_tile = to_device(m->slot_tile, s);
-        copy(m->d_tslots, p->d_tslots);
-        copy(m->d_tern, p->d_tern);
         m->d_pos = DBuf(sizeof(uint64_t) * 2 * size_t(n));
         CAD_HIP(hipMemcpyAsync(m->d_pos.p, d_pos, m->d_pos.bytes, hipMemcpyDeviceToDevice, s));
         m->d_tw = DBuf(sizeof(uint32_t) * 4 * size_t(n));

@@ -334,9 +334,6 @@ const EvalPlan& eval_weights_plan(cad_patterns* p)
     if (p->eval_plan) return *p->eval_plan;
     std::unique_ptr<EvalPlan> E(new EvalPlan);
     const PatternGroup& g = *p->group;
-    for (const PatternInfo& pi : g.patterns)
-        if (__builtin_popcountll(pi.mask) > 16)
-            throw Error(CAD_ERR_PATTERN, "expanded tables need patterns of at most 16 squares");
     // the patterns with the fewest columns a variation first
     std::vector<size_t> order(g.patterns.size());
     for (size_t i = 0; i < order.size(); i++) order[i] = i;

@@ -13,8 +13,7 @@ void weights_expand(cad_patterns* p, const float* d_w, float* d_tables);
 // configuration of each column in Configurations order wins, as in the
 // reference; synchronises the stream).
 void weights_compact(cad_patterns* p, const float* d_tables, float* d_w);
-// What the evaluator keeps in LDS (built on first use; throws for patterns of
-// more than 16 squares).
+// What the evaluator keeps in LDS (built on first use).
 const EvalPlan& eval_weights_plan(cad_patterns* p);
 // ScoreEstimator::Eval for n positions from compact weights (16-byte aligned).
 void eval_weights(cad_patterns* p, const float* d_w, const uint64_t* d_pos, int64_t n, float* d_out);

@@ -185,8 +185,6 @@ __device__ __forceinline__ uint32_t slot_index(const DevSlot& s, const uint8_t* 
     return idx;
 }
 
-
-
 // The four ternary words of a position: square q's digit P_q + 2 O_q in bits
 // 2 (q mod 16) of word q / 16 (each 16-bit half-board's bits spread to every
 // other bit).
@@ -252,96 +250,6 @@ __device__ __forceinline__ int uniform_u16(const uint16_t* p, int i)
 {
     const uint32_t w = __builtin_amdgcn_readfirstlane(reinterpret_cast<const uint32_t*>(p)[i >> 1]);
     return int((w >> (16 * (i & 1))) & 0xFFFFu);
-}
-
-// Four entries of a ternary-word program (two words each: the digit's shift,
-// then 3^j) at a wave-uniform address, through the constant address space so
-// that they load into scalar registers with one 32-byte load (the kernels
-// never write the arrays read this way).
-struct TernEntries {
-    uint32_t w[8];
-};
-__device__ __forceinline__ TernEntries scalar_load_entries(const uint32_t* p)
-{
-    const ConstWords c = (ConstWords)(p);
-    TernEntries e;
-#pragma unroll
-    for (int i = 0; i < 8; i++) e.w[i] = c[i];
-    return e;
-}
-
-// Adds entry q's term, digit x 3^j, to RPT rows (word W of each row's
-// ternary words): one bit-field extract (shift straight from the entry) and
-// one 24-bit multiply-add a row.
-template <int RPT, int W>
-__device__ __forceinline__ void tern_term(const TernEntries& e, int q, const uint32_t (&T)[RPT][4],
-                                          uint32_t (&v)[RPT])
-{
-#pragma unroll
-    for (int i = 0; i < RPT; i++) v[i] += __umul24((T[i][W] >> e.w[2 * q]) & 3u, e.w[2 * q + 1]);
-}
-
-// The n entries of word W from entry `off` on: whole groups of four, then the
-// last one to three behind uniform branches (no padding entries to evaluate).
-template <int RPT, int W>
-__device__ __forceinline__ uint32_t tern_word(const uint32_t* __restrict__ ent, uint32_t off, uint32_t n,
-                                              const uint32_t (&T)[RPT][4], uint32_t (&v)[RPT])
-{
-    for (uint32_t g = n >> 2; g > 0; g--, off += 4) {
-        const TernEntries e = scalar_load_entries(ent + 2 * off);
-#pragma unroll
-        for (int q = 0; q < 4; q++) tern_term<RPT, W>(e, q, T, v);
-    }
-    const uint32_t r = n & 3u;
-    if (r) {
-        const TernEntries e = scalar_load_entries(ent + 2 * off);
-        tern_term<RPT, W>(e, 0, T, v);
-        if (r > 1) tern_term<RPT, W>(e, 1, T, v);
-        if (r > 2) tern_term<RPT, W>(e, 2, T, v);
-    }
-    return off + r;
-}
-
-// The value sum_j 3^j (P[q_j] + 2 O[q_j]) of one square list for RPT rows,
-// from the list's ternary-word program (3^j < 2^24: the host builds no list of
-// more than 16 squares).  The entries are the same for the whole wave.
-template <int RPT>
-__device__ __forceinline__ void tern_values(const uint32_t* __restrict__ ent, uint32_t off, uint32_t nent,
-                                            const uint32_t (&T)[RPT][4], uint32_t (&v)[RPT])
-{
-#pragma unroll
-    for (int i = 0; i < RPT; i++) v[i] = 0u;
-    off = tern_word<RPT, 0>(ent, off, nent & 0xFFu, T, v);
-    off = tern_word<RPT, 1>(ent, off, (nent >> 8) & 0xFFu, T, v);
-    off = tern_word<RPT, 2>(ent, off, (nent >> 16) & 0xFFu, T, v);
-    tern_word<RPT, 3>(ent, off, nent >> 24, T, v);
-}
-
-// slot_index for RPT rows from their ternary words (the same values).
-template <int RPT>
-__device__ __forceinline__ void slot_index_rows(const DevSlot& s, const DevTern& t, const uint32_t* __restrict__ ent,
-                                                const uint32_t* __restrict__ dense, const uint32_t (&T)[RPT][4],
-                                                uint32_t (&idx)[RPT])
-{
-    tern_values<RPT>(ent, t.off[0], t.nent[0], T, idx);
-    if (s.kind == 0) return;
-    if (s.kind == 3) {
-#pragma unroll
-        for (int i = 0; i < RPT; i++) idx[i] = dense[s.dense_offset + idx[i]];
-        return;
-    }
-    uint32_t b[RPT];
-    tern_values<RPT>(ent, t.off[1], t.nent[1], T, b);
-#pragma unroll
-    for (int i = 0; i < RPT; i++) {
-        const uint32_t lo = idx[i] < b[i] ? idx[i] : b[i], hi = idx[i] < b[i] ? b[i] : idx[i];
-        idx[i] = lo * s.hs + hi - lo * (lo + 1u) / 2u;
-    }
-    if (s.kind == 2) {
-        tern_values<RPT>(ent, t.off[2], t.nent[2], T, b);
-#pragma unroll
-        for (int i = 0; i < RPT; i++) idx[i] = idx[i] * s.ds + b[i];
-    }
 }
 
 // The ternary words of n positions (a matrix-free matrix keeps them, so the
@@ -637,8 +545,6 @@ struct PositionsView {
     const DevSlot* __restrict__ slots;
     const uint8_t* __restrict__ sq;
     const uint32_t* __restrict__ dense;
-    const DevTern* __restrict__ tslots;  // the ternary-word programs of the same slots
-    const uint32_t* __restrict__ tern;
     const uint4* __restrict__ tw;        // every row's ternary words (computed once, at creation)
     TileView tiles;
     const uint32_t* __restrict__ slot_tiles;  // the index tile of every slot

@@ -544,24 +544,6 @@ void finish_lists(ScatterLists& L, int nsys)
 
 }  // namespace
 
-void append_ternary_list(const uint8_t* src, int n, std::vector<uint32_t>& tern, DevTern& t, int l)
-{
-    // the kernels multiply by 3^j in 24-bit arithmetic: 3^15 < 2^24
-    if (n > 16) throw Error(CAD_ERR_PATTERN, "a pattern list of more than 16 squares");
-    t.off[l] = uint32_t(tern.size() / 2);
-    t.nent[l] = 0;
-    for (int w = 0; w < 4; w++) {
-        uint32_t cnt = 0;
-        for (int j = 0; j < n; j++)
-            if (src[j] / 16 == w) {
-                tern.push_back(uint32_t(2 * (src[j] % 16)));
-                tern.push_back(pow3(j));
-                cnt++;
-            }
-        t.nent[l] |= cnt << (8 * w);
-    }
-}
-
 void IndexTiles::add(const SlotProgram* slots, int n, int first)
 {
     // row 4 j + role of the tile whose weights start at `at` gains 3^(e mod 5)

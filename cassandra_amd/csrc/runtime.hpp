@@ -73,14 +73,6 @@ private:
     size_t reserved = 0;
 };
 
-// Appends list l of a ternary-word program (DevTern): the squares src[j] of a
-// base-3 number sum_j 3^j (P[src_j] + 2 O[src_j]) as entries {2 (q mod 16),
-// 3^j} grouped by the word q / 16; sets t.off[l] and t.nent[l].  Throws for
-// more than 16 squares (the kernels multiply by 3^j in 24 bits).  A program
-// array must end with kTernPadding zero words.
-void append_ternary_list(const uint8_t* src, int n, std::vector<uint32_t>& tern, DevTern& t, int l);
-constexpr int kTernPadding = 6;
-
 // The index tiles (IndexTile) of a sequence of slot programs, and their
 // weights (two blocks of 1 KB a tile: lane l's 16 bytes are row l % 16 of the tile, squares
 // 16 (l / 16) .. + 15, byte 4 v + m the square v + 4 m of those, the order the
@@ -256,7 +248,6 @@ struct cad_patterns {
     cad_context* ctx = nullptr;
     std::unique_ptr<cad::PatternGroup> group;
     cad::DBuf d_slots, d_sq, d_dense;
-    cad::DBuf d_tslots, d_tern;             // the ternary-word form of the slot programs
     cad::DBuf d_tiles, d_weights;           // the slots as index tiles
     int ntiles = 0;
     std::vector<uint32_t> slot_tile;        // the index tile of every slot
@@ -264,7 +255,6 @@ struct cad_patterns {
     std::vector<uint32_t> slot_lo, slot_hi;  // global column range of every slot
     // scatter plans of the evaluator backward, one per minibatch size
     std::map<int64_t, std::unique_ptr<cad::ScatterPlan>> eval_plans;
-    cad::DBuf d_base0, d_syscol0;            // zeros
     std::unique_ptr<cad::ExpandedLayout> layout;  // expanded tables (built on first use)
     std::unique_ptr<cad::EvalPlan> eval_plan;     // the evaluator's (built on first use)
     // the training step's buffers: per-row gradient of the loss, the weight
@@ -298,7 +288,7 @@ struct cad_matrix {
     int64_t ld = 0;                 // rows rounded up to kIndexAlign (rows r >= rows are zero)
     // matrix-free: the positions and a copy of the pattern group's slot programs
     bool mf = false;
-    cad::DBuf d_pos, d_slots, d_sq, d_dense, d_tslots, d_tern, d_tw, d_tiles, d_weights, d_slot_tile;
+    cad::DBuf d_pos, d_slots, d_sq, d_dense, d_tw, d_tiles, d_weights, d_slot_tile;
     int ntiles = 0;
     std::vector<uint32_t> slot_tile;        // the index tile of every slot
     cad::TileView tiles() const { return cad::tile_view(d_tiles, d_weights, d_dense, ntiles); }
