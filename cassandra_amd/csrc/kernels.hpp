@@ -1662,14 +1662,13 @@ __device__ __forceinline__ VT scatter_scale(LsqrScalars* div, int mode, int sys,
 // can overflow: |term| < 2^ey and fewer than 2^cbits terms per column and
 // work item, so every sum stays below 2^(62 - 1); each term keeps at least 32
 // bits (rounding error <= 2^(ey - 33) of the largest term, far below FP32
-// rounding of the sums).  ymax holds, per system, the bits of max |y| (a
-// non-negative float, NaN and inf compare above every finite value); null in
-// an LSQR iteration, where |u_r / beta| < 2 by construction.
-// The kYmax scatter instantiation forms each system's max |y| itself from
-// the per-row-block maxima of k_absmax_blocks (ypart, the system's blocks at
-// yfirst[sys], ycount[sys]) instead of reading ymax.
+// rounding of the sums where y is of one size; a column that only terms of
+// 2^-15 of the largest or less reach keeps fewer bits than FP32 has).  Outside
+// an LSQR iteration, where |u_r / beta| < 2 by construction, the kYmax
+// instantiation takes the bits of each system's max |y| (a non-negative float,
+// NaN and inf above every finite value) from the row blocks' maxima that
+// k_absmax_blocks left (ypart, the system's blocks at yfirst[sys], ycount[sys]).
 struct FixedScale {
-    const unsigned* ymax;
     int cbits;
     const unsigned* ypart;
     const int32_t* yfirst;
@@ -1712,12 +1711,6 @@ __device__ __forceinline__ unsigned system_max(const FixedScale& fx, int sys, un
     return sh[0];
 }
 
-// The same for system sys, with its bits read from fx.ymax where given.
-__device__ __forceinline__ double fixed_scale(const FixedScale& fx, int sys, double sc)
-{
-    return fixed_scale_bits(fx.cbits, fx.ymax != nullptr, fx.ymax ? fx.ymax[sys] : 0u, sc);
-}
-
 template <class WT>
 __device__ __forceinline__ WT window_term(double v, double fscale)
 {
@@ -1740,7 +1733,7 @@ __device__ __forceinline__ double window_scale(const FixedScale& fx, int sys, VT
         const unsigned b = system_max<BS>(fx, sys, shm);
         return allowed ? fixed_scale_bits(fx.cbits, true, b, double(sc)) : 0.0;
     } else {
-        return allowed ? fixed_scale(fx, sys, double(sc)) : 0.0;
+        return allowed ? fixed_scale_bits(fx.cbits, false, 0u, double(sc)) : 0.0;
     }
 }
 
@@ -1758,9 +1751,8 @@ __device__ __forceinline__ void store_window(const double* __restrict__ win, uin
     }
 }
 
-// max |VT(y)| as float bits (non-negative floats order as unsigned integers;
-// NaN and inf above every finite value), the ymax of FixedScale, in two
-// launches without atomics: one value per row block, then one per system.
+// max |y| of each row block as float bits (non-negative floats order as unsigned
+// integers; NaN and inf above every finite value): the ypart of FixedScale.
 // 5M rows: 7.1 µs, 10.5 with one row a thread at a time.
 template <class YT>
 __global__ __launch_bounds__(kRowBlock) void k_absmax_blocks(const RowWork* __restrict__ work,
@@ -1783,33 +1775,6 @@ __global__ __launch_bounds__(kRowBlock) void k_absmax_blocks(const RowWork* __re
     if (threadIdx.x == 0) {
         for (int i = 1; i < kRowBlock / 64; i++) mb = max(mb, sh[i]);
         part[blockIdx.x] = mb;
-    }
-}
-
-__global__ __launch_bounds__(kRowBlock) void k_absmax_systems(const int32_t* __restrict__ first,
-                                                              const int32_t* __restrict__ count,
-                                                              const unsigned* __restrict__ part,
-                                                              unsigned* __restrict__ bits)
-{
-    __shared__ unsigned sh[kRowBlock / 64];
-    const int s = blockIdx.x;
-    unsigned mb = 0;
-    const int n = count[s];
-    const unsigned* __restrict__ p = part + first[s];
-    // eight in flight (the last again past the end): 20M rows took 19 µs with one
-    for (int i = threadIdx.x; i < n; i += 8 * kRowBlock) {
-        unsigned v[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = p[min(i + j * kRowBlock, n - 1)];
-#pragma unroll
-        for (int j = 0; j < 8; j++) mb = max(mb, v[j]);
-    }
-    for (int o = 32; o > 0; o >>= 1) mb = max(mb, unsigned(__shfl_xor(int(mb), o, 64)));
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = mb;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int i = 1; i < kRowBlock / 64; i++) mb = max(mb, sh[i]);
-        bits[s] = mb;
     }
 }
 

@@ -893,9 +893,8 @@ void build_plans(cad_matrix* m)
     up.put(g.d_row_counters, zeros);
     up.put(g.d_col_counters, zeros);
     up.reserve(g.d_partials, 2 * sizeof(double) * std::max<size_t>(1, std::max(g.rows.size(), g.cols.size())));
-    // max |y| per row block and per system, for the fixed-point FP32 scatter
+    // max |y| per row block, for the fixed-point FP32 scatter
     up.reserve(m->splan.d_ymax_part, sizeof(unsigned) * std::max<size_t>(1, g.rows.size()));
-    up.reserve(m->splan.d_ymax, sizeof(unsigned) * size_t(std::max(1, m->nsys)));
     up.flush(ctx.stream);
 }
 

@@ -126,8 +126,7 @@ struct ScatterPlan {
     // (matrix-free): of each slot, and of the row itself
     std::vector<double> slot_cost;
     double row_cost = 0.0;
-    DBuf d_ymax;          // per system: bits of max |y| of the last FP32 scatter (fixed-point scale)
-    DBuf d_ymax_part;     // the same per row block of the grid plan
+    DBuf d_ymax_part;     // per row block of the grid plan: bits of max |y| of the last FP32 scatter (fixed-point scale)
 };
 
 // LDS-staged gather of one value size: row tiles and the slot segments.

@@ -82,9 +82,10 @@ PT* partials(ScatterLists& L)
 // column reduction in chunk order (which writes every column of z).
 // The first-stage scatter kernel of a view: vector loads of rpt (4, or 8 for
 // u16 indices) consecutive rows for stored indices, two runs of 64 rows a wave
-// and step for a matrix-free matrix; f receives the kernel.  beta: the instantiation that forms an LSQR iteration's beta itself;
-// ymax: the instantiation that forms each system's max |y| from the row-block
-// maxima (FixedScale::ypart), used by FP32 PCG.
+// and step for a matrix-free matrix; f receives the kernel.  beta: the
+// instantiation that forms an LSQR iteration's beta itself; ymax: the one that
+// forms each system's max |y| from the row blocks' maxima (FixedScale::ypart),
+// of every other FP32 A^T y of a stored matrix.
 template <class VT, class YT, class View, class F>
 void with_scatter_kernel(int rpt, bool beta, bool ymax, F&& f)
 {
@@ -115,24 +116,17 @@ constexpr bool fixed_point_scatter()
 }
 
 template <class YT>
-void launch_absmax(ScatterPlan& sp, const YT* y, const GridPlan& g, int nsys, hipStream_t s, bool systems = true)
+void launch_absmax(ScatterPlan& sp, const YT* y, const GridPlan& g, hipStream_t s)
 {
     if (g.rows.empty()) return;
     hipLaunchKernelGGL(k_absmax_blocks<YT>, dim3(unsigned(g.rows.size())), dim3(kRowBlock), 0, s,
                        g.d_rows.as<RowWork>(), y, sp.d_ymax_part.as<unsigned>());
-    if (!systems) {
-        CAD_HIP(hipGetLastError());
-        return;
-    }
-    hipLaunchKernelGGL(k_absmax_systems, dim3(unsigned(nsys)), dim3(kRowBlock), 0, s, g.d_row_first.as<int32_t>(),
-                       g.d_row_count.as<int32_t>(), (const unsigned*)sp.d_ymax_part.as<unsigned>(),
-                       sp.d_ymax.as<unsigned>());
     CAD_HIP(hipGetLastError());
 }
 
-// yrows: the row blocks whose maxima k_absmax_blocks left in sp.d_ymax_part,
-// for the instantiation that forms max |y| itself (FP32 windows of a stored
-// matrix only; null: read sp.d_ymax).
+// yrows: the row blocks whose maxima k_absmax_blocks left in sp.d_ymax_part
+// (FP32 windows of a stored matrix outside an LSQR iteration, whose terms are
+// bounded by construction; null otherwise).
 template <class VT, class YT, class View>
 void launch_scatter_tiles(ScatterPlan& sp, const View& view, int rpt, const uint32_t* sys_col, const YT* y,
                           const LsqrScalars* div, int mode, hipStream_t s, bool y_padded = false,
@@ -143,11 +137,8 @@ void launch_scatter_tiles(ScatterPlan& sp, const View& view, int rpt, const uint
     const ScatterWork* work = al ? al->scatter.as<ScatterWork>() : L.d_work.as<ScatterWork>();
     const int nwork = al ? al->nscatter : int(L.work.size());
     if (nwork == 0) return;
-    // the fixed-point windows read max |y| per system outside an LSQR
-    // iteration, whose terms are bounded by construction
-    const bool ymax = yrows && fixed_point_scatter<VT, View>() && mode != kScatterLsqr;
-    const FixedScale fx{fixed_point_scatter<VT, View>() && mode != kScatterLsqr ? sp.d_ymax.as<unsigned>() : nullptr,
-                        al ? al->cbits : L.cbits, ymax ? sp.d_ymax_part.as<unsigned>() : nullptr,
+    const bool ymax = fixed_point_scatter<VT, View>() && mode != kScatterLsqr;
+    const FixedScale fx{al ? al->cbits : L.cbits, ymax ? sp.d_ymax_part.as<unsigned>() : nullptr,
                         ymax ? yrows->d_row_first.as<int32_t>() : nullptr,
                         ymax ? yrows->d_row_count.as<int32_t>() : nullptr};
     VT* part = al ? al->part.as<VT>() : partials<VT>(L);
@@ -173,14 +164,13 @@ void launch_scatter_reduce(ScatterPlan& sp, const LsqrScalars* div, int mode, ZT
 
 template <class VT, class YT, class ZT, class View>
 void launch_scatter(ScatterPlan& sp, const View& view, int rpt, const uint32_t* sys_col, const YT* y,
-                    const LsqrScalars* div, int mode, ZT* z, const GridPlan& g, int nsys, hipStream_t s,
-                    bool y_padded = false)
+                    const LsqrScalars* div, int mode, ZT* z, const GridPlan& g, hipStream_t s, bool y_padded = false)
 {
     // the fixed-point window tiles take the row blocks' maxima themselves, a
     // launch less (A x and A^T y of 5M rows of FIT8 279 -> 274 µs, of 50,001
     // rows of FIT4 57.7 -> 55.5)
     if (fixed_point_scatter<VT, View>() && mode != kScatterLsqr && !lists<VT>(sp).work.empty())
-        launch_absmax(sp, y, g, nsys, s, false);
+        launch_absmax(sp, y, g, s);
     launch_scatter_tiles<VT, YT>(sp, view, rpt, sys_col, y, div, mode, s, y_padded, nullptr, GridSys{}, &g);
     launch_scatter_reduce<VT>(sp, div, mode, z, s);
 }
@@ -207,7 +197,7 @@ void scatter(cad_matrix* m, const YT* y, const LsqrScalars* div, ZT* z, hipStrea
     const int mode = div ? kScatterLsqr : kScatterAll;
     with_view(m, [&](auto view) {
         launch_scatter<VT, YT, ZT>(m->splan, view, m->tune.srpt, m->d_sys_col.as<uint32_t>(), y, div, mode, z,
-                                   m->grid, m->nsys, s, y_padded);
+                                   m->grid, s, y_padded);
     });
 }
 
@@ -217,7 +207,7 @@ void scatter_restart(cad_matrix* m, const YT* y, const LsqrScalars* sel, ZT* z, 
 {
     with_view(m, [&](auto view) {
         launch_scatter<VT, YT, ZT>(m->splan, view, m->tune.srpt, m->d_sys_col.as<uint32_t>(), y, sel,
-                                   kScatterRestart, z, m->grid, m->nsys, s);
+                                   kScatterRestart, z, m->grid, s);
     });
 }
 
@@ -1133,7 +1123,7 @@ static void pcg_iteration(cad_matrix* m, Workspace& ws, hipStream_t s)
     ScatterLists& L = lists<VT>(m->splan);
     with_view(m, [&](auto view) {
         const bool fixed = fixed_point_scatter<VT, decltype(view)>() && !L.work.empty();
-        if (fixed) launch_absmax(m->splan, ws.t.as<VT>(), g, m->nsys, s, false);
+        if (fixed) launch_absmax(m->splan, ws.t.as<VT>(), g, s);
         launch_scatter_tiles<VT, VT>(m->splan, view, m->tune.srpt, m->d_sys_col.as<uint32_t>(), ws.t.as<VT>(),
                                      nullptr, kScatterAll, s, false, nullptr, GridSys{}, fixed ? &g : nullptr);
     });
@@ -1510,9 +1500,10 @@ void kernel_times(cad_matrix* m, int reps, double* us, int n)
         partials<float>(lists<float>(sp));
         const uint32_t* sc = m->d_sys_col.as<uint32_t>();
         const float* y = y4.as<float>();
-        if (fixed_point_scatter<float, View>())
-            v[3] = t.us([&] { launch_absmax(sp, y, m->grid, m->nsys, s); }, s, reps);
-        v[1] = t.us([&] { launch_scatter_tiles<float, float>(sp, view, m->tune.srpt, sc, y, nullptr, kScatterAll, s); },
+        // the parts as launch_scatter launches them
+        if (fixed_point_scatter<float, View>()) v[3] = t.us([&] { launch_absmax(sp, y, m->grid, s); }, s, reps);
+        v[1] = t.us([&] { launch_scatter_tiles<float, float>(sp, view, m->tune.srpt, sc, y, nullptr, kScatterAll, s,
+                                                             false, nullptr, GridSys{}, &m->grid); },
                     s, reps);
         v[2] = t.us([&] { launch_scatter_reduce<float>(sp, nullptr, kScatterAll, z4.as<float>(), s); }, s, reps);
     });
