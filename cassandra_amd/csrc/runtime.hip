@@ -380,19 +380,20 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
     // columns are computed whether or not they fall into the window
     // (ScatterPlan::slot_cost), after the row's digits (row_cost).
     const double lam = std::min(1.0, std::max(0.0, tune.scatter_balance));
-    auto win_cost = [&](const SlotGroup& g, uint32_t W) {
-        if (!sp.slot_cost.empty() && vbytes == 8) {
-            double c = sp.row_cost;
-            for (int j = 0; j < g.nslots; j++) c += sp.slot_cost[L.slot_list[size_t(g.first + j)]];
-            return c;
+    // the slots' own part of each group (summed once: the sort below asks often)
+    std::vector<double> own(L.groups.size(), 0.0);
+    for (size_t i = 0; i < L.groups.size(); i++)
+        for (int j = 0; j < L.groups[i].nslots; j++) {
+            const size_t slot = L.slot_list[size_t(L.groups[i].first + j)];
+            own[i] += !sp.slot_cost.empty() ? sp.slot_cost[slot] : tune.weigh_narrow ? sp.narrow[slot] : 0.0;
         }
+    auto win_cost = [&](size_t group, uint32_t W) {
+        const SlotGroup& g = L.groups[group];
+        if (!sp.slot_cost.empty() && vbytes == 8) return sp.row_cost + own[group];
         const double frac = double(W) / double(std::max<uint32_t>(1, g.col_hi - g.col_lo));
-        if (lam == 1.0 && vbytes == 8) {
-            double narrow = 0;
-            for (int j = 0; j < g.nslots && tune.weigh_narrow; j++) narrow += sp.narrow[L.slot_list[size_t(g.first + j)]];
-            return fp32 ? 4.1 + g.nslots * (1.0 + 0.26 * frac) + 0.32 * narrow
-                        : 3.0 + g.nslots * (1.0 + 2.9 * frac) + 0.45 * narrow;
-        }
+        if (lam == 1.0 && vbytes == 8)
+            return fp32 ? 4.1 + g.nslots * (1.0 + 0.26 * frac) + 0.32 * own[group]
+                        : 3.0 + g.nslots * (1.0 + 2.9 * frac) + 0.45 * own[group];
         return g.nslots * (lam + (1.0 - lam) * frac);
     };
     int nrun = 0;  // systems planned here that have rows: their windows run side by side
@@ -433,7 +434,7 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
                 auto limit = [&](double c) {
                     return std::max<int64_t>(1, std::min<int64_t>(int64_t(c), (R + kScatterBlock - 1) / kScatterBlock));
                 };
-                Win w{wl, wh, s, int(gi), R, 0, limit(cap), 0, double(R) * win_cost(g, W)};
+                Win w{wl, wh, s, int(gi), R, 0, limit(cap), 0, double(R) * win_cost(gi, W)};
                 w.most = idle ? std::max(w.cap, limit(floor_c)) : w.cap;
                 total += w.time;
                 wins.push_back(w);
@@ -512,11 +513,17 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
     // longest first: a launch of more tiles than CUs then starts its big
     // chunks in the first wave and fills in with the small ones (each tile
     // writes its own slice, so the order changes no sum)
-    auto cost = [&](const ScatterWork& w) {
-        return double(w.row_end - w.row_begin) * win_cost(L.groups[size_t(w.group)], w.win_hi - w.win_lo);
-    };
-    std::stable_sort(L.work.begin(), L.work.end(),
-                     [&](const ScatterWork& a, const ScatterWork& b) { return cost(a) > cost(b); });
+    std::vector<std::pair<double, size_t>> order;
+    order.reserve(L.work.size());
+    for (size_t i = 0; i < L.work.size(); i++) {
+        const ScatterWork& w = L.work[i];
+        order.push_back({-double(w.row_end - w.row_begin) * win_cost(size_t(w.group), w.win_hi - w.win_lo), i});
+    }
+    std::sort(order.begin(), order.end());
+    std::vector<ScatterWork> sorted;
+    sorted.reserve(order.size());
+    for (const auto& o : order) sorted.push_back(L.work[o.second]);
+    L.work = std::move(sorted);
 }
 
 // The host side of a list after planning: the bound on the terms a window
