@@ -112,7 +112,7 @@ __host__ __device__ constexpr int wide_step_slots(int entry_bytes)
 // The gather over long tiles (k_gather_long): consecutive rows a thread takes
 // together, the most runs of them in a tile, the slots of a narrow step, and
 // those of a wide one (whose values all stay in registers: FP32 with two slots
-// and three runs spilled, 110 µs against 99 with one at 5M rows of FIT8, where
+// and three runs spilled, 110 µs against 95 with one at 5M rows of FIT8, where
 // two runs take 45 µs with two slots and 51 with one at 4M rows of FIT4).
 __host__ __device__ constexpr int long_rpt(int vbytes) { return vbytes == 8 ? 4 : 8; }
 __host__ __device__ constexpr int long_max_runs(int vbytes) { return vbytes == 8 ? 2 : 3; }

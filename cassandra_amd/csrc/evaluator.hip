@@ -118,9 +118,10 @@ constexpr int kEvalBlock = 1024;
 // the values meet in LDS, where wave 0 adds them in slot order (0.0f for the
 // slots a tile does not have: no partial sum is -0.0f).  Walking the slots in
 // one thread took a dependent chain of descriptor, program and table loads per
-// slot: 64 positions x 52 slots 16.4 µs against 3.8 here, 65,536 12.0 (4
-// patterns, 18 slots: 5.6, slot by slot 15.8).  Bound by latency, and above
-// 30,000 positions by the columns' lines in L1.
+// slot: 64 positions x 52 slots 35 µs against 3.7 here, 65,536 43 against 11.4 (4
+// patterns, 18 slots: 15.9 and 6.1).  Bound by latency, and above 30,000
+// positions by the columns' lines in L1.  (The times of this kernel and the next
+// are launches back to back.)
 __global__ __launch_bounds__(kEvalBlock) void k_eval_block(const uint64_t* __restrict__ pos, int64_t n, TileView tv,
                                                            const float* __restrict__ w, uint32_t cols,
                                                            float* __restrict__ out)
@@ -173,14 +174,13 @@ __global__ __launch_bounds__(kEvalBlock) void k_eval_block(const uint64_t* __res
 // Large batches: one block a CU keeps the weights of the patterns with the
 // most variations a column in LDS (EvalPlan) and its waves walk the positions,
 // 64 C at a time; the other patterns' weights come through L1, where a wave's
-// load of 64 columns takes as many lines, and which bounds the kernel (20 of the
-// 52 slots of 12 patterns: 64 x 20 lines a wave are about 0.85 of its time).
-// 1M positions of 12 patterns: 59 µs, 85 from the expanded tables, 135 with no
-// weights in LDS; of 4 patterns 40 (52 with none).  Two runs of positions a wave
-// share a tile's weights and hide each other's latency (1M: 64 µs with one);
-// where one run a wave covers the batch, one is faster (262,144: 22 against 29).
-// A second phase of staging in place of the L1 loads would cost what it saves:
-// 160 KB for each CU take as long as 4 slots of its 4,000 positions.
+// load of 64 columns takes as many lines, which bounds the kernel.
+// 1M positions of 12 patterns (52 slots, 32 of them in LDS): 55 µs, 81 from the
+// expanded tables, 134 in the block kernel; of 4 patterns 38, 40 and 53.  Two
+// runs of positions a wave share a tile's weights and hide each other's latency
+// (1M: 60 µs with one); where one run a wave covers the batch, one is faster
+// (262,144: 20 against 26).  (Staging every pattern in phases, as
+// k_gather_tile_mf does, was not tried.)
 template <int C>
 __global__ __launch_bounds__(kEvalBlock) void k_eval_staged(const uint64_t* __restrict__ pos, int64_t n, TileView tv,
                                                             const int32_t* __restrict__ tile_lds,
@@ -249,11 +249,14 @@ int blocks_for(uint64_t n, int cap = 4096)
 
 }  // namespace
 
-// Positions a CU from which a batch is scored from LDS: the staging costs about
-// 6 µs and a pass of the staged block is long (131,072 positions on 256 CUs,
-// block / staged: 12 patterns of 52 slots 21.4 / 18.4 µs, of 54 slots 21.3 /
-// 20.3, 46 slots 15.2 / 16.4, 4 patterns 9.4 / 11.3; twice as many: 38.7 / 21.7,
-// 38.2 / 23.1, 27.5 / 17.2, 16.2 / 13.6).
+// Positions a CU from which a batch is scored from LDS: the staging comes before
+// the first position, and a pass of the staged block is long (131,072 positions
+// on 256 CUs, block / staged: 18 slots 10.0 / 10.0 µs, 46 slots 15.1 / 15.0, 52
+// slots 20.6 / 16.8, 54 slots 21.1 / 18.3; half as many 6.1 / 9.8, 8.4 / 14.7,
+// 11.4 / 16.5, 12.0 / 17.9; twice as many 16.8 / 12.6, 27.0 / 15.9, 38.2 / 20.0,
+// 37.7 / 21.2).  Sets of which nothing fits stay with the block kernel: 4M
+// positions of three patterns of 11 and 12 squares (24 slots) 381 µs, from the
+// expanded tables 413; of a single one of 10 squares (8 slots) 86 and 82.
 constexpr int64_t kEvalStagedRows = 512;
 // Most positions of one launch of the block kernel.
 constexpr int64_t kEvalBlockRows = int64_t(1) << 26;

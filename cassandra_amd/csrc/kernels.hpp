@@ -472,7 +472,7 @@ __global__ __launch_bounds__(kRowBlock) void k_index_extract(const uint64_t* __r
 // store instruction writes consecutive words; one 4-byte store per column,
 // rows apart, wrote partial lines.  With all slots in one chunk the 64 rows
 // are one run of memory and leave in 16-byte stores (vec: out is aligned).
-// 5M rows of FIT4: 131 µs for 440 MB (3.4 TB/s); 1,051 µs with the scattered
+// 5M rows of FIT4: 117 µs for 440 MB (3.8 TB/s); 1,051 µs with the scattered
 // stores.
 __global__ __launch_bounds__(kRowBlock) void k_index_extract_rows(const uint64_t* __restrict__ pos, int64_t n,
                                                                   TileView tv, int k, int chunk, int pitch,
@@ -533,7 +533,8 @@ __global__ __launch_bounds__(kRowBlock) void k_index_extract_rows(const uint64_t
 
 // Most slots a chunk of k_index_extract_rows holds in LDS (14 KB a wave), and
 // the row pitch: the chunk itself where it holds all k slots (the LDS then has
-// the layout of the memory), else odd.
+// the layout of the memory), else odd.  (A chunk of 32 slots, whose rows start in
+// the same LDS bank, takes 1M rows 41 µs, one of 34 slots 40.)
 constexpr int kExtractChunk = 56;
 
 // Matrix-free view of a pattern matrix: the column of slot s in row r is
@@ -1301,11 +1302,10 @@ __device__ __forceinline__ void gather_tile_sub(const SlotMajor<IdxT>& m, const 
 // The stored gather over long tiles: as gather_tile_single, with R runs of
 // kTileBlock * RPT rows a tile that share every staging, wide segments too
 // (their windows are walked once for all runs, in steps of kWide slots whose
-// values stay in registers).  A staging costs a CU about 2 µs (160 KB through
-// the L2, two barriers, the latency) whatever the rows it serves, and a block
-// its start and end; so a CU's rows are one tile where the registers allow
-// it.  (5M rows of FIT8: FP64 165 µs against 334 with 2,048 rows a tile, FP32
-// 99 against 121 with three tiles a CU; 1.2M rows of edax in FP64 46 against
+// values stay in registers).  A staging (160 KB through the L2, two barriers,
+// the latency) costs a CU the same whatever the rows it serves, and a block its
+// start and end; so a CU's rows are one tile where the registers allow it.  (5M rows of FIT8: FP64 165 µs against 334 with 2,048 rows a tile, FP32
+// 95 against 121 with three tiles a CU; 1.2M rows of edax in FP64 46 against
 // 102.)  Steps hold at most kLongStep slots; the entries of the next (step, run)
 // load while this one sums.  Entries of rows outside the tile are read like
 // the others (they are valid columns) and their sums dropped.
@@ -1493,9 +1493,9 @@ __global__ __launch_bounds__(BS) void k_gather_tile(SlotMajor<IdxT> m, const Row
 // 16-lane group to one row per lane, and the row sums run in slot order.  A
 // wide step holds one tile (four slots), its columns computed once, before
 // the window loop.
-// 20M rows of FIT12: 1,021 µs (digit by digit 1,764): 54 % of the cycles issue
+// 20M rows of FIT12: 998 µs (digit by digit 1,764): 54 % of the cycles issue
 // vector instructions, and staging with its barriers takes about a third (26
-// µs a tile of 2,048 rows when nothing else is done).  Four runs are what the
+// µs a tile of 4,096 rows when nothing else is done).  Four runs are what the
 // registers hold: with two it takes 1,336 µs; a loop over more rows a block,
 // computing during the staging, and taking the digits anew in every phase so
 // that eight runs fit all spilled or took longer (1,180 to 1,450 µs).
@@ -1789,8 +1789,8 @@ __global__ __launch_bounds__(kRowBlock) void k_absmax_blocks(const RowWork* __re
 // many as a group of up to four slots or of up to eight has, and no second row
 // where there is none (4,096 rows of 4 slots 8.3 µs with eight loads for each of
 // two rows, 7.0 so, both with the column sums; 65,536 rows of FIT4 21.1 and 17.5).
-// Row-major rows are the slower ones: every lane's entries lie in lines of their
-// own.
+// 65,536 rows of FIT4 alone 9.9 µs slot-major and 12.4 row-major, where every
+// lane's entries lie in lines of their own.
 // Groups are runs of at most kMaxSegSlots consecutive slots.
 template <class VT>
 __global__ __launch_bounds__(kScatterBlock) void k_scatter_part(const int32_t* __restrict__ idx, int64_t row_stride,
@@ -2040,8 +2040,9 @@ __global__ __launch_bounds__(kScatterBlock) void k_scatter_tile(SlotMajor<IdxT> 
 // slots are runs of whole patterns, so its tiles follow each other.  The windows
 // are FP64 whatever VT is: the terms of up to 32 slots and a million rows meet
 // in one window, and a fixed-point word with room for that many terms resolves
-// no more than 2^-39 of max |y|.  20M rows of FIT12: 1,745 µs (2,570 with the
-// lists evaluated digit by digit); a window of 32 slots takes 1,099 cycles per
+// no more than 2^-39 of max |y|.  20M rows of FIT12: 1,694 µs (2,570 with the
+// lists evaluated digit by digit): 48 % of the cycles issue vector instructions,
+// and the LDS is busy 48 % of them.  A window of 32 slots takes 1,099 cycles per
 // 64 rows, where fixed point, whose adds are faster, took 790.
 template <class VT, class YT, int RPT, bool kBeta = false>
 __global__ __launch_bounds__(kScatterBlock) void k_scatter_tile_mf(PositionsView m,
@@ -2814,8 +2815,7 @@ __device__ __forceinline__ VT row_gather(const int32_t* __restrict__ row, int k,
 }
 
 // Forward of the differentiable evaluator: out[r] = the sum of row r (65,536
-// rows of FIT4: 4.5 µs back to back, 7.9 with an entry, then its weight, at a
-// time).
+// rows of FIT4: 6.0 µs, 9.6 with an entry, then its weight, at a time).
 template <class VT, int V>
 __global__ __launch_bounds__(kRowBlock) void k_eval_forward(const int32_t* __restrict__ idx, int64_t B, int k,
                                                             const VT* __restrict__ w, uint32_t cols,
