@@ -545,8 +545,9 @@ void finish_lists(ScatterLists& L, int nsys)
         while (n) b++, n >>= 1;
         L.cbits = std::max(L.cbits, b);
     }
-    std::stable_sort(L.reduce.begin(), L.reduce.end(),
-                     [](const ReduceWork& a, const ReduceWork& b) { return a.sys < b.sys; });
+    const auto by_system = [](const ReduceWork& a, const ReduceWork& b) { return a.sys < b.sys; };
+    if (!std::is_sorted(L.reduce.begin(), L.reduce.end(), by_system))
+        std::stable_sort(L.reduce.begin(), L.reduce.end(), by_system);
     L.red_first.assign(size_t(nsys), 0);
     L.red_count.assign(size_t(nsys), 0);
     for (size_t i = L.reduce.size(); i-- > 0;) {
