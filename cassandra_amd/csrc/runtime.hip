@@ -406,8 +406,13 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
     // (50 systems, about 30 running: 120 µs an iteration in 1,382 tiles, 300 in
     // 256)
     const double share = tune.blocks_per_cu * std::max(cus, 1);
-    const double target =
-        share * (nrun > 1 && (on || double(windows) * nrun > 0.75 * share) ? kMultiSystemTiles : 1.0);
+    const bool several = nrun > 1 && (on || double(windows) * nrun > 0.75 * share);
+    // one system whose windows are more than half as many as the CUs: in one wave
+    // some windows would have one chunk and others two (200,000 rows of 20 slots
+    // over 3M columns: 668 µs, 368 in two; 2M rows of five patterns of 12 squares
+    // in FP64 1,409 and 818)
+    const bool coarse = nrun == 1 && vbytes == 8 && 2 * windows > cus;
+    const double target = share * (several ? kMultiSystemTiles : coarse ? 2.0 : 1.0);
     int64_t off = 0;
     if (tune.scatter_order == 1) {
         make_scatter_lists_xcd(sp, sys_rows, sys_col, cols_per_sys, wmax, vbytes, ibytes, target, cus, tune, L, on);

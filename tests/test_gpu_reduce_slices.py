@@ -48,3 +48,18 @@ def test_batch_of_few_slices(ctx, oracle):
         want = oracle.spmtv(g.indices(pos[lo:hi]), y[lo:hi], P.cols)
         for v in z.values():
             assert np.array_equal(v[s * P.cols:(s + 1) * P.cols].astype(np.float64), want)
+
+
+# more windows than half the CUs (131 of 20,352 columns): two waves of tiles
+@pytest.mark.parametrize("rows", [3, 5000, 40001])
+def test_many_windows(ctx, oracle, rows):
+    print("many windows", rows, flush=True)
+    masks = [N.B6] * 5
+    pos = oracle.random_play(600 + rows, rows, 12, 40)
+    idx = oracle.Group(masks).indices(pos)
+    A = Patterns(ctx, masks).matrix(torch.from_numpy(pos.view(np.int64)).cuda())
+    y = np.random.default_rng(rows).integers(-64, 65, rows).astype(np.float64)
+    want = oracle.spmtv(idx, y, A.cols)
+    for dtype in (torch.float32, torch.float64):
+        z = A.spmtv(torch.from_numpy(y).cuda().to(dtype)).cpu().numpy()
+        assert np.array_equal(z.astype(np.float64), want)
