@@ -410,7 +410,7 @@ void make_scatter_lists(const ScatterPlan& sp, const std::vector<int64_t>& sys_r
     // one system whose windows are more than half as many as the CUs: in one wave
     // some windows would have one chunk and others two (200,000 rows of 20 slots
     // over 3M columns: 668 µs, 368 in two; 2M rows of five patterns of 12 squares
-    // in FP64 1,409 and 818)
+    // in FP64 1,409 and 818); the lists of 4-byte counts have four waves already
     const bool coarse = nrun == 1 && vbytes == 8 && 2 * windows > cus;
     const double target = share * (several ? kMultiSystemTiles : coarse ? 2.0 : 1.0);
     int64_t off = 0;
